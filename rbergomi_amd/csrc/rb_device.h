@@ -50,18 +50,7 @@ __host__ __device__ __forceinline__ uint4 philox_block(PhiloxKey key, uint64_t p
     return philox10(make_uint4(q, uint32_t(path), uint32_t(path >> 32), stream), key);
 }
 
-// Box-Muller in FP64 on u = (x + 1/2) 2^-32: (r cos 2 pi u1, r sin 2 pi u1), r = sqrt(-2 ln u0)
-__device__ __forceinline__ void box_muller_f64(uint32_t x0, uint32_t x1, double& z0, double& z1) {
-    const double u0 = (double(x0) + 0.5) * 2.3283064365386963e-10;
-    const double u1 = (double(x1) + 0.5) * 2.3283064365386963e-10;
-    const double r = sqrt(-2.0 * log(u0));
-    double s, c;
-    sincospi(2.0 * u1, &s, &c);
-    z0 = r * c;
-    z1 = r * s;
-}
-
-// The same transform in FP32 (mixed-precision kernels): identical counters, FP32 rounding.
+// Box-Muller in FP32 (mixed-precision kernels; the FP64 form on the same counters: rb_math64.h).
 // Written with the hardware instructions directly, so that every call site compiles to the same
 // instruction sequence (a library sqrt was lowered correctly rounded at some call sites and as a
 // scaled one-ulp square root at others, so the same counter gave different FP32 normals in
@@ -82,14 +71,7 @@ __device__ __forceinline__ void box_muller_f32(uint32_t x0, uint32_t x1, float& 
     z1 = r * __builtin_amdgcn_sinf(u1);
 }
 
-// Four normals of path p, stream s, steps 4q..4q+3 in FP64
-__device__ __forceinline__ void normals4_f64(PhiloxKey key, uint64_t p, uint32_t s, uint32_t q,
-                                             double z[4]) {
-    const uint4 x = philox_block(key, p, s, q);
-    box_muller_f64(x.x, x.y, z[0], z[1]);
-    box_muller_f64(x.z, x.w, z[2], z[3]);
-}
-
+// Four normals of path p, stream s, steps 4q..4q+3
 __device__ __forceinline__ void normals4_f32(PhiloxKey key, uint64_t p, uint32_t s, uint32_t q,
                                              float z[4]) {
     const uint4 x = philox_block(key, p, s, q);

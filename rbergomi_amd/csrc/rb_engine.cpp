@@ -121,7 +121,7 @@ int validate(const Request& r, std::string& err) {
     return ST_OK;
 }
 
-Layout make_layout(const Request& r) {
+Layout make_layout(const Request& r, bool gamma, bool comp) {
     Layout L;
     const int N = r.N;
     L.N = N;
@@ -145,8 +145,8 @@ Layout make_layout(const Request& r) {
             L.units.push_back(un);
             // Gamma_0 = 0, Gamma_k = ((k+1)^(a+1) - k^(a+1))/(a+1)  (getGamma :143-149)
             const double alpha = H - 0.5;
-            L.gamma.push_back(0.0);
-            for (int k = 1; k < N; ++k)
+            if (gamma) L.gamma.push_back(0.0);
+            for (int k = 1; gamma && k < N; ++k)
                 L.gamma.push_back((std::pow(k + 1.0, alpha + 1.0) - std::pow(double(k), alpha + 1.0)) /
                                   (alpha + 1.0));
             unit_of_par[h] = u;
@@ -185,8 +185,8 @@ Layout make_layout(const Request& r) {
                 G.crho = std::sqrt(1.0 - r.rho[h] * r.rho[h]);
                 L.groups.push_back(G);
                 // compensator of updateV (:73-80): 0.5 eta^2 ((i-1) dt)^(2H), or (i dt) in exact mode
-                L.comp.push_back(0.0);
-                for (int i = 1; i < N; ++i) {
+                if (comp) L.comp.push_back(0.0);
+                for (int i = 1; comp && i < N; ++i) {
                     const double tc = r.comp == COMP_EXACT ? i * G.dt : (i - 1) * G.dt;
                     L.comp.push_back(0.5 * eta * eta * std::pow(tc, 2 * H));
                 }
@@ -310,16 +310,35 @@ void ws_free(void* p) {
     ws_evict(WS_KEEP, -1);
 }
 
+// A plan's device buffers are one workspace block, with everything to upload at its front: one
+// allocation and one copy per plan.
 template <class T>
-static hipError_t dalloc(T** p, size_t n, hipStream_t) {
-    return ws_alloc(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(T));
+void Plan::dalloc(T** p, size_t n) {
+    mem.push_back({reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(T)});
 }
 
 template <class T>
-static hipError_t upload(T** p, const std::vector<T>& v, hipStream_t st) {
-    hipError_t e = dalloc(p, v.size(), st);
-    if (e != hipSuccess || v.empty()) return e;
-    return hipMemcpyAsync(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
+void Plan::upload(T** p, const std::vector<T>& v) {
+    const size_t at = (up.size() + 255) / 256 * 256;
+    up.resize(at + v.size() * sizeof(T));
+    if (!v.empty()) std::memcpy(up.data() + at, v.data(), v.size() * sizeof(T));
+    up_at.push_back({reinterpret_cast<void**>(p), at});
+}
+
+int Plan::commit(std::string& err) {
+    size_t total = (up.size() + 255) / 256 * 256;
+    for (const auto& m : mem) total += (m.second + 255) / 256 * 256;
+    RB_TRY(ws_alloc(&d_block, total));
+    char* base = static_cast<char*>(d_block);
+    for (const auto& u : up_at) *u.first = base + u.second;
+    size_t at = (up.size() + 255) / 256 * 256;
+    for (const auto& m : mem) {
+        *m.first = base + at;
+        at += (m.second + 255) / 256 * 256;
+    }
+    // `up` outlives the copy: it is the plan's, and the plan waits for its stream before it goes
+    if (!up.empty()) RB_TRY(hipMemcpyAsync(base, up.data(), up.size(), hipMemcpyHostToDevice, stream));
+    return ST_OK;
 }
 
 Plan::~Plan() {
@@ -329,10 +348,7 @@ Plan::~Plan() {
     fused_batch.reset();  // stream-ordered frees on this plan's stream
     fused_fft.reset();
     if (stream) (void)hipStreamSynchronize(stream);
-    void* bufs[] = {d_units, d_gamma, d_groups, d_comp, d_opts,  d_Z,     d_Wt,   d_ints,
-                    d_partial, d_price, d_stat, d_iv, d_payoff, d_tw, d_ghat, d_ints2,
-                    d_Qg, d_alpha, d_exc, d_count, d_chol, d_sobol, d_shift};
-    for (void* b : bufs) ws_free(b);  // the stream has synchronized above
+    ws_free(d_block);  // the stream has synchronized above
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
     if (own_stream && stream) (void)hipStreamDestroy(stream);
 }
@@ -341,7 +357,10 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     int rc = validate(r, err);
     if (rc) return rc;
     req = r;
-    lay = make_layout(r);
+    path64 = r.precision == PREC_FP64 && r.scheme == SCHEME_HYBRID && r.N <= PATH64_MFMA_MAX_N;
+    // the staged scan's compensator table: the staged FP64 and FP32 paths, and caller's or Sobol'
+    // Gaussians at a mixed precision
+    lay = make_layout(r, !path64, !path64 && (r.precision == PREC_FP64 || r.precision == PREC_FP32 || quadrature || r.gauss >= 1));
     int ndev = 0;
     RB_TRY(hipGetDeviceCount(&ndev));
     if (ndev < 1) {
@@ -354,6 +373,7 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         RB_TRY(device_props(device, prop));
         keep_pool_cached(device);
         lds_limit = prop.sharedMemPerBlock;
+        cus = prop.multiProcessorCount;
         const int kind = volterra_conv_kind(r.N, lds_limit);
         const size_t conv_lds = kind == 0 ? volterra_mfma_lds_bytes(r.N)
                                 : kind == 1 ? volterra_mfma_long_lds_bytes(r.N, volterra_mfma_long_segment(r.N, lds_limit))
@@ -435,7 +455,8 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
             return ST_ERR_ARG;
         }
     }
-    const double per_path = 8.0 * N * (nstreams + nunits) + 16.0 * ngroups * (r.turbo ? 2 : 1) +
+    const bool need_z = !path64 || quadrature || r.gauss >= 1;
+    const double per_path = 8.0 * N * ((need_z ? nstreams : 0) + (path64 ? 0 : nunits)) + 16.0 * ngroups * (r.turbo ? 2 : 1) +
                             (quadrature ? 8.0 * nopt : 0.0);
     long ch = long(6.0e9 / per_path);
     // RBERGOMI_MAX_CHUNK caps the paths per chunk (used to test chunk boundaries)
@@ -456,11 +477,15 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         chunk = std::max(chunk, mc);
     }
     nblk = (r.M + 255) / 256;
-    RB_TRY(upload(&d_units, lay.units, stream));
-    RB_TRY(upload(&d_gamma, lay.gamma, stream));
-    RB_TRY(upload(&d_groups, lay.groups, stream));
-    RB_TRY(upload(&d_comp, lay.comp, stream));
-    RB_TRY(upload(&d_opts, lay.options, stream));
+    upload(&d_units, lay.units);
+    upload(&d_opts, lay.options);
+    if (path64) {
+        init_path64();
+    } else {
+        upload(&d_gamma, lay.gamma);
+        upload(&d_groups, lay.groups);
+        upload(&d_comp, lay.comp);
+    }
     if (conv_fft) {
         rc = init_fft(err);
         if (rc) return rc;
@@ -468,13 +493,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if (r.gauss >= 1) {
         std::vector<uint32_t> V;
         sobol_directions(nstreams * N, V);
-        RB_TRY(upload(&d_sobol, V, stream));
+        upload(&d_sobol, V);
         if (!r.seed.empty()) {
             // digital shift: Philox block (0, dimension, 0, stream 7) of the seed's key
             const PhiloxKey key = philox_key(r.seed.data(), int(r.seed.size()));
             std::vector<uint32_t> sh(size_t(nstreams) * N);
             for (size_t d = 0; d < sh.size(); ++d) sh[d] = philox_block(key, uint64_t(d), 7u, 0u).x;
-            RB_TRY(upload(&d_shift, sh, stream));
+            upload(&d_shift, sh);
         }
     }
     if (r.scheme == SCHEME_CHOLESKY) {
@@ -485,24 +510,34 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
             if (rc) return rc;
             all.insert(all.end(), L.begin(), L.end());
         }
-        RB_TRY(upload(&d_chol, all, stream));
+        upload(&d_chol, all);
     }
-    RB_TRY(dalloc(&d_Z, size_t(chunk) * nstreams * N, stream));
-    RB_TRY(dalloc(&d_Wt, size_t(nunits) * chunk * N, stream));
-    RB_TRY(dalloc(&d_ints, size_t(ngroups) * chunk * 2, stream));
-    RB_TRY(dalloc(&d_partial, size_t(nopt) * nblk * 2, stream));
-    RB_TRY(dalloc(&d_price, nopt, stream));
-    RB_TRY(dalloc(&d_stat, nopt, stream));
-    RB_TRY(dalloc(&d_iv, nopt, stream));
-    if (quadrature) RB_TRY(dalloc(&d_payoff, size_t(chunk) * nopt, stream));
+    if (need_z) dalloc(&d_Z, size_t(chunk) * nstreams * N);
+    if (!path64) dalloc(&d_Wt, size_t(nunits) * chunk * N);
+    dalloc(&d_ints, size_t(ngroups) * chunk * 2);
+    dalloc(&d_partial, size_t(nopt) * nblk * 2);
+    dalloc(&d_price, size_t(3) * nopt);  // price, stat, iv
+    if (quadrature) dalloc(&d_payoff, size_t(chunk) * nopt);
     if (r.turbo) {
-        RB_TRY(dalloc(&d_ints2, size_t(ngroups) * chunk * 2, stream));
-        RB_TRY(dalloc(&d_Qg, size_t(ngroups), stream));
-        RB_TRY(dalloc(&d_alpha, size_t(nopt), stream));
-        RB_TRY(dalloc(&d_exc, size_t(nopt) * nblk, stream));
-        RB_TRY(dalloc(&d_count, size_t(nopt), stream));
+        dalloc(&d_ints2, size_t(ngroups) * chunk * 2);
+        dalloc(&d_Qg, size_t(ngroups));
+        dalloc(&d_alpha, size_t(nopt));
+        dalloc(&d_exc, size_t(nopt) * nblk);
+        dalloc(&d_count, size_t(nopt));
     }
-    RB_TRY(hipStreamSynchronize(stream));
+    rc = commit(err);
+    if (rc) return rc;
+    d_stat = d_price + nopt;
+    d_iv = d_stat + nopt;
+    if (path64) {
+        p64.units = d_units;
+        p64.groups = d_p64groups;
+        p64.jobs = d_p64jobs;
+        p64.gamma = d_p64tab;
+        p64.ptab = d_p64tab + size_t(nunits) * p64.tlen;
+        RB_TRY(launch_path64_tables(d_units, int(nunits), N, p64.tlen, r.comp == COMP_EXACT ? 0.0 : 1.0, d_p64tab,
+                                    d_p64tab + size_t(nunits) * p64.tlen, stream));
+    }
     return ST_OK;
 }
 
@@ -517,6 +552,8 @@ void Plan::begin_timing() {
         times[K_VOLTERRA].name = "k_volterra_chol_f64";
     else if (conv_fft)
         times[K_VOLTERRA].name = "k_volterra_fft";
+    else if (path64)
+        times[K_VOLTERRA].name = "k_path64";
     else if (volterra_conv_kind(req.N, lds_limit) == 0)
         times[K_VOLTERRA].name = "k_volterra_mfma_f64";
     else if (volterra_conv_kind(req.N, lds_limit) == 1)
@@ -562,21 +599,46 @@ void Plan::end_timing() {
         mark(slot_, nullptr, nullptr);       \
     } while (0)
 
+int Plan::integrals(uint64_t p0, long np, bool from_z, int signs, std::string& err) {
+    const PhiloxKey key = philox_key(req.seed.data(), int(req.seed.size()));
+    if (path64) {
+        Path64Args a = p64;
+        a.key = key;
+        a.p0 = long(p0);
+        a.np = np;
+        a.src = from_z ? P64_MEMORY : P64_PHILOX;
+        a.signs = signs;
+        a.Z = d_Z;
+        a.zstride = long(nstreams) * req.N;
+        a.ints = d_ints;
+        a.ints2 = d_ints2;
+        path64_shape(a, cus);
+        RB_LAUNCH(K_VOLTERRA, launch_path64(a, stream));
+        return ST_OK;
+    }
+    const int N = req.N, ngroups = int(lay.groups.size());
+    const long zs = long(nstreams) * N;
+    if (!from_z) RB_LAUNCH(K_NORMALS, launch_normals_f64(key, long(p0), np, nstreams, N, d_Z, stream));
+    RB_LAUNCH(K_VOLTERRA, conv(np, zs));
+    RB_LAUNCH(K_SCAN, launch_scan_f64(req.method, d_Z, zs, d_Wt, np, N, d_groups, ngroups, d_comp, d_ints, stream));
+    if (signs == 2)
+        RB_LAUNCH(K_SCAN, launch_scan_f64(METHOD_RT, d_Z, zs, d_Wt, np, N, d_groups, ngroups, d_comp, d_ints2,
+                                          stream, -1.0));
+    return ST_OK;
+}
+
 // Enqueue one pricing run on the plan's stream (no synchronization).
 int Plan::enqueue(std::string& err) {
     if (fused) return fused_batch->launch(stream, err, capturing ? nullptr : this);
     if (fused_fft) return fused_fft->launch(stream, err, capturing ? nullptr : this);
     const int N = req.N;
     const int nopt = int(lay.options.size());
-    const PhiloxKey key = philox_key(req.seed.data(), int(req.seed.size()));
     const int ngroups = int(lay.groups.size());
     if (req.turbo) {
         // pilot paths (counters TURBO_PILOT_BASE + m, disjoint from the main paths): Q and alpha
         const long mc = req.m_control;
-        RB_LAUNCH(K_NORMALS, launch_normals_f64(key, TURBO_PILOT_BASE, mc, nstreams, N, d_Z, stream));
-        RB_LAUNCH(K_VOLTERRA, conv(mc, long(nstreams) * N));
-        RB_LAUNCH(K_SCAN, launch_scan_f64(METHOD_RT, d_Z, long(nstreams) * N, d_Wt, mc, N, d_groups,
-                                          ngroups, d_comp, d_ints, stream, 1.0));
+        const int rc = integrals(TURBO_PILOT_BASE, mc, false, 1, err);
+        if (rc) return rc;
         RB_LAUNCH(K_PAYOFF, launch_turbo_q(d_ints, mc, ngroups, d_Qg, stream));
         RB_LAUNCH(K_PAYOFF, launch_turbo_alpha(d_ints, mc, d_opts, nopt, d_Qg, d_alpha, stream));
     }
@@ -585,14 +647,10 @@ int Plan::enqueue(std::string& err) {
         if (req.gauss >= 1) {
             RB_LAUNCH(K_NORMALS, launch_normals_sobol_f64(d_sobol, d_shift, p0, np, nstreams, N, d_Z, stream));
             if (req.gauss == 2) RB_LAUNCH(K_NORMALS, launch_bridge_f64(d_Z, np * nstreams, N, stream));
-        } else
-            RB_LAUNCH(K_NORMALS, launch_normals_f64(key, p0, np, nstreams, N, d_Z, stream));
-        RB_LAUNCH(K_VOLTERRA, conv(np, long(nstreams) * N));
-        RB_LAUNCH(K_SCAN, launch_scan_f64(req.method, d_Z, long(nstreams) * N, d_Wt, np, N, d_groups,
-                                          ngroups, d_comp, d_ints, stream));
+        }
+        const int rc = integrals(uint64_t(p0), np, req.gauss >= 1, req.turbo ? 2 : 1, err);
+        if (rc) return rc;
         if (req.turbo) {
-            RB_LAUNCH(K_SCAN, launch_scan_f64(METHOD_RT, d_Z, long(nstreams) * N, d_Wt, np, N, d_groups,
-                                              ngroups, d_comp, d_ints2, stream, -1.0));
             RB_LAUNCH(K_PAYOFF, launch_turbo_payoff(d_ints, d_ints2, np, d_opts, nopt, d_Qg, d_alpha,
                                                     req.q_max, p0 / 256, nblk, d_partial, d_exc, stream));
         } else {
@@ -654,9 +712,8 @@ int Plan::run_samples(const double* Z_host, double* payoff_host, std::string& er
         const long np = std::min(chunk, req.M - p0);
         RB_TRY(hipMemcpyAsync(d_Z, Z_host + size_t(p0) * nstreams * N,
                               size_t(np) * nstreams * N * sizeof(double), hipMemcpyHostToDevice, stream));
-        RB_LAUNCH(K_VOLTERRA, conv(np, long(nstreams) * N));
-        RB_LAUNCH(K_SCAN, launch_scan_f64(req.method, d_Z, long(nstreams) * N, d_Wt, np, N, d_groups,
-                                          int(lay.groups.size()), d_comp, d_ints, stream));
+        const int rc = integrals(0, np, true, 1, err);
+        if (rc) return rc;
         RB_LAUNCH(K_PAYOFF, launch_payoff_f64(d_ints, np, 0, d_opts, nopt, req.method, p0 / 256, nblk,
                                               d_partial, d_payoff, stream));
         RB_TRY(hipMemcpyAsync(payoff_host + size_t(p0) * nopt, d_payoff, size_t(np) * nopt * sizeof(double),
@@ -716,9 +773,51 @@ int Plan::init_fft(std::string& err) {
         fft_host(a, -1);
         for (int k = 0; k < L; ++k) gh[u * L + k] = make_float2(float(a[k].real()), float(a[k].imag()));
     }
-    RB_TRY(upload(&d_tw, tw, stream));
-    RB_TRY(upload(&d_ghat, gh, stream));
+    upload(&d_tw, tw);
+    upload(&d_ghat, gh);
     return ST_OK;
+}
+
+// Tables of the single-pass FP64 path: groups ordered by unit with their exponent's coefficients,
+// jobs of one unit and up to greg groups, and gamma and P of every unit, formed on the device.
+void Plan::init_path64() {
+    const int N = req.N, nunits = int(lay.units.size()), ngroups = int(lay.groups.size());
+    std::vector<int> order(ngroups), count(nunits, 0);
+    for (int g = 0; g < ngroups; ++g) {
+        order[g] = g;
+        ++count[lay.groups[g].unit];
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return lay.groups[x].unit < lay.groups[y].unit; });
+    p64.N = N;
+    p64.tlen = (N + 15) / 16 * 16;
+    p64.mc = req.method == METHOD_MC;
+    p64.greg = path64_greg(*std::max_element(count.begin(), count.end()), req.turbo ? 2 : 1);
+    constexpr double L2E16 = 23.083120654223414192;  // 16 log2(e): half the exponent, in 32nds of an octave
+    std::vector<Path64Group> groups(ngroups);
+    std::vector<Path64Job> jobs;
+    for (int k = 0; k < ngroups; ++k) {
+        const Group& G = lay.groups[order[k]];
+        const Unit& un = lay.units[G.unit];
+        Path64Group& o = groups[k];
+        o.c1 = L2E16 * G.eta * G.TH * un.sc;
+        o.al = std::min(std::max(L2E16 * 0.5 * G.eta * G.eta * std::pow(G.dt, 2.0 * un.H), P64_AL_MIN), P64_AL_MAX);
+        o.xi = G.xi;
+        o.sxi = std::sqrt(G.xi);
+        o.dt = G.dt;
+        o.sdt = G.sdt;
+        o.rho = G.rho;
+        o.crho = G.crho;
+        o.out = order[k];
+        o.pad = 0;
+        if (jobs.empty() || jobs.back().unit != G.unit || jobs.back().gn == p64.greg)
+            jobs.push_back(Path64Job{G.unit, k, 0, 0});
+        ++jobs.back().gn;
+    }
+    p64.njobs = int(jobs.size());
+    upload(&d_units, lay.units);
+    upload(&d_p64groups, groups);
+    upload(&d_p64jobs, jobs);
+    dalloc(&d_p64tab, size_t(2) * nunits * p64.tlen);
 }
 
 hipError_t Plan::conv(long np, long zstride) {
@@ -756,11 +855,13 @@ int Plan::results(double* price, double* iv, double* stat, std::string& err) {
         RB_TRY(hipStreamSynchronize(stream));
         return ST_OK;
     }
-    const size_t n = lay.options.size() * sizeof(double);
-    if (price) RB_TRY(hipMemcpyAsync(price, d_price, n, hipMemcpyDeviceToHost, stream));
-    if (iv) RB_TRY(hipMemcpyAsync(iv, d_iv, n, hipMemcpyDeviceToHost, stream));
-    if (stat) RB_TRY(hipMemcpyAsync(stat, d_stat, n, hipMemcpyDeviceToHost, stream));
+    const size_t n = lay.options.size();
+    std::vector<double> got(3 * n);  // price, stat, iv
+    RB_TRY(hipMemcpyAsync(got.data(), d_price, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream));
     RB_TRY(hipStreamSynchronize(stream));
+    if (price) std::copy_n(got.begin(), n, price);
+    if (stat) std::copy_n(got.begin() + n, n, stat);
+    if (iv) std::copy_n(got.begin() + 2 * n, n, iv);
     return ST_OK;
 }
 

@@ -11,6 +11,7 @@
 #include "rb_device.h"
 #include "rb_fused.h"
 #include "rb_fused_host.h"
+#include "rb_path64.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -85,7 +86,9 @@ std::vector<uint64_t> primitive_polynomials(int count);
 constexpr long TURBO_PILOT_BASE = 1L << 62;
 
 int validate(const Request& r, std::string& err);
-Layout make_layout(const Request& r);
+// gamma, comp: whether the per-step tables are wanted too (the FP64 path kernels form theirs on the
+// device, and only the staged scan reads comp)
+Layout make_layout(const Request& r, bool gamma = true, bool comp = false);
 PhiloxKey philox_key(const uint64_t* seed, int n);
 // FFT in FP64 on the host (radix-2, a.size() a power of two; sign -1 forward, unnormalised)
 void fft_host(std::vector<std::complex<double>>& a, int sign);
@@ -114,6 +117,16 @@ struct Plan {
     long chunk = 0;          // paths per chunk
     long nblk = 0;           // 256-path blocks over all M
     int nstreams = 2;        // Gaussian blocks per path: W1, W1perp (+ Wperp for plain MC)
+    // the block that holds every device buffer below, and what its front is filled from
+    void* d_block = nullptr;
+    std::vector<std::pair<void**, size_t>> mem;    // buffers and their bytes
+    std::vector<std::pair<void**, size_t>> up_at;  // uploaded tables and their places in `up`
+    std::vector<char> up;
+    template <class T>
+    void dalloc(T** p, size_t n);
+    template <class T>
+    void upload(T** p, const std::vector<T>& v);
+    int commit(std::string& err);
     // device tables
     Unit* d_units = nullptr;
     double* d_gamma = nullptr;
@@ -138,6 +151,13 @@ struct Plan {
     double* d_alpha = nullptr;    // [options] control-variate coefficients
     int* d_exc = nullptr;         // [options][nblk] Q <= Iv evaluations per path block
     long* d_count = nullptr;      // [options] their totals
+    // single-pass FP64 path (hybrid scheme, FP64): no Gaussians or Wtilde in HBM unless the caller's
+    bool path64 = false;
+    Path64Args p64{};             // tables and launch shape; the paths are set per chunk
+    Path64Group* d_p64groups = nullptr;
+    Path64Job* d_p64jobs = nullptr;
+    double* d_p64tab = nullptr;   // gamma and P of every unit
+    int cus = 256;                // compute units of the device
     size_t lds_limit = 65536;     // LDS bytes one workgroup may use on the plan's device
     // long-path FP32 FFT convolution (replaces the FP64 convolution in the staged pipeline)
     bool conv_fft = false;
@@ -172,7 +192,11 @@ struct Plan {
     int turbo_results(double* alpha, double* Q, long* exceptions, std::string& err);
     int init_fused(std::string& err);
     int init_fft(std::string& err);
+    void init_path64();
     hipError_t conv(long np, long zstride);
+    // enqueue the integrals of np paths into d_ints (signs = 2: the mirrored paths' into d_ints2
+    // too): Philox paths from counter p0, or the Gaussians in d_Z
+    int integrals(uint64_t p0, long np, bool from_z, int signs, std::string& err);
     // enqueue one run on the plan's stream, no synchronization
     int enqueue(std::string& err);
     void begin_timing();

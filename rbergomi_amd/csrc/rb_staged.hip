@@ -20,6 +20,7 @@
 
 #include "rb_device.h"
 #include "rb_kernels.h"
+#include "rb_math64.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -44,6 +45,9 @@ hipError_t allow_lds(const void* fn, size_t bytes) {
 // One thread per (path, stream, 4-step block).  out[(p*nstreams + s)*N + j]
 __global__ void k_normals_f64(PhiloxKey key, long p0, long np, int nstreams, int N,
                               double* __restrict__ out) {
+    __shared__ double2 lg[LOG_N];
+    load_log_tab(lg, threadIdx.x, blockDim.x);
+    __syncthreads();
     const int nq = (N + 3) / 4;
     const long total = np * nstreams * nq;
     for (long t = blockIdx.x * long(blockDim.x) + threadIdx.x; t < total;
@@ -53,7 +57,7 @@ __global__ void k_normals_f64(PhiloxKey key, long p0, long np, int nstreams, int
         const int s = int(ps % nstreams);
         const long p = ps / nstreams;
         double z[4];
-        normals4_f64(key, uint64_t(p0 + p), uint32_t(s), uint32_t(q), z);
+        normals4_f64(lg, key, uint64_t(p0 + p), uint32_t(s), uint32_t(q), z);
         double* o = out + ps * N + 4 * q;
         if (4 * q + 3 < N) {
             o[0] = z[0]; o[1] = z[1]; o[2] = z[2]; o[3] = z[3];

@@ -357,7 +357,7 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     int rc = validate(r, err);
     if (rc) return rc;
     req = r;
-    path64 = r.precision == PREC_FP64 && r.scheme == SCHEME_HYBRID && r.N <= PATH64_MFMA_MAX_N;
+    path64 = r.precision == PREC_FP64 && r.scheme == SCHEME_HYBRID && r.N <= PATH64_FFT_MAX_N;
     // the staged scan's compensator table: the staged FP64 and FP32 paths, and caller's or Sobol'
     // Gaussians at a mixed precision
     lay = make_layout(r, !path64, !path64 && (r.precision == PREC_FP64 || r.precision == PREC_FP32 || quadrature || r.gauss >= 1));
@@ -374,10 +374,9 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         keep_pool_cached(device);
         lds_limit = prop.sharedMemPerBlock;
         cus = prop.multiProcessorCount;
-        const int kind = volterra_conv_kind(r.N, lds_limit);
-        const size_t conv_lds = kind == 0 ? volterra_mfma_lds_bytes(r.N)
-                                : kind == 1 ? volterra_mfma_long_lds_bytes(r.N, volterra_mfma_long_segment(r.N, lds_limit))
-                                            : volterra_f64_lds_bytes(r.N);
+        const size_t conv_lds = volterra_conv_mfma(r.N, lds_limit)
+                                    ? volterra_mfma_long_lds_bytes(r.N, volterra_mfma_long_segment(r.N, lds_limit))
+                                    : volterra_f64_lds_bytes(r.N);
         if (conv_lds > prop.sharedMemPerBlock) {
             err = "N = " + std::to_string(r.N) + " needs more LDS than one workgroup can hold";
             return ST_ERR_LIMIT;
@@ -537,6 +536,12 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         p64.ptab = d_p64tab + size_t(nunits) * p64.tlen;
         RB_TRY(launch_path64_tables(d_units, int(nunits), N, p64.tlen, r.comp == COMP_EXACT ? 0.0 : 1.0, d_p64tab,
                                     d_p64tab + size_t(nunits) * p64.tlen, stream));
+        if (path64_uses_fft(N)) {
+            p64.tw = d_p64fft;
+            p64.ghat = d_p64fft + path64_fft_table(N);
+            RB_TRY(launch_path64_fft_tables(p64.gamma, int(nunits), N, p64.tlen, d_p64fft,
+                                            d_p64fft + path64_fft_table(N), stream));
+        }
     }
     return ST_OK;
 }
@@ -553,10 +558,8 @@ void Plan::begin_timing() {
     else if (conv_fft)
         times[K_VOLTERRA].name = "k_volterra_fft";
     else if (path64)
-        times[K_VOLTERRA].name = "k_path64";
-    else if (volterra_conv_kind(req.N, lds_limit) == 0)
-        times[K_VOLTERRA].name = "k_volterra_mfma_f64";
-    else if (volterra_conv_kind(req.N, lds_limit) == 1)
+        times[K_VOLTERRA].name = path64_uses_fft(req.N) ? "k_path64_fft" : "k_path64";
+    else if (volterra_conv_mfma(req.N, lds_limit))
         times[K_VOLTERRA].name = "k_volterra_mfma_long_f64";
 }
 
@@ -612,8 +615,13 @@ int Plan::integrals(uint64_t p0, long np, bool from_z, int signs, std::string& e
         a.zstride = long(nstreams) * req.N;
         a.ints = d_ints;
         a.ints2 = d_ints2;
-        path64_shape(a, cus);
-        RB_LAUNCH(K_VOLTERRA, launch_path64(a, stream));
+        if (path64_uses_fft(req.N)) {
+            path64_fft_shape(a, cus);
+            RB_LAUNCH(K_VOLTERRA, launch_path64_fft(a, stream));
+        } else {
+            path64_shape(a, cus);
+            RB_LAUNCH(K_VOLTERRA, launch_path64(a, stream));
+        }
         return ST_OK;
     }
     const int N = req.N, ngroups = int(lay.groups.size());
@@ -818,6 +826,7 @@ void Plan::init_path64() {
     upload(&d_p64groups, groups);
     upload(&d_p64jobs, jobs);
     dalloc(&d_p64tab, size_t(2) * nunits * p64.tlen);
+    if (path64_uses_fft(N)) dalloc(&d_p64fft, path64_fft_table(N) + (size_t(nunits) << path64_fft_log2(N)));
 }
 
 hipError_t Plan::conv(long np, long zstride) {

@@ -157,6 +157,7 @@ struct Plan {
     Path64Group* d_p64groups = nullptr;
     Path64Job* d_p64jobs = nullptr;
     double* d_p64tab = nullptr;   // gamma and P of every unit
+    double2* d_p64fft = nullptr;  // twiddles, and the spectrum of every unit's gamma
     int cus = 256;                // compute units of the device
     size_t lds_limit = 65536;     // LDS bytes one workgroup may use on the plan's device
     // long-path FP32 FFT convolution (replaces the FP64 convolution in the staged pipeline)

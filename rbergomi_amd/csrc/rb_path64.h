@@ -56,20 +56,30 @@ struct Path64Args {
     double* ints;          // [groups][np][2]: (integral of v, of sqrt(v) dW), plain MC (ln S_T, 0)
     double* ints2;
     // FFT kernel only
-    int log2L;
-    const double2* tw;     // [L/2] exp(-2 pi i k / L)
-    const double2* ghat;   // [units][L] transform of gamma, in bit-reversed order, over L
+    const double2* tw;     // twiddles of both transforms (Fft64)
+    const double2* ghat;   // [units][L] spectrum of gamma over L, in the middle pass's order
 };
 
 // gamma and ptab of every unit (off: 1 for the reference compensator ((i-1) dt)^2H, 0 for (i dt)^2H)
 hipError_t launch_path64_tables(const Unit* units, int nunits, int N, int tlen, double off, double* gamma,
                                 double* ptab, hipStream_t st);
 
-// The matrix-core kernel (N <= 512): groups per job, launch shape, LDS
+// The matrix-core kernel (N <= 512 by its LDS and registers): groups per job, launch shape, LDS
 constexpr int PATH64_MFMA_MAX_N = 512;
 int path64_greg(int groups_of_largest_unit, int signs);
 void path64_shape(Path64Args& a, int cus);
 size_t path64_lds_bytes(const Path64Args& a);
 hipError_t launch_path64(const Path64Args& a, hipStream_t st);
+
+// The transform kernel (N <= 4096, and whether it is taken for N): length 2^log2 >= 2N, twiddle and spectrum tables (path64_fft_table
+// and L entries per unit), LDS
+constexpr int PATH64_FFT_MAX_N = 4096, PATH64_FFT_MIN_LOG2 = 9;
+bool path64_uses_fft(int N);
+int path64_fft_log2(int N);
+void path64_fft_shape(Path64Args& a, int cus);
+size_t path64_fft_table(int N);
+hipError_t launch_path64_fft_tables(const double* gamma, int nunits, int N, int tlen, double2* tw, double2* ghat,
+                                    hipStream_t st);
+hipError_t launch_path64_fft(const Path64Args& a, hipStream_t st);
 
 }  // namespace rb

@@ -1,7 +1,8 @@
-"""The single-pass FP64 path kernel (k_path64) at the edges of its tiles and dispatch, against the
+"""The single-pass FP64 path kernels (k_path64, k_path64_fft) at the edges of its tiles and dispatch, against the
 oracle on the same Gaussians: row blocks of 16 (N = 16 k, 16 k + 1, 16 k + 2), the sub-tile counts
 (N <= 17, <= 33, above), tiles with absent paths, groups beyond one job (2, 4, 8 per job), many units
-with the paths' second stream kept in LDS or not, and both workgroup sizes.
+with the paths' second stream kept in LDS or not, and both workgroup sizes; for the transform
+kernel (N > 384) both ends of every transform length, an odd number of paths and absent pairs.
 
 Tolerances are the FP64 path's: integrals 1e-10 relative with a floor of 1e-3, prices and standard
 errors 1e-12 absolute."""
@@ -33,7 +34,8 @@ def _params(units, mats, seed):
 
 
 EDGES = [(1, 3), (2, 64), (16, 65), (17, 70), (18, 33), (33, 40), (34, 17), (64, 16), (65, 15), (113, 20), (129, 1),
-         (241, 18), (257, 16), (304, 17), (497, 3), (511, 5), (512, 33)]
+         (241, 18), (257, 16), (304, 17), (384, 33), (385, 9), (512, 8), (513, 5), (1024, 3), (1025, 1), (2048, 3),
+         (2049, 2), (4095, 1), (4096, 3)]
 
 
 @pytest.mark.parametrize("N,M", EDGES)
@@ -56,7 +58,8 @@ def test_integrals_at_tile_edges(rb, orc, N, M):
 # (units, maturities, N): groups per job 2, 4 and 8 with remainders; units with W1perp in LDS
 # (N = 100, 200) and drawn again (N = 400); 512 threads with and without it
 SHAPES = [(1, 1, 100), (1, 3, 300), (1, 5, 100), (1, 9, 260), (1, 17, 64), (3, 2, 100), (5, 1, 200), (4, 3, 400),
-          (2, 9, 30), (70, 1, 48)]
+          (2, 9, 30), (70, 1, 48),
+          (1, 1, 500), (3, 2, 385), (1, 9, 1000), (2, 2, 1500), (5, 1, 4000)]
 
 
 @pytest.mark.parametrize("method", [0, 1])

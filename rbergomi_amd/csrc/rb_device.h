@@ -100,19 +100,6 @@ __device__ inline double norm_inv_f64(double u) {
     return u < 0.5 ? x : -x;
 }
 
-// Romano-Touzi payoff: C_BS(S', K, tau = 1, sigma) with sigma = sqrt((1-rho^2) Iv),
-// ln S' = -rho^2 Iv / 2 + rho Is  (rBergLib/rBergomiMT.cpp:383-388, BlackScholes.cpp:22-26).
-// ln(S'/K) is formed as lnS - lnK, which avoids a log per strike.
-__device__ __forceinline__ double rt_payoff_f64(double Iv, double Is, double rho, double K,
-                                                double lnK) {
-    const double sig = sqrt((1.0 - rho * rho) * Iv);
-    const double lnS = -0.5 * rho * rho * Iv + rho * Is;
-    const double S = exp(lnS);
-    const double d1 = (lnS - lnK + 0.5 * sig * sig) / sig;
-    const double d2 = d1 - sig;
-    return phi_f64(d1) * S - phi_f64(d2) * K;
-}
-
 __device__ __forceinline__ double bs_price_f64(double K, double tau, double sig, bool call) {
     const double st = sig * sqrt(tau);
     const double d1 = (-log(K) + 0.5 * st * st) / st;

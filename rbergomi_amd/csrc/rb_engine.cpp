@@ -29,7 +29,7 @@ const char* last_error() { return g_last_error.c_str(); }
 
 const char* kernel_name(int id) {
     static const char* names[K_COUNT] = {"k_normals_f64", "k_volterra_f64", "k_scan_f64",
-                                         "k_payoff_f64",  "k_reduce_f64",   "k_iv_f64",
+                                         "k_payoff64",    "k_reduce_iv",    "k_iv",
                                          "k_fused"};
     return id >= 0 && id < K_COUNT ? names[id] : "?";
 }
@@ -463,8 +463,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         const long cap = std::atol(env);
         if (cap > 0) ch = std::min(ch, cap);
     }
-    ch = std::max<long>(256, (ch / 256) * 256);
-    const long Mr = ((r.M + 255) / 256) * 256;
+    // paths per payoff thread, so that a block's sums cover 256 ppt paths: as many as leave 2048
+    // blocks of the whole option table (one per thread otherwise, and in the turbo-charged estimator)
+    ppt = r.turbo ? 1 : 4;
+    while (ppt > 1 && r.M / (256L * ppt) * ((nopt + PAY64_OPTS - 1) / PAY64_OPTS) < 2048) ppt /= 2;
+    const long pblk = 256L * ppt;
+    ch = std::max(pblk, ch / pblk * pblk);
+    const long Mr = (r.M + pblk - 1) / pblk * pblk;
     chunk = std::min(ch, Mr);
     if (r.turbo) {
         // the pilot paths are priced as one chunk (two-pass covariances over all of them)
@@ -475,9 +480,10 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         }
         chunk = std::max(chunk, mc);
     }
-    nblk = (r.M + 255) / 256;
+    nblk = (r.M + pblk - 1) / pblk;
     upload(&d_units, lay.units);
     upload(&d_opts, lay.options);
+    init_payoffs();
     if (path64) {
         init_path64();
     } else {
@@ -662,15 +668,17 @@ int Plan::enqueue(std::string& err) {
             RB_LAUNCH(K_PAYOFF, launch_turbo_payoff(d_ints, d_ints2, np, d_opts, nopt, d_Qg, d_alpha,
                                                     req.q_max, p0 / 256, nblk, d_partial, d_exc, stream));
         } else {
-            RB_LAUNCH(K_PAYOFF, launch_payoff_f64(d_ints, np, p0, d_opts, nopt, req.method, p0 / 256,
-                                                  nblk, d_partial, nullptr, stream));
+            RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt, req.method,
+                                                p0 / (256 * ppt), nblk, d_partial, nullptr, stream));
         }
     }
-    RB_LAUNCH(K_REDUCE, launch_reduce_f64(d_partial, nblk, req.M, nopt, d_price, d_stat, stream));
-    if (req.turbo)
+    RB_LAUNCH(K_REDUCE, launch_reduce_iv(d_partial, ReduceRows{nullptr, nullptr, nullptr, nblk, req.M}, d_opts, nopt,
+                                         d_price, d_stat, req.turbo ? nullptr : d_iv, nullptr, stream));
+    if (req.turbo) {
         RB_LAUNCH(K_REDUCE, launch_turbo_adjust(d_price, d_opts, nopt, d_Qg, d_alpha, req.q_max, d_exc,
                                                 nblk, req.M, d_count, stream));
-    RB_LAUNCH(K_IV, launch_iv_f64(d_price, d_opts, nopt, d_iv, stream));
+        RB_LAUNCH(K_IV, launch_iv(d_price, d_opts, nopt, d_iv, stream));
+    }
     return ST_OK;
 }
 
@@ -722,14 +730,14 @@ int Plan::run_samples(const double* Z_host, double* payoff_host, std::string& er
                               size_t(np) * nstreams * N * sizeof(double), hipMemcpyHostToDevice, stream));
         const int rc = integrals(0, np, true, 1, err);
         if (rc) return rc;
-        RB_LAUNCH(K_PAYOFF, launch_payoff_f64(d_ints, np, 0, d_opts, nopt, req.method, p0 / 256, nblk,
-                                              d_partial, d_payoff, stream));
+        RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt, req.method,
+                                            p0 / (256 * ppt), nblk, d_partial, d_payoff, stream));
         RB_TRY(hipMemcpyAsync(payoff_host + size_t(p0) * nopt, d_payoff, size_t(np) * nopt * sizeof(double),
                               hipMemcpyDeviceToHost, stream));
         RB_TRY(hipStreamSynchronize(stream));
     }
-    RB_LAUNCH(K_REDUCE, launch_reduce_f64(d_partial, nblk, req.M, nopt, d_price, d_stat, stream));
-    RB_LAUNCH(K_IV, launch_iv_f64(d_price, d_opts, nopt, d_iv, stream));
+    RB_LAUNCH(K_REDUCE, launch_reduce_iv(d_partial, ReduceRows{nullptr, nullptr, nullptr, nblk, req.M}, d_opts, nopt,
+                                         d_price, d_stat, d_iv, nullptr, stream));
     RB_TRY(hipStreamSynchronize(stream));
     end_timing();
     return ST_OK;
@@ -784,6 +792,32 @@ int Plan::init_fft(std::string& err) {
     upload(&d_tw, tw);
     upload(&d_ghat, gh);
     return ST_OK;
+}
+
+// Jobs of the payoff stage: runs of up to PAY64_OPTS options of one (group, rho), shorter where the
+// path blocks alone leave compute units without one.
+void Plan::init_payoffs() {
+    const int nopt = int(lay.options.size());
+    std::vector<int> order(nopt);
+    for (int I = 0; I < nopt; ++I) order[I] = I;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        const Option &a = lay.options[x], &b = lay.options[y];
+        return a.group != b.group ? a.group < b.group : a.rho < b.rho;
+    });
+    int most = PAY64_OPTS;
+    while (most > 1 && nblk * ((nopt + most - 1) / most) < 4L * cus) most /= 2;
+    std::vector<PayJob64> jobs;
+    std::vector<PayOpt64> opts(nopt);
+    for (int k = 0; k < nopt; ++k) {
+        const Option& o = lay.options[order[k]];
+        opts[k] = PayOpt64{o.K, o.lnK, order[k], 0};
+        if (jobs.empty() || jobs.back().group != o.group || jobs.back().rho != o.rho || jobs.back().n == most)
+            jobs.push_back(PayJob64{o.group, k, 0, 0, o.rho});
+        ++jobs.back().n;
+    }
+    npayjobs = int(jobs.size());
+    upload(&d_payjobs, jobs);
+    upload(&d_payopts, opts);
 }
 
 // Tables of the single-pass FP64 path: groups ordered by unit with their exponent's coefficients,

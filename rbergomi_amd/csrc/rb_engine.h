@@ -12,6 +12,7 @@
 #include "rb_fused.h"
 #include "rb_fused_host.h"
 #include "rb_path64.h"
+#include "rb_payoff64.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -115,7 +116,8 @@ struct Plan {
     bool own_stream = false;
     bool profile = false;
     long chunk = 0;          // paths per chunk
-    long nblk = 0;           // 256-path blocks over all M
+    int ppt = 1;             // paths per payoff thread
+    long nblk = 0;           // blocks of 256 ppt paths over all M
     int nstreams = 2;        // Gaussian blocks per path: W1, W1perp (+ Wperp for plain MC)
     // the block that holds every device buffer below, and what its front is filled from
     void* d_block = nullptr;
@@ -133,6 +135,9 @@ struct Plan {
     Group* d_groups = nullptr;
     double* d_comp = nullptr;
     Option* d_opts = nullptr;
+    PayJob64* d_payjobs = nullptr;
+    PayOpt64* d_payopts = nullptr;
+    int npayjobs = 0;
     // device work buffers
     double* d_Z = nullptr;        // [chunk][nstreams][N]
     double* d_Wt = nullptr;       // [units][chunk][N]
@@ -193,6 +198,7 @@ struct Plan {
     int turbo_results(double* alpha, double* Q, long* exceptions, std::string& err);
     int init_fused(std::string& err);
     int init_fft(std::string& err);
+    void init_payoffs();
     void init_path64();
     hipError_t conv(long np, long zstride);
     // enqueue the integrals of np paths into d_ints (signs = 2: the mirrored paths' into d_ints2

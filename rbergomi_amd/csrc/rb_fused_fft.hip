@@ -22,7 +22,7 @@
 // Plain Monte Carlo (computeIV_tensor's estimator, MC = true): a third sum sqrt(v) Wperp with
 // Wperp from stream 2, ln S_T = rho Is + sqrt(1 - rho^2) Ip - Iv / 2 and the payoff (S_T - K)^+
 // in FP64 (updateZ/updateS, rBergLib/rBergomiMT.cpp:111-137).
-// Outputs the same per-item option sums as the GEMM kernel, reduced by k_reduce_rows.
+// Outputs the same per-item option sums as the GEMM kernel, reduced by k_reduce_iv.
 #include <hip/hip_runtime.h>
 
 #include "rb_fft_lds.h"

@@ -784,8 +784,8 @@ int FusedBatch::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_
     mark(s);
     if (kend) RB_TRY(hipEventRecord(kend, st));
     s = timed(K_REDUCE);
-    RB_TRY(launch_reduce_rows_iv(d_partial, d_row_off, d_row_n, d_row_M, d_ivopts, total_out, d_price, d_stat, d_iv,
-                                 d_counter, st));
+    RB_TRY(launch_reduce_iv(d_partial, ReduceRows{d_row_off, d_row_n, d_row_M, 0, 0}, d_ivopts, total_out, d_price,
+                            d_stat, d_iv, d_counter, st));
     mark(s);
     counter_dirty = total_out < 1;
     return ST_OK;
@@ -967,10 +967,8 @@ int FftFused::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_t 
     mark(s);
     if (kend) RB_TRY(hipEventRecord(kend, st));
     s = timed(K_REDUCE);
-    RB_TRY(launch_reduce_rows(d_partial, d_row_off, d_row_n, d_row_M, total_out, d_price, d_stat, st));
-    mark(s);
-    s = timed(K_IV);
-    RB_TRY(launch_iv_f64(d_price, d_ivopts, total_out, d_iv, st));
+    RB_TRY(launch_reduce_iv(d_partial, ReduceRows{d_row_off, d_row_n, d_row_M, 0, 0}, d_ivopts, total_out, d_price,
+                            d_stat, d_iv, nullptr, st));
     mark(s);
     return ST_OK;
 }

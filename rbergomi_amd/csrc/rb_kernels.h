@@ -37,22 +37,18 @@ inline hipError_t launch_volterra_conv_f64(const double* Z, long zstride, long n
 hipError_t launch_scan_f64(int method, const double* Z, long zstride, const double* Wt, long np,
                            int N, const Group* groups, int ngroups, const double* comp,
                            double* out, hipStream_t st, double sign = 1.0);
-hipError_t launch_payoff_f64(const double* ints, long np, long p0, const Option* opts,
-                             int out_size, int method, long blk0, long nblk_total,
-                             double* partial, double* payoff, hipStream_t st);
-hipError_t launch_reduce_f64(const double* partial, long nblk, long M, int out_size,
-                             double* price, double* stat, hipStream_t st);
-hipError_t launch_reduce_rows(const double* partial, const long* row_off, const long* row_n,
-                              const long* row_M, int nrows, double* price, double* stat,
-                              hipStream_t st);
-// launch_reduce_rows and launch_iv_f64 in one kernel, which also sets *counter to zero (nrows >= 1)
-hipError_t launch_reduce_rows_iv(const double* partial, const long* row_off, const long* row_n,
-                                 const long* row_M, const Option* opts, int nrows, double* price,
-                                 double* stat, double* iv, int* counter, hipStream_t st);
+// Prices, standard errors, implied vols (iv may be null) of rows of (sum, sum of squares) pairs, and
+// *counter (may be null) to zero (rb_reduce.hip): row I has n[I] pairs at partial + off[I] over M[I]
+// paths, or where these are null all_n pairs, rows one after another, and all_M paths
+struct ReduceRows {
+    const long *off, *n, *M;
+    long all_n, all_M;
+};
+hipError_t launch_reduce_iv(const double* partial, const ReduceRows& rows, const Option* opts, int nrows, double* price,
+                            double* stat, double* iv, int* counter, hipStream_t st);
+hipError_t launch_iv(const double* price, const Option* opts, int nrows, double* iv, hipStream_t st);
 hipError_t launch_iv_ref_f64(const double* price, const double* K, const double* T, int n, double* iv,
                              hipStream_t st);
-hipError_t launch_iv_f64(const double* price, const Option* opts, int n, double* iv,
-                         hipStream_t st);
 hipError_t launch_philox_probe(const void* ctr, PhiloxKey key, long n, void* out, hipStream_t st);
 // MFMA layout probe (rb_probe.hip)
 hipError_t launch_probe_mfma_layout(const float* A, const float* B, float* out, int mode,

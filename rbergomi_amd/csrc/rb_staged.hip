@@ -9,10 +9,7 @@
 //   k_scan_rt_f64    Sum v, Sum sqrt(v) W1 per (path, group)
 //                                              <- scaleWtilde/updateV/intVdt/intRootVdW (:73-80,163-167,427-436)
 //   k_scan_mc_f64    log S per (path, group)   <- updateZ/scaleZ/updateS (:111-136)
-//   k_payoff_f64     payoff per (path, option), block partial sums in FP64
-//                                              <- BS_call_price / posPart (:383-391, :264-266)
-//   k_reduce_f64     ordered sum of block partials -> price, stat   (:404-409)
-//   k_iv_f64         implied vols                                    (IV_call, :421-423)
+// Payoffs and sums: rb_payoff64.hip, rb_reduce.hip.
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -246,152 +243,6 @@ k_scan_mc_f64(const double* __restrict__ Z, long zstride, const double* __restri
     }
 }
 
-// ---------------------------------------------------------------- payoffs
-// Grid (path tiles of 256, options).  Block sums (payoff, payoff^2) in FP64 with a fixed tree;
-// partial[(I*nblk_total + blk0 + blockIdx.x)*2 + {0,1}].  If payoff != nullptr the per-path
-// payoffs are also written at payoff[(p0+p)*out_size + I] (quadrature layout).
-__global__ void __launch_bounds__(256)
-k_payoff_f64(const double* __restrict__ ints, long np, long p0, const Option* __restrict__ opts,
-             int out_size, int method, long blk0, long nblk_total, double* __restrict__ partial,
-             double* __restrict__ payoff) {
-    __shared__ double s1[256], s2[256];
-    const int I = blockIdx.y;
-    const Option o = opts[I];
-    const long p = long(blockIdx.x) * 256 + threadIdx.x;
-    double x = 0.0;
-    if (p < np) {
-        const double* iv = ints + (long(o.group) * np + p) * 2;
-        if (method == METHOD_RT) {
-            x = rt_payoff_f64(iv[0], iv[1], o.rho, o.K, o.lnK);
-        } else {
-            const double S = exp(iv[0]);
-            x = S - o.K > 0.0 ? S - o.K : 0.0;
-        }
-        if (payoff) payoff[(p0 + p) * out_size + I] = x;
-    }
-    s1[threadIdx.x] = x;
-    s2[threadIdx.x] = x * x;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            s1[threadIdx.x] += s1[threadIdx.x + off];
-            s2[threadIdx.x] += s2[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && partial) {
-        double* d = partial + (long(I) * nblk_total + blk0 + blockIdx.x) * 2;
-        d[0] = s1[0];
-        d[1] = s2[0];
-    }
-}
-
-// One block per option: ordered strided sums then a fixed tree => deterministic.
-// price = S/M, stat = sqrt(S2/M - price^2)/sqrt(M)   (rBergLib/rBergomiMT.cpp:404-409)
-__global__ void __launch_bounds__(256)
-k_reduce_f64(const double* __restrict__ partial, long nblk, int stride_blk, long M,
-             double* __restrict__ price, double* __restrict__ stat) {
-    __shared__ double s1[256], s2[256];
-    const int I = blockIdx.x;
-    double a = 0.0, b = 0.0;
-    for (long k = threadIdx.x; k < nblk; k += 256) {
-        const double* d = partial + (long(I) * nblk + k) * stride_blk;
-        a += d[0];
-        b += d[1];
-    }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            s1[threadIdx.x] += s1[threadIdx.x + off];
-            s2[threadIdx.x] += s2[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double m = double(M);
-        const double pr = s1[0] / m;
-        price[I] = pr;
-        stat[I] = sqrt(s2[0] / m - pr * pr) / sqrt(m);
-    }
-}
-
-// One block per output row: rows of (sum, sum of squares) pairs at partial + row_off[b],
-// row_n[b] pairs long; same ordered strided sums and fixed tree as k_reduce_f64.
-__global__ void __launch_bounds__(256)
-k_reduce_rows(const double* __restrict__ partial, const long* __restrict__ row_off,
-              const long* __restrict__ row_n, const long* __restrict__ row_M,
-              double* __restrict__ price, double* __restrict__ stat) {
-    __shared__ double s1[256], s2[256];
-    const int I = blockIdx.x;
-    const double* base = partial + row_off[I];
-    const long n = row_n[I];
-    double a = 0.0, b = 0.0;
-    for (long k = threadIdx.x; k < n; k += 256) {
-        a += base[2 * k];
-        b += base[2 * k + 1];
-    }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            s1[threadIdx.x] += s1[threadIdx.x + off];
-            s2[threadIdx.x] += s2[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double m = double(row_M[I]);
-        const double pr = s1[0] / m;
-        price[I] = pr;
-        stat[I] = sqrt(s2[0] / m - pr * pr) / sqrt(m);
-    }
-}
-
-// k_reduce_rows and k_iv_f64 in one launch (the same sums, the same vols), and the fused
-// kernel's item counter set back to zero for the batch's next launch
-__global__ void __launch_bounds__(256)
-k_reduce_rows_iv(const double* __restrict__ partial, const long* __restrict__ row_off,
-                 const long* __restrict__ row_n, const long* __restrict__ row_M,
-                 const Option* __restrict__ opts, double* __restrict__ price, double* __restrict__ stat,
-                 double* __restrict__ iv, int* __restrict__ counter) {
-    __shared__ double s1[256], s2[256];
-    const int I = blockIdx.x;
-    const double* base = partial + row_off[I];
-    const long n = row_n[I];
-    double a = 0.0, b = 0.0;
-    for (long k = threadIdx.x; k < n; k += 256) {
-        a += base[2 * k];
-        b += base[2 * k + 1];
-    }
-    s1[threadIdx.x] = a;
-    s2[threadIdx.x] = b;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            s1[threadIdx.x] += s1[threadIdx.x + off];
-            s2[threadIdx.x] += s2[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double m = double(row_M[I]);
-        const double pr = s1[0] / m;
-        price[I] = pr;
-        stat[I] = sqrt(s2[0] / m - pr * pr) / sqrt(m);
-        iv[I] = implied_vol_f64(pr, opts[I].K, opts[I].T);
-        if (I == 0) *counter = 0;
-    }
-}
-
-__global__ void k_iv_f64(const double* __restrict__ price, const Option* __restrict__ opts,
-                         int n, double* __restrict__ iv) {
-    const int I = blockIdx.x * blockDim.x + threadIdx.x;
-    if (I < n) iv[I] = implied_vol_f64(price[I], opts[I].K, opts[I].T);
-}
-
 // implied vols to the reference's tolerance (implied_vol_reference_f64)
 __global__ void k_iv_ref_f64(const double* __restrict__ price, const double* __restrict__ K,
                              const double* __restrict__ T, int n, double* __restrict__ iv) {
@@ -500,46 +351,6 @@ hipError_t launch_scan_f64(int method, const double* Z, long zstride, const doub
     else
         hipLaunchKernelGGL(k_scan_mc_f64, grid, dim3(256), 0, st, Z, zstride, Wt, np, N, groups,
                            ngroups, comp, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_payoff_f64(const double* ints, long np, long p0, const Option* opts,
-                             int out_size, int method, long blk0, long nblk_total,
-                             double* partial, double* payoff, hipStream_t st) {
-    dim3 grid(unsigned((np + 255) / 256), unsigned(out_size));
-    hipLaunchKernelGGL(k_payoff_f64, grid, dim3(256), 0, st, ints, np, p0, opts, out_size, method,
-                       blk0, nblk_total, partial, payoff);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_f64(const double* partial, long nblk, long M, int out_size,
-                             double* price, double* stat, hipStream_t st) {
-    hipLaunchKernelGGL(k_reduce_f64, dim3(out_size), dim3(256), 0, st, partial, nblk, 2, M, price,
-                       stat);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_rows(const double* partial, const long* row_off, const long* row_n,
-                              const long* row_M, int nrows, double* price, double* stat,
-                              hipStream_t st) {
-    if (nrows < 1) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_rows, dim3(nrows), dim3(256), 0, st, partial, row_off, row_n, row_M,
-                       price, stat);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_rows_iv(const double* partial, const long* row_off, const long* row_n,
-                                 const long* row_M, const Option* opts, int nrows, double* price,
-                                 double* stat, double* iv, int* counter, hipStream_t st) {
-    if (nrows < 1) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_rows_iv, dim3(nrows), dim3(256), 0, st, partial, row_off, row_n, row_M,
-                       opts, price, stat, iv, counter);
-    return hipGetLastError();
-}
-
-hipError_t launch_iv_f64(const double* price, const Option* opts, int n, double* iv,
-                         hipStream_t st) {
-    hipLaunchKernelGGL(k_iv_f64, dim3((n + 63) / 64), dim3(64), 0, st, price, opts, n, iv);
     return hipGetLastError();
 }
 

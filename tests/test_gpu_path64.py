@@ -76,6 +76,22 @@ def test_seeded_prices_match_oracle(rb, orc, units, mats, N, method):
     assert np.max(np.abs(stat - st)) < 1e-12
 
 
+# payoff sums of one, two and four paths per thread, each with a ragged last block, on 33 options (two
+# jobs); the oracle prices the same paths
+@pytest.mark.parametrize("M", [1000, (1 << 19) + 257, (1 << 20) + 1031])
+@pytest.mark.parametrize("method", [0, 1])
+def test_payoff_sums_of_several_paths_per_thread(rb, orc, M, method):
+    print("payoff sums M=%d method=%d" % (M, method), flush=True)
+    xi, N, seed = 0.04, 3, [M]
+    K = np.exp(np.linspace(-0.4, 0.3, 33))
+    price, _, stat = rb.price_v2(xi, [0.1], [1.9], [-0.7], np.full(33, 0.7), K, N, M, seed, method=method)
+    fn = orc.payoff_mc_samples if method else orc.payoff_rt_samples
+    pay = fn(xi, [0.1], [1.9], [-0.7], np.full(33, 0.7), K, N, orc.normals_philox(seed, 0, M, 3 if method else 2, N))
+    pr, st = orc.price_stat(pay)
+    assert np.max(np.abs(price - pr)) < 1e-12
+    assert np.max(np.abs(stat - st)) < 1e-12
+
+
 def test_extreme_coefficients_stay_finite_where_the_model_is(rb):
     """eta = 0 (the integrand is exactly xi past the last step's pad), and an eta whose exponents
     underflow: prices of the first are Black-Scholes on xi, none is NaN"""

@@ -4,7 +4,10 @@ host, against long double: 2^(y/32), -2 ln u, and Box-Muller on edge and random 
 Bounds, in units of eps = 2^-52: exp2 rounds a table entry (1/2), a product folded into one FMA
 (1/2) and carries a fit error of 0.4, so 1.5 eps bounds it; the logarithm adds a table term and a
 polynomial (two roundings of terms not larger than twice the result), 2 eps; the normals relative to
-their radius add a square root, a product and a polynomial of one rounding each, 3 eps."""
+their radius add a square root, a product and a polynomial of one rounding each, 3 eps.  A payoff is a
+sum of S', K and two tails, each rounded a few times: 8 eps of S' + K (to first order it does not
+depend on the rounding of d1, since S' phi(d1) = K phi(d2)); zero variance gives the intrinsic value,
+and NaN at the money as 0 / 0 does."""
 import os
 import shutil
 import subprocess
@@ -44,7 +47,25 @@ int main() {
         const long double th = 2 * acosl(-1.0L) * (((long double)x1 + 0.5L) * 0x1p-32L), rad = sqrtl(w);
         e_bm = fmaxl(e_bm, fmaxl(fabsl(z0 - rad * cosl(th)), fabsl(z1 - rad * sinl(th))) / rad);
     }
-    std::printf("%.4Lf %.4Lf %.4Lf\n", e_exp / 0x1p-52L, e_log / 0x1p-52L, e_bm / 0x1p-52L);
+    long double e_pay = 0;
+    for (int i = 0; i < 300000; ++i) {
+        auto u = [&] { return double(g() >> 11) * 0x1p-53; };
+        PathRt64 q;
+        q.lnS = (u() - 0.5) * (i & 1 ? 0.6 : 6.0);
+        q.sig = i % 3 ? exp(-9.0 * u()) * 1.5 : 0.05 + u();
+        q.S = exp(q.lnS);
+        q.isig = 1.0 / q.sig;
+        const double K = exp((u() - 0.5) * 1.5), lnK = log(K);
+        const long double S = expl((long double)q.lnS), d1 = ((long double)q.lnS - logl(K)) / q.sig + q.sig / 2.0L, d2 = d1 - q.sig;
+        const long double want = 0.5L * (S * erfcl(-d1 * sqrtl(0.5L)) - K * erfcl(-d2 * sqrtl(0.5L)));
+        e_pay = fmaxl(e_pay, fabsl(rt_payoff64(EXP2_TAB, q, K, lnK) - want) / (S + K));
+    }
+    auto at = [](double lnS, double K) {
+        PathRt64 q{lnS, exp(lnS), 0.0, INFINITY};
+        return rt_payoff64(EXP2_TAB, q, K, log(K));
+    };
+    std::printf("%.4Lf %.4Lf %.4Lf %.4Lf\n", e_exp / 0x1p-52L, e_log / 0x1p-52L, e_bm / 0x1p-52L, e_pay / 0x1p-52L);
+    std::printf("%.17g %.17g %.17g\n", at(0.0, 0.5), at(0.0, 2.0), at(0.0, 1.0));
     std::printf("%.17g %.17g %.17g %.17g\n", exp2_32(EXP2_TAB, 1e300), exp2_32(EXP2_TAB, -1e300), exp2_32(EXP2_TAB, 0.0),
                 exp2_32(EXP2_TAB, 32.0 * 1023));
     return 0;
@@ -71,7 +92,9 @@ def test_elementary_functions(tmp_path):
     assert r.returncode == 0, r.stderr[-3000:]
     out = subprocess.run([exe], capture_output=True, text=True, timeout=600)
     assert out.returncode == 0
-    first, second = out.stdout.strip().splitlines()
-    e_exp, e_log, e_bm = (float(x) for x in first.split())
-    assert e_exp < 1.5 and e_log < 2.0 and e_bm < 3.0, first
+    first, zero, second = out.stdout.strip().splitlines()
+    e_exp, e_log, e_bm, e_pay = (float(x) for x in first.split())
+    assert e_exp < 1.5 and e_log < 2.0 and e_bm < 3.0 and e_pay < 8.0, first
+    inside, outside, at_money = (float(x) for x in zero.split())
+    assert (inside, outside) == (0.5, 0.0) and at_money != at_money
     assert [float(x) for x in second.split()] == [float("inf"), 0.0, 1.0, float(2 ** 1023)]

@@ -336,8 +336,22 @@ int Plan::commit(std::string& err) {
         *m.first = base + at;
         at += (m.second + 255) / 256 * 256;
     }
-    // `up` outlives the copy: it is the plan's, and the plan waits for its stream before it goes
-    if (!up.empty()) RB_TRY(hipMemcpyAsync(base, up.data(), up.size(), hipMemcpyHostToDevice, stream));
+    // tables and results share a pinned block (the copy reads it and the last kernel writes it without
+    // the host waiting); it is the plan's, and the plan waits for its stream before it goes
+    const size_t res = (up.size() + 255) / 256 * 256;
+    unsigned char* h = host.reserve(res + 3 * lay.options.size() * sizeof(double));
+    if (!h) {
+        err = "cannot allocate pinned host memory";
+        return ST_ERR_NOMEM;
+    }
+    d_price = reinterpret_cast<double*>(h + res);
+    d_stat = d_price + lay.options.size();
+    d_iv = d_stat + lay.options.size();
+    if (!up.empty()) {
+        std::memcpy(h, up.data(), up.size());
+        RB_TRY(hipMemcpyAsync(base, h, up.size(), hipMemcpyHostToDevice, stream));
+    }
+    std::vector<char>().swap(up);
     return ST_OK;
 }
 
@@ -350,7 +364,7 @@ Plan::~Plan() {
     if (stream) (void)hipStreamSynchronize(stream);
     ws_free(d_block);  // the stream has synchronized above
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
-    if (own_stream && stream) (void)hipStreamDestroy(stream);
+    if (own_stream && stream) stream_put(stream, device);
 }
 
 int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& err) {
@@ -385,7 +399,7 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if (st) {
         stream = st;
     } else {
-        RB_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        RB_TRY(stream_get(&stream));
         own_stream = true;
     }
     const bool split = fused_mode_of(r.precision) >= 0;  // a fused-kernel precision
@@ -417,6 +431,7 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if ((fft1 || (split && r.N > 1024)) && r.N <= 8192 && !quadrature && r.gauss == 0) {
         // long paths on device Gaussians (or any N on request): the single-launch FFT kernel
         fused_fft.reset(new FftFused());
+        fused_fft->to_host = true;
         const int rc = fused_fft->build(r, lay, device, stream, err);
         if (rc) return rc;
         nblk = fused_fft->args.nitems;
@@ -521,7 +536,6 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if (!path64) dalloc(&d_Wt, size_t(nunits) * chunk * N);
     dalloc(&d_ints, size_t(ngroups) * chunk * 2);
     dalloc(&d_partial, size_t(nopt) * nblk * 2);
-    dalloc(&d_price, size_t(3) * nopt);  // price, stat, iv
     if (quadrature) dalloc(&d_payoff, size_t(chunk) * nopt);
     if (r.turbo) {
         dalloc(&d_ints2, size_t(ngroups) * chunk * 2);
@@ -532,8 +546,6 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     }
     rc = commit(err);
     if (rc) return rc;
-    d_stat = d_price + nopt;
-    d_iv = d_stat + nopt;
     if (path64) {
         p64.units = d_units;
         p64.groups = d_p64groups;
@@ -891,20 +903,17 @@ int Plan::turbo_results(double* alpha, double* Q, long* exceptions, std::string&
 }
 
 int Plan::results(double* price, double* iv, double* stat, std::string& err) {
-    if (fused || fused_fft) {
-        const int rc = fused ? fused_batch->results(0, price, iv, stat, stream, err)
-                             : fused_fft->results(price, iv, stat, stream, err);
-        if (rc) return rc;
-        RB_TRY(hipStreamSynchronize(stream));
-        return ST_OK;
-    }
-    const size_t n = lay.options.size();
-    std::vector<double> got(3 * n);  // price, stat, iv
-    RB_TRY(hipMemcpyAsync(got.data(), d_price, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream));
     RB_TRY(hipStreamSynchronize(stream));
-    if (price) std::copy_n(got.begin(), n, price);
-    if (stat) std::copy_n(got.begin() + n, n, stat);
-    if (iv) std::copy_n(got.begin() + 2 * n, n, iv);
+    if (fused) {
+        fused_batch->fetch(0, price, iv, stat);
+    } else if (fused_fft) {
+        fused_fft->fetch(price, iv, stat);
+    } else {
+        const size_t n = lay.options.size();
+        if (price) std::copy_n(d_price, n, price);
+        if (stat) std::copy_n(d_stat, n, stat);
+        if (iv) std::copy_n(d_iv, n, iv);
+    }
     return ST_OK;
 }
 

@@ -11,6 +11,7 @@
 #include "rb_device.h"
 #include "rb_fused.h"
 #include "rb_fused_host.h"
+#include "rb_hostmem.h"
 #include "rb_path64.h"
 #include "rb_payoff64.h"
 #include "rb_types.h"
@@ -124,6 +125,7 @@ struct Plan {
     std::vector<std::pair<void**, size_t>> mem;    // buffers and their bytes
     std::vector<std::pair<void**, size_t>> up_at;  // uploaded tables and their places in `up`
     std::vector<char> up;
+    Pinned host;                                   // `up` on its way to the device, and the results
     template <class T>
     void dalloc(T** p, size_t n);
     template <class T>
@@ -143,6 +145,7 @@ struct Plan {
     double* d_Wt = nullptr;       // [units][chunk][N]
     double* d_ints = nullptr;     // [groups][chunk][2]
     double* d_partial = nullptr;  // [options][nblk][2]
+    // results, in the plan's pinned host memory: the reduction writes them there
     double* d_price = nullptr;
     double* d_stat = nullptr;
     double* d_iv = nullptr;

@@ -377,14 +377,6 @@ int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHos
     } while (0)
 
 template <class T>
-static hipError_t upload_vec(T** p, const std::vector<T>& v, hipStream_t st) {
-    // stream-ordered allocation: freeing a batch never waits for other streams
-    hipError_t e = hipMallocAsync(reinterpret_cast<void**>(p), std::max<size_t>(v.size(), 1) * sizeof(T), st);
-    if (e != hipSuccess || v.empty()) return e;
-    return hipMemcpyAsync(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
-}
-
-template <class T>
 static hipError_t alloc_async(T** p, size_t n, hipStream_t st) {
     return hipMallocAsync(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(T), st);
 }
@@ -463,6 +455,10 @@ std::vector<std::pair<int, int>> FusedBatch::split(const std::vector<const Fused
 FusedBatch::~FusedBatch() { release(); }
 
 void FusedBatch::release() {
+    // the stream reads and writes the pinned blocks until it has passed the launch
+    if (up.data() || out.data()) (void)hipStreamSynchronize(stream);
+    up.release();
+    out.release();
     if (d_block && !arena) (void)hipFreeAsync(d_block, stream);
     d_block = nullptr;
     d_reqs = nullptr;
@@ -683,7 +679,8 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
                  o_ireq = place(item_req.size() * sizeof(int)), o_iloc = place(item_local.size() * sizeof(int)),
                  o_reqs = place(R.size() * sizeof(FusedReq)), o_cnt = place(sizeof(int));
     const size_t up_bytes = off;
-    const size_t o_part = place(size_t(poff) * sizeof(double)), o_out = place(size_t(total_out) * 3 * sizeof(double));
+    const size_t res_bytes = std::max<size_t>(1, size_t(total_out) * 3 * sizeof(double));
+    const size_t o_part = place(size_t(poff) * sizeof(double)), o_out = place(to_host ? 1 : res_bytes);
     RB_TRY(batch_alloc(arena, &d_block, off, st));
     d_fu = reinterpret_cast<FusedUnit*>(d_block + o_fu);
     d_fg = reinterpret_cast<FusedGroup*>(d_block + o_fg);
@@ -701,7 +698,11 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
     d_counter = reinterpret_cast<int*>(d_block + o_cnt);
     counter_dirty = false;
     d_partial = reinterpret_cast<double*>(d_block + o_part);
-    d_price = reinterpret_cast<double*>(d_block + o_out);
+    d_price = reinterpret_cast<double*>(to_host ? reinterpret_cast<char*>(out.reserve(res_bytes)) : d_block + o_out);
+    if (!d_price) {
+        err = "cannot allocate pinned host memory";
+        return ST_ERR_NOMEM;
+    }
     d_iv = d_price + total_out;
     d_stat = d_price + 2 * size_t(total_out);
     for (FusedReq& r : R) {
@@ -713,10 +714,10 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
         r.ptab = d_ptab;
         r.partial = d_partial + size_t(r.partial);
     }
-    unsigned char* h = stage ? stage(up_bytes) : nullptr;
+    unsigned char* h = arena ? nullptr : up.reserve(up_bytes);
     const bool staged = h != nullptr;
     if (staged) {
-        // packed into the caller's pinned staging: one copy, not waited for
+        // packed into pinned memory: one copy, not waited for
         auto pack = [&](size_t o, const auto& v) {
             if (!v.empty()) std::memcpy(h + o, v.data(), v.size() * sizeof(v[0]));
         };
@@ -791,6 +792,13 @@ int FusedBatch::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_
     return ST_OK;
 }
 
+void FusedBatch::fetch(int q, double* price, double* iv, double* stat) const {
+    const long a = out_off[q], b = out_off[q + 1];
+    if (price) std::copy(d_price + a, d_price + b, price);
+    if (iv) std::copy(d_iv + a, d_iv + b, iv);
+    if (stat) std::copy(d_stat + a, d_stat + b, stat);
+}
+
 int FusedBatch::results(int q, double* price, double* iv, double* stat, hipStream_t st,
                         std::string& err) {
     const size_t n = size_t(out_off[q + 1] - out_off[q]) * sizeof(double);
@@ -804,10 +812,12 @@ int FusedBatch::results(int q, double* price, double* iv, double* stat, hipStrea
 FftFused::~FftFused() { release(); }
 
 void FftFused::release() {
-    void* bufs[] = {d_fu, d_fg, d_fpg, d_fo, d_ptab, d_ghat, d_tw, d_partial, d_counter, d_row_off, d_row_n,
-                    d_row_M, d_price, d_stat, d_iv, d_ivopts};
-    for (void* b : bufs)
-        if (b) (void)hipFreeAsync(b, stream);
+    // the stream reads and writes the pinned blocks until it has passed the launch
+    if (up.data() || out.data()) (void)hipStreamSynchronize(stream);
+    up.release();
+    out.release();
+    if (d_block) (void)hipFreeAsync(d_block, stream);
+    d_block = nullptr;
     d_fu = nullptr;
     d_fg = nullptr;
     d_fpg = nullptr;
@@ -921,22 +931,61 @@ int FftFused::build(const Request& req, const Layout& lay, int device, hipStream
     }
     std::vector<long> row_off(a.out_size), row_n(a.out_size, a.nitems), row_M(a.out_size, a.M);
     for (int I = 0; I < a.out_size; ++I) row_off[I] = long(I) * a.nitems * 2;
-    RB_TRY(upload_vec(&d_fu, tabs.fu, st));
-    RB_TRY(upload_vec(&d_fg, tabs.fg, st));
-    RB_TRY(upload_vec(&d_fpg, tabs.fpg, st));
-    RB_TRY(upload_vec(&d_fo, tabs.fo, st));
-    RB_TRY(upload_vec(&d_ptab, tabs.ptab, st));
-    RB_TRY(upload_vec(&d_ghat, gh, st));
-    RB_TRY(upload_vec(&d_tw, tw, st));
-    RB_TRY(upload_vec(&d_row_off, row_off, st));
-    RB_TRY(upload_vec(&d_row_n, row_n, st));
-    RB_TRY(upload_vec(&d_row_M, row_M, st));
-    RB_TRY(upload_vec(&d_ivopts, lay.options, st));
-    RB_TRY(alloc_async(&d_partial, size_t(a.out_size) * a.nitems * 2, st));
-    RB_TRY(alloc_async(&d_counter, 1, st));
-    RB_TRY(alloc_async(&d_price, size_t(a.out_size), st));
-    RB_TRY(alloc_async(&d_stat, size_t(a.out_size), st));
-    RB_TRY(alloc_async(&d_iv, size_t(a.out_size), st));
+    // one device block: the tables (one upload from pinned memory, not waited for), then the partial
+    // sums, the item counter and the results
+    size_t off = 0;
+    auto place = [&](size_t bytes) {
+        const size_t o = off;
+        off += (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
+        return o;
+    };
+    const size_t o_fu = place(tabs.fu.size() * sizeof(FusedUnit)), o_fg = place(tabs.fg.size() * sizeof(FusedGroup)),
+                 o_fpg = place(tabs.fpg.size() * sizeof(FusedPG)), o_fo = place(tabs.fo.size() * sizeof(FusedOption)),
+                 o_ptab = place(tabs.ptab.size() * sizeof(float)), o_gh = place(gh.size() * sizeof(float2)),
+                 o_tw = place(tw.size() * sizeof(float2)), o_roff = place(row_off.size() * sizeof(long)),
+                 o_rn = place(row_n.size() * sizeof(long)), o_rm = place(row_M.size() * sizeof(long)),
+                 o_ivo = place(lay.options.size() * sizeof(Option));
+    const size_t up_bytes = off;
+    const size_t res_bytes = size_t(a.out_size) * 3 * sizeof(double);
+    const size_t o_part = place(size_t(a.out_size) * a.nitems * 2 * sizeof(double)), o_cnt = place(sizeof(int)),
+                 o_out = place(to_host ? 1 : res_bytes);
+    RB_TRY(alloc_async(&d_block, off, st));
+    d_fu = reinterpret_cast<FusedUnit*>(d_block + o_fu);
+    d_fg = reinterpret_cast<FusedGroup*>(d_block + o_fg);
+    d_fpg = reinterpret_cast<FusedPG*>(d_block + o_fpg);
+    d_fo = reinterpret_cast<FusedOption*>(d_block + o_fo);
+    d_ptab = reinterpret_cast<float*>(d_block + o_ptab);
+    d_ghat = reinterpret_cast<float2*>(d_block + o_gh);
+    d_tw = reinterpret_cast<float2*>(d_block + o_tw);
+    d_row_off = reinterpret_cast<long*>(d_block + o_roff);
+    d_row_n = reinterpret_cast<long*>(d_block + o_rn);
+    d_row_M = reinterpret_cast<long*>(d_block + o_rm);
+    d_ivopts = reinterpret_cast<Option*>(d_block + o_ivo);
+    d_partial = reinterpret_cast<double*>(d_block + o_part);
+    d_counter = reinterpret_cast<int*>(d_block + o_cnt);
+    unsigned char* h = up.reserve(up_bytes);
+    d_price = reinterpret_cast<double*>(to_host ? reinterpret_cast<char*>(out.reserve(res_bytes)) : d_block + o_out);
+    if (!h || !d_price) {
+        err = "cannot allocate pinned host memory";
+        return ST_ERR_NOMEM;
+    }
+    d_iv = d_price + a.out_size;
+    d_stat = d_iv + a.out_size;
+    auto pack = [&](size_t o, const auto& v) {
+        if (!v.empty()) std::memcpy(h + o, v.data(), v.size() * sizeof(v[0]));
+    };
+    pack(o_fu, tabs.fu);
+    pack(o_fg, tabs.fg);
+    pack(o_fpg, tabs.fpg);
+    pack(o_fo, tabs.fo);
+    pack(o_ptab, tabs.ptab);
+    pack(o_gh, gh);
+    pack(o_tw, tw);
+    pack(o_roff, row_off);
+    pack(o_rn, row_n);
+    pack(o_rm, row_M);
+    pack(o_ivo, lay.options);
+    RB_TRY(hipMemcpyAsync(d_block, h, up_bytes, hipMemcpyHostToDevice, st));
     a.units = d_fu;
     a.groups = d_fg;
     a.pgs = d_fpg;
@@ -950,7 +999,6 @@ int FftFused::build(const Request& req, const Layout& lay, int device, hipStream
                                                                         : prop.sharedMemPerBlock);
     const int per_cu = int(std::max<size_t>(1, std::min<size_t>(4, lds_cu / lds)));
     grid = int(std::min<long>(a.nitems, long(prop.multiProcessorCount) * per_cu));
-    RB_TRY(hipStreamSynchronize(st));
     return ST_OK;
 }
 
@@ -973,15 +1021,12 @@ int FftFused::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_t 
     return ST_OK;
 }
 
-int FftFused::results(double* price, double* iv, double* stat, hipStream_t st, std::string& err) {
-    const size_t n = size_t(total_out) * sizeof(double);
-    if (price) RB_TRY(hipMemcpyAsync(price, d_price, n, hipMemcpyDeviceToHost, st));
-    if (iv) RB_TRY(hipMemcpyAsync(iv, d_iv, n, hipMemcpyDeviceToHost, st));
-    if (stat) RB_TRY(hipMemcpyAsync(stat, d_stat, n, hipMemcpyDeviceToHost, st));
-    return ST_OK;
+void FftFused::fetch(double* price, double* iv, double* stat) const {
+    if (price) std::copy_n(d_price, total_out, price);
+    if (iv) std::copy_n(d_iv, total_out, iv);
+    if (stat) std::copy_n(d_stat, total_out, stat);
 }
 
-// ---------------------------------------------------------------- autotuning
 int autotune_fused(const Request& shape, const std::vector<int>& Ns, int mode, int device,
                    std::vector<int>& chosen, std::vector<double>& best_ms, std::string& err) {
     chosen.assign(Ns.size(), 0);
@@ -1057,6 +1102,7 @@ int Plan::init_fused(std::string& err) {
     int rc = plan_fused_request(req, lay, fused_mode, *fused_req, err);
     if (rc) return rc;
     fused_batch.reset(new FusedBatch());
+    fused_batch->to_host = true;
     rc = fused_batch->build({fused_req.get()}, fused_mode, device, stream, err);
     if (rc) return rc;
     nblk = fused_req->r.nitems;

@@ -4,10 +4,10 @@
 
 #include <string>
 #include <array>
-#include <functional>
 #include <vector>
 
 #include "rb_fused.h"
+#include "rb_hostmem.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -61,6 +61,11 @@ struct FftFused {
     double* d_stat = nullptr;
     double* d_iv = nullptr;
     Option* d_ivopts = nullptr;
+    char* d_block = nullptr;     // the one device allocation every pointer above points into
+    Pinned up, out;              // the tables on their way to the device; the results (to_host)
+    // results in pinned host memory, written there by the reduction, for fetch (set before build);
+    // otherwise in device memory, price | iv | stat, for the owner's copy
+    bool to_host = false;
 
     ~FftFused();
     void release();
@@ -70,7 +75,8 @@ struct FftFused {
     int build(const Request& req, const Layout& lay, int device, hipStream_t st, std::string& err);
     int launch(hipStream_t st, std::string& err, Plan* timing = nullptr, hipEvent_t kbeg = nullptr,
                hipEvent_t kend = nullptr);
-    int results(double* price, double* iv, double* stat, hipStream_t st, std::string& err);
+    // the results of the last launch (to_host), after the caller has waited for it
+    void fetch(double* price, double* iv, double* stat) const;
 };
 
 // Tile shape (path blocks per tile) per (padded N, operand mode, plain MC): an autotuned entry,
@@ -140,11 +146,13 @@ struct FusedBatch {
     char* d_block = nullptr;     // the one device allocation every pointer above points into
 
     DevArena* arena = nullptr;   // when set, buffers come from it (see DevArena)
-    // pinned host memory of at least the bytes asked for, or null: when set, build packs the
-    // tables there, copies them in one piece and returns without waiting for the copy (the
-    // caller keeps the memory untouched until the batch's stream has passed the launch);
-    // otherwise each table is copied from its host vector and build waits for the copies
-    std::function<unsigned char*(size_t)> stage;
+    // the tables on their way to the device (build packs them there and copies them in one piece,
+    // not waited for; an arena, which allocates nothing, copies each from its host vector and waits),
+    // and the results (to_host)
+    Pinned up, out;
+    // results in pinned host memory, written there by the reduction, for fetch (set before build);
+    // otherwise in device memory, price | iv | stat, for the owner's copy
+    bool to_host = false;
 
     ~FusedBatch();
     void release();
@@ -166,7 +174,9 @@ struct FusedBatch {
     // (may be null) are recorded on st right before and after the fused kernel
     int launch(hipStream_t st, std::string& err, Plan* timing = nullptr, hipEvent_t kbeg = nullptr,
                hipEvent_t kend = nullptr);
-    // enqueue the copies of request q's results (caller synchronizes the stream)
+    // the results of request q from the last launch (to_host), after the caller has waited for it
+    void fetch(int q, double* price, double* iv, double* stat) const;
+    // enqueue the copies of request q's results (not to_host; the caller synchronizes the stream)
     int results(int q, double* price, double* iv, double* stat, hipStream_t st, std::string& err);
 };
 

@@ -138,7 +138,6 @@ struct Flight {
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
     hipEvent_t kbeg = nullptr, kend = nullptr;  // around the pricing kernel (timing events)
-    double* pinned = nullptr;  // [3][total_out]: price, iv, stat
     std::vector<Job*> jobs;
     size_t footprint = 0;
 };
@@ -163,10 +162,6 @@ struct rb_server {
     std::map<long, std::unique_ptr<Job>> jobs;
     std::vector<std::unique_ptr<Flight>> flights;
     std::vector<hipStream_t> free_streams;
-    std::map<hipStream_t, std::pair<double*, size_t>> pinned;  // reusable result staging per stream
-    // reusable upload staging per stream (pinned: the batch's one table copy runs without the
-    // server thread waiting for it; a stream is reused only after its flight has completed)
-    std::map<hipStream_t, std::pair<unsigned char*, size_t>> upinned;
     size_t inflight_bytes = 0;
     bool stop = false;
     long next_ticket = 1;
@@ -201,7 +196,6 @@ bool rb_server::reap(std::unique_lock<std::mutex>& lk) {
             ++f;
             continue;
         }
-        const int total = F.batch ? F.batch->total_out : F.fft->total_out;
         const Clock::time_point now = Clock::now();
         if (q == hipSuccess && F.kbeg) {
             float a = 0.f, b = 0.f;
@@ -215,10 +209,8 @@ bool rb_server::reap(std::unique_lock<std::mutex>& lk) {
         for (size_t i = 0; i < F.jobs.size(); ++i) {
             Job& j = *F.jobs[i];
             if (q == hipSuccess) {
-                const long o = F.batch ? F.batch->out_off[i] : 0;
-                std::memcpy(j.price, F.pinned + o, j.out * sizeof(double));
-                if (j.iv) std::memcpy(j.iv, F.pinned + total + o, j.out * sizeof(double));
-                std::memcpy(j.stat, F.pinned + 2 * total + o, j.out * sizeof(double));
+                if (F.batch) F.batch->fetch(int(i), j.price, j.iv, j.stat);
+                else F.fft->fetch(j.price, j.iv, j.stat);
                 j.status = ST_OK;
                 latencies.push_back(std::chrono::duration<double, std::milli>(now - j.t_submit).count());
                 path_steps += double(j.req.M) * j.req.N;
@@ -278,7 +270,7 @@ bool rb_server::launch(std::unique_lock<std::mutex>& lk) {
     if (!free_streams.empty()) {
         F->stream = free_streams.back();
         free_streams.pop_back();
-    } else if (hipStreamCreateWithFlags(&F->stream, hipStreamNonBlocking) != hipSuccess) {
+    } else if (stream_get(&F->stream) != hipSuccess) {
         F->stream = nullptr;
     }
     lk.unlock();
@@ -297,70 +289,22 @@ bool rb_server::launch(std::unique_lock<std::mutex>& lk) {
             rc = ST_ERR_DEVICE;
         }
     }
-    int total = 0;
-    double* d_price = nullptr;
-    double* d_iv = nullptr;
-    double* d_stat = nullptr;
     if (take[0]->long_path) {
         F->fft.reset(new FftFused());
+        F->fft->to_host = true;
         if (!rc) rc = F->fft->build(take[0]->req, take[0]->lay, device, F->stream, err);
         if (!rc) rc = F->fft->launch(F->stream, err, nullptr, F->kbeg, F->kend);
-        if (!rc) {
-            total = F->fft->total_out;
-            d_price = F->fft->d_price;
-            d_iv = F->fft->d_iv;
-            d_stat = F->fft->d_stat;
-        }
     } else {
         std::vector<const FusedHostReq*> hr;
         for (Job* j : take) hr.push_back(&j->fh);
         F->batch.reset(new FusedBatch());
-        auto& up = upinned[F->stream];  // only the server thread touches the pool
-        F->batch->stage = [&up](size_t bytes) -> unsigned char* {
-            if (up.second < bytes) {
-                if (up.first) (void)hipHostFree(up.first);
-                up.first = nullptr;
-                up.second = 0;
-                if (hipHostMalloc(reinterpret_cast<void**>(&up.first), 2 * bytes) == hipSuccess) up.second = 2 * bytes;
-            }
-            return up.first;
-        };
-        const int mode = fused_mode_of(cfg.precision);
-        if (!rc) rc = F->batch->build(hr, mode, device, F->stream, err);
+        F->batch->to_host = true;
+        if (!rc) rc = F->batch->build(hr, fused_mode_of(cfg.precision), device, F->stream, err);
         if (!rc) rc = F->batch->launch(F->stream, err, nullptr, F->kbeg, F->kend);
-        if (!rc) {
-            total = F->batch->total_out;
-            d_price = F->batch->d_price;
-            d_iv = F->batch->d_iv;
-            d_stat = F->batch->d_stat;
-        }
     }
-    if (!rc) {
-        auto& pb = pinned[F->stream];  // only the server thread touches the pool
-        const size_t need = size_t(std::max(1, 3 * total));
-        if (pb.second < need) {
-            if (pb.first) (void)hipHostFree(pb.first);
-            pb.first = nullptr;
-            pb.second = 0;
-            if (hipHostMalloc(reinterpret_cast<void**>(&pb.first), 2 * need * sizeof(double)) == hipSuccess)
-                pb.second = 2 * need;
-        }
-        F->pinned = pb.first;
-        if (!F->pinned) rc = ST_ERR_NOMEM;
-    }
-    if (!rc) {
-        const size_t n = size_t(total) * sizeof(double);
-        // one copy when the results lie price | iv | stat in device memory (fused batches)
-        const bool adjacent = d_iv == d_price + total && d_stat == d_price + 2 * size_t(total);
-        if ((adjacent ? hipMemcpyAsync(F->pinned, d_price, 3 * n, hipMemcpyDeviceToHost, F->stream)
-                      : hipMemcpyAsync(F->pinned, d_price, n, hipMemcpyDeviceToHost, F->stream) ||
-                            hipMemcpyAsync(F->pinned + total, d_iv, n, hipMemcpyDeviceToHost, F->stream) ||
-                            hipMemcpyAsync(F->pinned + 2 * total, d_stat, n, hipMemcpyDeviceToHost, F->stream)) ||
-            hipEventCreateWithFlags(&F->done, hipEventDisableTiming) ||
-            hipEventRecord(F->done, F->stream)) {
-            err = "cannot enqueue the result copies";
-            rc = ST_ERR_DEVICE;
-        }
+    if (!rc && (hipEventCreateWithFlags(&F->done, hipEventDisableTiming) || hipEventRecord(F->done, F->stream))) {
+        err = "cannot record the batch's completion";
+        rc = ST_ERR_DEVICE;
     }
     lk.lock();
     if (rc) {
@@ -421,7 +365,7 @@ struct rb_batch {
         fused.clear();
         longs.clear();
         if (st) (void)hipStreamSynchronize(st);
-        if (own_stream && st) (void)hipStreamDestroy(st);
+        if (own_stream && st) stream_put(st, device);
     }
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -459,12 +403,14 @@ struct rb_batch {
         runs = FusedBatch::split(hr, lds_block, lds_cu, false);
         for (const std::pair<int, int>& run : runs) {
             fused.emplace_back(new FusedBatch());
+            fused.back()->to_host = true;
             const std::vector<const FusedHostReq*> part(hr.begin() + run.first, hr.begin() + run.second);
             rc = fused.back()->build(part, fused_mode_of(cfg.precision), device, st, err);
             if (rc) return rc;
         }
         for (int i : long_idx) {
             longs.emplace_back(new FftFused());
+            longs.back()->to_host = true;
             rc = longs.back()->build(jobs[i]->req, jobs[i]->lay, device, st, err);
             if (rc) return rc;
         }
@@ -510,20 +456,18 @@ int rb_batch::run(std::string& err) {
         const int rc = enqueue(err);
         if (rc) return rc;
     }
-    for (size_t r = 0; r < runs.size(); ++r)
-        for (int k = runs[r].first; k < runs[r].second; ++k) {
-            const Job& j = *jobs[short_idx[k]];
-            const int rc = fused[r]->results(k - runs[r].first, j.price, j.iv, j.stat, st, err);
-            if (rc) return rc;
-        }
-    for (size_t l = 0; l < long_idx.size(); ++l) {
-        const Job& j = *jobs[long_idx[l]];
-        const int rc = longs[l]->results(j.price, j.iv, j.stat, st, err);
-        if (rc) return rc;
-    }
     if (hipStreamSynchronize(st) != hipSuccess) {
         err = "batch execution failed on the device";
         return ST_ERR_DEVICE;
+    }
+    for (size_t r = 0; r < runs.size(); ++r)
+        for (int k = runs[r].first; k < runs[r].second; ++k) {
+            const Job& j = *jobs[short_idx[k]];
+            fused[r]->fetch(k - runs[r].first, j.price, j.iv, j.stat);
+        }
+    for (size_t l = 0; l < long_idx.size(); ++l) {
+        const Job& j = *jobs[long_idx[l]];
+        longs[l]->fetch(j.price, j.iv, j.stat);
     }
     return ST_OK;
 }
@@ -547,7 +491,7 @@ int rb_batch_create(const rb_request* reqs, int n, const rb_config* cfg, void* s
     if (!rc) {
         if (stream) {
             b->st = static_cast<hipStream_t>(stream);
-        } else if (hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking) == hipSuccess) {
+        } else if (stream_get(&b->st) == hipSuccess) {
             b->own_stream = true;
         } else {
             err = "cannot create a stream";
@@ -861,11 +805,7 @@ void rb_server_destroy(rb_server* s) {
     s->cv_work.notify_all();
     if (s->th.joinable()) s->th.join();
     for (hipStream_t st : s->free_streams) (void)hipStreamSynchronize(st);
-    for (auto& kv : s->pinned)
-        if (kv.second.first) (void)hipHostFree(kv.second.first);
-    for (auto& kv : s->upinned)
-        if (kv.second.first) (void)hipHostFree(kv.second.first);
-    for (hipStream_t st : s->free_streams) (void)hipStreamDestroy(st);
+    for (hipStream_t st : s->free_streams) stream_put(st, s->device);
     if (s->epoch) (void)hipEventDestroy(s->epoch);
     delete s;
 }

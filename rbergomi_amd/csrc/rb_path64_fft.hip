@@ -15,7 +15,9 @@
 // What bounds it: FP64 vector issue; per pair and 64 steps about 330 instructions of Gaussians, 70 of
 // each group and 45 log2 L of the transforms (six-FMA butterflies, rb_fft64.h), where the
 // triangular product on the matrix cores (which keep the vector unit) takes N / 2.  A thread's 16
-// points and 16 steps of each stream fill the registers of two waves per SIMD (4 to 54 spilled),
+// points and 16 steps of each stream fill the registers of two waves per SIMD (4 to 26 spilled for
+// plain MC, none or 4 for Romano-Touzi; with the passes' twiddles hoisted out of the loop over the jobs
+// 40 to 100, and N = 512 took 1.19 ms per 1.6e8 path steps where it takes 1.08, N = 4096 2.23, now 1.72),
 // and its 17 KB of LDS per wave the CU's.  N = 2048, M = 16384, one maturity: 3.05 (k_normals,
 // k_volterra_mfma_long, k_scan) -> 0.29 ms; 1.2e11 paths*steps/s at N = 1024 and 2048.
 #include <hip/hip_runtime.h>
@@ -219,7 +221,12 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
 #pragma unroll
                 for (int r = 0; r < 4; ++r) z[fpad64(4 * (t + TP * j) + r)] = w1[j][r];
         }
-        const Fft64Run<LOG2L, Sync> fft{z, A.tw, t, sync};
+        // the twiddles' address is hidden from the loop over the jobs: hoisted out of it, every pass's
+        // twiddles would stay in registers (40 to 100 spilled)
+        int hide = 0;
+        asm volatile("" : "+s"(hide));
+        const double2* tw = A.tw + hide;
+        const Fft64Run<LOG2L, Sync> fft{z, tw, t, sync};
         {
             double2 x[16];
             fft.forward(x);

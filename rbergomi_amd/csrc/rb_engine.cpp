@@ -372,9 +372,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if (rc) return rc;
     req = r;
     path64 = r.precision == PREC_FP64 && r.scheme == SCHEME_HYBRID && r.N <= PATH64_FFT_MAX_N;
+    // long paths on device Gaussians (or any N on request): the FFT kernel, which forms its own Gamma
+    const bool split = fused_mode_of(r.precision) >= 0;  // a fused-kernel precision
+    const bool fft1 = r.precision == PREC_FP32_FFT;      // the FFT kernel at every N
+    const bool on_fft = (fft1 || (split && r.N > 1024)) && r.N <= 8192 && !quadrature && r.gauss == 0;
     // the staged scan's compensator table: the staged FP64 and FP32 paths, and caller's or Sobol'
     // Gaussians at a mixed precision
-    lay = make_layout(r, !path64, !path64 && (r.precision == PREC_FP64 || r.precision == PREC_FP32 || quadrature || r.gauss >= 1));
+    lay = make_layout(r, !path64 && !on_fft, !path64 && (r.precision == PREC_FP64 || r.precision == PREC_FP32 || quadrature || r.gauss >= 1));
     int ndev = 0;
     RB_TRY(hipGetDeviceCount(&ndev));
     if (ndev < 1) {
@@ -402,7 +406,6 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         RB_TRY(stream_get(&stream));
         own_stream = true;
     }
-    const bool split = fused_mode_of(r.precision) >= 0;  // a fused-kernel precision
     if (r.turbo && (r.precision != PREC_FP64 || r.method != METHOD_RT || quadrature)) {
         err = "the turbo-charged estimator runs the Romano-Touzi FP64 path on device Gaussians";
         return ST_ERR_ARG;
@@ -427,15 +430,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         err = "the Cholesky scheme covers N <= 2048";
         return ST_ERR_LIMIT;
     }
-    const bool fft1 = r.precision == PREC_FP32_FFT;  // the single-launch FFT kernel at every N
-    if ((fft1 || (split && r.N > 1024)) && r.N <= 8192 && !quadrature && r.gauss == 0) {
-        // long paths on device Gaussians (or any N on request): the single-launch FFT kernel
+    if (on_fft) {
         fused_fft.reset(new FftFused());
         fused_fft->to_host = true;
         const int rc = fused_fft->build(r, lay, device, stream, err);
         if (rc) return rc;
-        nblk = fused_fft->args.nitems;
-        chunk = r.M;
+        nblk = fused_fft->nblk;
+        chunk = fused_fft->chunk;
         return ST_OK;
     }
     if (r.precision == PREC_FP32 || ((split || fft1) && (r.N > 1024 || quadrature || r.gauss >= 1))) {
@@ -478,10 +479,8 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         const long cap = std::atol(env);
         if (cap > 0) ch = std::min(ch, cap);
     }
-    // paths per payoff thread, so that a block's sums cover 256 ppt paths: as many as leave 2048
-    // blocks of the whole option table (one per thread otherwise, and in the turbo-charged estimator)
-    ppt = r.turbo ? 1 : 4;
-    while (ppt > 1 && r.M / (256L * ppt) * ((nopt + PAY64_OPTS - 1) / PAY64_OPTS) < 2048) ppt /= 2;
+    // one path per payoff thread in the turbo-charged estimator, whose own payoff kernel sums 256
+    ppt = r.turbo ? 1 : payoff_paths_per_thread(r.M, nopt);
     const long pblk = 256L * ppt;
     ch = std::max(pblk, ch / pblk * pblk);
     const long Mr = (r.M + pblk - 1) / pblk * pblk;
@@ -680,7 +679,8 @@ int Plan::enqueue(std::string& err) {
             RB_LAUNCH(K_PAYOFF, launch_turbo_payoff(d_ints, d_ints2, np, d_opts, nopt, d_Qg, d_alpha,
                                                     req.q_max, p0 / 256, nblk, d_partial, d_exc, stream));
         } else {
-            RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt, req.method,
+            RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt,
+                                                req.method == METHOD_MC ? PAY_MC64 : PAY_RT64,
                                                 p0 / (256 * ppt), nblk, d_partial, nullptr, stream));
         }
     }
@@ -742,7 +742,8 @@ int Plan::run_samples(const double* Z_host, double* payoff_host, std::string& er
                               size_t(np) * nstreams * N * sizeof(double), hipMemcpyHostToDevice, stream));
         const int rc = integrals(0, np, true, 1, err);
         if (rc) return rc;
-        RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt, req.method,
+        RB_LAUNCH(K_PAYOFF, launch_payoff64(d_ints, np, ppt, d_payjobs, npayjobs, d_payopts, nopt,
+                                                req.method == METHOD_MC ? PAY_MC64 : PAY_RT64,
                                             p0 / (256 * ppt), nblk, d_partial, d_payoff, stream));
         RB_TRY(hipMemcpyAsync(payoff_host + size_t(p0) * nopt, d_payoff, size_t(np) * nopt * sizeof(double),
                               hipMemcpyDeviceToHost, stream));
@@ -806,27 +807,33 @@ int Plan::init_fft(std::string& err) {
     return ST_OK;
 }
 
-// Jobs of the payoff stage: runs of up to PAY64_OPTS options of one (group, rho), shorter where the
-// path blocks alone leave compute units without one.
-void Plan::init_payoffs() {
-    const int nopt = int(lay.options.size());
-    std::vector<int> order(nopt);
-    for (int I = 0; I < nopt; ++I) order[I] = I;
-    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-        const Option &a = lay.options[x], &b = lay.options[y];
-        return a.group != b.group ? a.group < b.group : a.rho < b.rho;
-    });
+void payoff_jobs(const std::vector<PayRow>& rows, long nblk, int cus, std::vector<PayJob64>& jobs,
+                 std::vector<PayOpt64>& opts) {
+    const int n = int(rows.size());
     int most = PAY64_OPTS;
-    while (most > 1 && nblk * ((nopt + most - 1) / most) < 4L * cus) most /= 2;
-    std::vector<PayJob64> jobs;
-    std::vector<PayOpt64> opts(nopt);
-    for (int k = 0; k < nopt; ++k) {
-        const Option& o = lay.options[order[k]];
-        opts[k] = PayOpt64{o.K, o.lnK, order[k], 0};
+    while (most > 1 && nblk * ((n + most - 1) / most) < 4L * cus) most /= 2;
+    jobs.clear();
+    opts.clear();
+    for (int k = 0; k < n; ++k) {
+        const PayRow& o = rows[k];
+        opts.push_back(PayOpt64{o.K, o.lnK, o.out, 0});
         if (jobs.empty() || jobs.back().group != o.group || jobs.back().rho != o.rho || jobs.back().n == most)
             jobs.push_back(PayJob64{o.group, k, 0, 0, o.rho});
         ++jobs.back().n;
     }
+}
+
+void Plan::init_payoffs() {
+    std::vector<PayRow> rows;
+    for (size_t I = 0; I < lay.options.size(); ++I) {
+        const Option& o = lay.options[I];
+        rows.push_back(PayRow{o.group, int(I), o.rho, o.K, o.lnK});
+    }
+    std::stable_sort(rows.begin(), rows.end(),
+                     [](const PayRow& a, const PayRow& b) { return a.group != b.group ? a.group < b.group : a.rho < b.rho; });
+    std::vector<PayJob64> jobs;
+    std::vector<PayOpt64> opts;
+    payoff_jobs(rows, nblk, cus, jobs, opts);
     npayjobs = int(jobs.size());
     upload(&d_payjobs, jobs);
     upload(&d_payopts, opts);

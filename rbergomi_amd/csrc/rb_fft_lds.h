@@ -220,22 +220,64 @@ __device__ __forceinline__ void fft_dif_inv_r4_t(float2* z, const float2* __rest
 //  - bit-reversed (fft_convolve_r16_br): forward by decimation in time from bit-reversed input to
 //    natural order, G in natural order, inverse by decimation in frequency to bit-reversed output.
 
+// Twiddles of a pass: W_{2^(SB + r + 1)}^{pos + 2^SB m}, m < max(1, 2^(r - 1)), from the plain table
+// tw[k] = exp(-2 pi i k / L), or from one ordered by pass, [8][2^SB] for stages r = 0, 1, 2, 3 from rows
+// 0, 1, 2, 4 on (consecutive lanes read consecutive entries, where the plain table's stride is up
+// to 2 KB), passes in order of SB; the pass at the bottom has constants.
+template <int LOG2L, int SB, int r>
+__host__ __device__ __forceinline__ float2 fft_tw(const float2* tw, int pos, int m) {
+    return tw[(pos + (m << SB)) << (LOG2L - SB - r - 1)];
+}
+struct FftPassTable {
+    const float2* tab;
+};
+constexpr int fft_pass_off(int sb) { return sb < 4 ? 0 : fft_pass_off(sb - 4) + (sb - 4 > 0 ? 8 << (sb - 4) : 0); }
+constexpr int fft_pass_row(int r) { return r < 2 ? r : r == 2 ? 2 : 4; }
+template <int LOG2L, int SB, int r>
+__host__ __device__ __forceinline__ float2 fft_tw(FftPassTable tw, int pos, int m) {
+    if constexpr (SB == 0) {
+        constexpr float C8 = 0.92387953251128673848f, S8 = 0.38268343236508978178f, C4 = 0.70710678118654752440f;
+        const int e = m << (3 - r);  // sixteenths of a turn
+        return e == 0 ? make_float2(1.f, 0.f) : e == 1 ? make_float2(C8, -S8) : e == 2 ? make_float2(C4, -C4)
+                                                                                  : make_float2(S8, -C8);
+    } else {
+        return tw.tab[fft_pass_off(SB) + ((fft_pass_row(r) + m) << SB) + pos];
+    }
+}
+
+// a w.  Each part is one rounded product and one FMA; which product is rounded first is free, and
+// written out so that a price does not depend on how a kernel was compiled: through the FP32 payoffs
+// a last bit anywhere moves it by 5e-9.
+enum FftMul {
+    FFT_MUL_X,  // imaginary part: a.y w.x first
+    FFT_MUL_Y,  // a.x w.y first
+    FFT_MUL_R,  // a.x w.y first, and a.x w.x in the real part, where the others take a.y w.y
+};
+template <FftMul F>
+__host__ __device__ __forceinline__ float2 fft_mul(float2 a, float2 w) {
+    const float re = F == FFT_MUL_R ? __builtin_fmaf(-a.y, w.y, a.x * w.x) : __builtin_fmaf(a.x, w.x, -(a.y * w.y));
+    const float im = F == FFT_MUL_X ? __builtin_fmaf(a.x, w.y, a.y * w.x) : __builtin_fmaf(a.y, w.x, a.x * w.y);
+    return make_float2(re, im);
+}
+
 // Stage SB + r of a group's points (distance 2^r in the group, 2^(SB + r) in the transform),
 // twiddle W = W_{2^(SB + r + 1)}^{pos + 2^SB m}, m = k mod 2^r, conjugated for the inverse (CONJ):
 // decimation in time maps (a, b) to (a + W b, a - W b), decimation in frequency to
 // (a + b, (a - b) W).  The upper half of a stage's twiddles is W_4 = -i (conjugate: +i) times the
-// lower half.
-template <int LOG2L, int SB, int R, int r, bool DIT, bool CONJ>
-__host__ __device__ __forceinline__ void fft_stage(float2 (&x)[1 << R], const float2* __restrict__ tw, int pos) {
-    constexpr int h = 1 << r, G = 1 << R, span = 1 << SB;
+// lower half.  The natural order's products take the form named below; `first`: the products of its
+// forward stages 2 (points 0 and 1) and 1 (point 0) take FFT_MUL_X.
+template <int LOG2L, int SB, int R, int r, bool DIT, bool CONJ, class TW>
+__host__ __device__ __forceinline__ void fft_stage(float2 (&x)[1 << R], TW tw, int pos, bool first) {
+    constexpr int h = 1 << r, G = 1 << R;
     constexpr int NL = h > 1 ? h / 2 : 1;  // twiddles read from the table
+    constexpr bool NAT = DIT == CONJ;
     float2 w[h];
     if constexpr (SB == 0 && r == 0) {
         w[0] = make_float2(1.f, 0.f);
     } else {
 #pragma unroll
         for (int m = 0; m < NL; ++m) {
-            const float2 c = tw[(pos + span * m) << (LOG2L - SB - r - 1)];
+            const float2 c = fft_tw<LOG2L, SB, r>(tw, pos, m);
             w[m] = CONJ ? make_float2(c.x, -c.y) : c;
         }
 #pragma unroll
@@ -249,6 +291,7 @@ __host__ __device__ __forceinline__ void fft_stage(float2 (&x)[1 << R], const fl
         // unit twiddles at the first two stages of a transform (pos = 0): no multiply
         const bool one = SB == 0 && m == 0 && r <= 1;
         const bool rot = SB == 0 && m == 1 && r == 1;
+        const bool upper = h > 1 && m >= NL;
         const float2 a = x[k], b = x[k + h];
         if constexpr (DIT) {
             float2 y;
@@ -256,8 +299,14 @@ __host__ __device__ __forceinline__ void fft_stage(float2 (&x)[1 << R], const fl
                 y = b;
             else if (rot)
                 y = CONJ ? make_float2(-b.y, b.x) : make_float2(b.y, -b.x);
-            else
+            else if (!NAT)
                 y = cmulf(w[m], b);
+            else if (!upper)
+                y = r == 1 ? fft_mul<FFT_MUL_R>(b, w[m]) : fft_mul<FFT_MUL_Y>(b, w[m]);
+            else if (r == 1 || (SB == 0 && r == 3 && m % 2 == 0))
+                y = fft_mul<FFT_MUL_Y>(b, w[m]);
+            else
+                y = fft_mul<FFT_MUL_X>(b, w[m]);
             x[k] = make_float2(a.x + y.x, a.y + y.y);
             x[k + h] = make_float2(a.x - y.x, a.y - y.y);
         } else {
@@ -267,26 +316,56 @@ __host__ __device__ __forceinline__ void fft_stage(float2 (&x)[1 << R], const fl
                 x[k + h] = d;
             else if (rot)
                 x[k + h] = CONJ ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
-            else
+            else if (!NAT)
                 x[k + h] = cmulf(d, w[m]);
+            else if (!upper && (r == 0 || r == 3))
+                x[k + h] = fft_mul<FFT_MUL_X>(d, w[m]);
+            else if (!upper && k < r && first)
+                x[k + h] = fft_mul<FFT_MUL_X>(d, w[m]);
+            else
+                x[k + h] = fft_mul<FFT_MUL_Y>(d, w[m]);
         }
     }
 }
 
 // stages SB .. SB + R - 1 of a group: decimation in time upwards, in frequency downwards
-template <int LOG2L, int SB, int R, bool CONJ>
-__host__ __device__ __forceinline__ void fft_stages_dit(float2 (&x)[1 << R], const float2* __restrict__ tw, int pos) {
-    fft_stage<LOG2L, SB, R, 0, true, CONJ>(x, tw, pos);
-    if constexpr (R > 1) fft_stage<LOG2L, SB, R, 1, true, CONJ>(x, tw, pos);
-    if constexpr (R > 2) fft_stage<LOG2L, SB, R, 2, true, CONJ>(x, tw, pos);
-    if constexpr (R > 3) fft_stage<LOG2L, SB, R, 3, true, CONJ>(x, tw, pos);
+template <int LOG2L, int SB, int R, bool CONJ, class TW>
+__host__ __device__ __forceinline__ void fft_stages_dit(float2 (&x)[1 << R], TW tw, int pos) {
+    fft_stage<LOG2L, SB, R, 0, true, CONJ>(x, tw, pos, false);
+    if constexpr (R > 1) fft_stage<LOG2L, SB, R, 1, true, CONJ>(x, tw, pos, false);
+    if constexpr (R > 2) fft_stage<LOG2L, SB, R, 2, true, CONJ>(x, tw, pos, false);
+    if constexpr (R > 3) fft_stage<LOG2L, SB, R, 3, true, CONJ>(x, tw, pos, false);
 }
-template <int LOG2L, int SB, int R, bool CONJ>
-__host__ __device__ __forceinline__ void fft_stages_dif(float2 (&x)[1 << R], const float2* __restrict__ tw, int pos) {
-    if constexpr (R > 3) fft_stage<LOG2L, SB, R, 3, false, CONJ>(x, tw, pos);
-    if constexpr (R > 2) fft_stage<LOG2L, SB, R, 2, false, CONJ>(x, tw, pos);
-    if constexpr (R > 1) fft_stage<LOG2L, SB, R, 1, false, CONJ>(x, tw, pos);
-    fft_stage<LOG2L, SB, R, 0, false, CONJ>(x, tw, pos);
+template <int LOG2L, int SB, int R, bool CONJ, class TW>
+__host__ __device__ __forceinline__ void fft_stages_dif(float2 (&x)[1 << R], TW tw, int pos, bool first) {
+    if constexpr (R > 3) fft_stage<LOG2L, SB, R, 3, false, CONJ>(x, tw, pos, first);
+    if constexpr (R > 2) fft_stage<LOG2L, SB, R, 2, false, CONJ>(x, tw, pos, first);
+    if constexpr (R > 1) fft_stage<LOG2L, SB, R, 1, false, CONJ>(x, tw, pos, first);
+    fft_stage<LOG2L, SB, R, 0, false, CONJ>(x, tw, pos, first);
+}
+// `first` of a group of the natural forward pass: the bottom pass; L = 2^13: the upper half's groups;
+// L = 2^14: every pass but the top one
+template <int LOG2L, int SB, int R>
+__host__ __device__ __forceinline__ bool fft_first(int t) {
+    return SB == 0 || (LOG2L == 13 && t >= ((1 << LOG2L) >> R) / 2) || (LOG2L == 14 && SB + R < LOG2L - 1);
+}
+
+// Spectrum in the bottom pass: element i of the bit-reversed order, plain, or point k of group t at
+// k 2^(LOG2L - R) + t (consecutive lanes read consecutive entries; plain, a lane reads a line of its own)
+template <int LOG2L, int R>
+__host__ __device__ __forceinline__ float2 fft_spec(const float2* G, int t, int k) {
+    return G[(t << R) + k];
+}
+struct FftSpectrum {
+    const float2* tab;
+};
+template <int LOG2L, int R>
+__host__ __device__ __forceinline__ float2 fft_spec(FftSpectrum G, int t, int k) {
+    return G.tab[(k << (LOG2L - R)) + t];
+}
+__host__ __device__ __forceinline__ int fft_spectrum_slot(int log2L, int i) {
+    const int R = (log2L - 1) % 4 == 0 ? 4 : (log2L - 1) % 4;
+    return ((i & ((1 << R) - 1)) << (log2L - R)) + (i >> R);
 }
 
 enum FftPassKind {
@@ -298,27 +377,34 @@ enum FftPassKind {
     FFT_MID_BR,   // forward DIT, product with G, inverse DIF (bit-reversed order)
 };
 
-// group t of a pass over stages SB .. SB + R - 1
-template <int LOG2L, int SB, int R, int KIND>
-__host__ __device__ __forceinline__ void fft_group(float2* z, const float2* __restrict__ tw,
-                                                   const float2* __restrict__ G, int t) {
+// group t of a pass over stages SB .. SB + R - 1; element i in slot i + (i >> PAD)
+template <int LOG2L, int SB, int R, int KIND, int PAD = 5, class TW, class GT>
+__host__ __device__ __forceinline__ void fft_group(float2* z, TW tw, GT G, int t) {
     constexpr int span = 1 << SB, NP = 1 << R;
     const int pos = t & (span - 1);
     const int i0 = ((t >> SB) << (SB + R)) + pos;
-    const int q = fpad(i0);
+    const int q = i0 + (i0 >> PAD);
     float2 x[NP];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) x[k] = z[q + k * span + ((k * span) >> 5)];
-    if constexpr (KIND == FFT_FWD_DIF || KIND == FFT_MID_NAT) fft_stages_dif<LOG2L, SB, R, false>(x, tw, pos);
+    for (int k = 0; k < NP; ++k) x[k] = z[q + k * span + ((k * span) >> PAD)];
+    if constexpr (KIND == FFT_FWD_DIF || KIND == FFT_MID_NAT)
+        fft_stages_dif<LOG2L, SB, R, false>(x, tw, pos, fft_first<LOG2L, SB, R>(t));
     if constexpr (KIND == FFT_FWD_DIT || KIND == FFT_MID_BR) fft_stages_dit<LOG2L, SB, R, false>(x, tw, pos);
-    if constexpr (KIND == FFT_MID_NAT || KIND == FFT_MID_BR) {
+    if constexpr (KIND == FFT_MID_NAT) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            const float2 g = fft_spec<LOG2L, R>(G, t, k);
+            x[k] = R > 2 && k == 0 ? fft_mul<FFT_MUL_X>(x[k], g) : fft_mul<FFT_MUL_Y>(x[k], g);
+        }
+    }
+    if constexpr (KIND == FFT_MID_BR) {
 #pragma unroll
         for (int k = 0; k < NP; ++k) x[k] = cmulf(x[k], G[i0 + k * span]);
     }
     if constexpr (KIND == FFT_INV_DIT || KIND == FFT_MID_NAT) fft_stages_dit<LOG2L, SB, R, true>(x, tw, pos);
-    if constexpr (KIND == FFT_INV_DIF || KIND == FFT_MID_BR) fft_stages_dif<LOG2L, SB, R, true>(x, tw, pos);
+    if constexpr (KIND == FFT_INV_DIF || KIND == FFT_MID_BR) fft_stages_dif<LOG2L, SB, R, true>(x, tw, pos, false);
 #pragma unroll
-    for (int k = 0; k < NP; ++k) z[q + k * span + ((k * span) >> 5)] = x[k];
+    for (int k = 0; k < NP; ++k) z[q + k * span + ((k * span) >> PAD)] = x[k];
 }
 
 // The runner of a pass: a workgroup of 256 threads takes every group of the pass, then meets at a
@@ -345,20 +431,19 @@ struct FftWorkgroup {
 template <int LOG2L>
 constexpr int fft_mid_stages() { return (LOG2L - 1) % 4 == 0 ? 4 : (LOG2L - 1) % 4; }
 
-template <int LOG2L, int S, class X>  // inverse passes from stage S up to LOG2L - 2
-__host__ __device__ __forceinline__ void fft_nat_inv(float2* z, const float2* __restrict__ tw, const X& x) {
+template <int LOG2L, int S, class TW, class X>  // inverse passes from stage S up to LOG2L - 2
+__host__ __device__ __forceinline__ void fft_nat_inv(float2* z, TW tw, const X& x) {
     if constexpr (S <= LOG2L - 2) {
-        x.template pass<LOG2L, S, 4, FFT_INV_DIT>(z, tw, nullptr);
+        x.template pass<LOG2L, S, 4, FFT_INV_DIT>(z, tw, static_cast<const float2*>(nullptr));
         fft_nat_inv<LOG2L, S + 4>(z, tw, x);
     }
 }
 
-template <int LOG2L, int S, class X>  // forward passes from stage S down to the middle pass
-__host__ __device__ __forceinline__ void fft_nat_fwd(float2* z, const float2* __restrict__ tw,
-                                                     const float2* __restrict__ G, const X& x) {
+template <int LOG2L, int S, class TW, class GT, class X>  // forward passes from stage S down to the middle pass
+__host__ __device__ __forceinline__ void fft_nat_fwd(float2* z, TW tw, GT G, const X& x) {
     constexpr int RM = fft_mid_stages<LOG2L>();
     if constexpr (S >= RM) {
-        x.template pass<LOG2L, S - 3, 4, FFT_FWD_DIF>(z, tw, nullptr);
+        x.template pass<LOG2L, S - 3, 4, FFT_FWD_DIF>(z, tw, static_cast<const float2*>(nullptr));
         fft_nat_fwd<LOG2L, S - 4>(z, tw, G, x);
     } else {
         static_assert(S == RM - 1, "passes of four stages down to the middle pass");
@@ -370,9 +455,8 @@ __host__ __device__ __forceinline__ void fft_nat_fwd(float2* z, const float2* __
 // Stages 0 .. LOG2L - 2 of the forward transform, the product with G (bit-reversed order) and
 // stages 0 .. LOG2L - 2 of the inverse; z holds the input after the forward top stage and is left
 // ready for the inverse top stage.  With FftWorkgroup: starts after and ends with a barrier.
-template <int LOG2L, class X>
-__host__ __device__ __forceinline__ void fft_convolve_r16(float2* z, const float2* __restrict__ tw,
-                                                          const float2* __restrict__ G, const X& x) {
+template <int LOG2L, class TW, class GT, class X>
+__host__ __device__ __forceinline__ void fft_convolve_r16(float2* z, TW tw, GT G, const X& x) {
     static_assert(LOG2L >= 10 && LOG2L <= 14, "transform lengths 2^10 .. 2^14");
     fft_nat_fwd<LOG2L, LOG2L - 2>(z, tw, G, x);
 }
@@ -381,7 +465,7 @@ __host__ __device__ __forceinline__ void fft_convolve_r16(float2* z, const float
 template <int LOG2L, int S, class X>  // inverse passes from stage S down to 0
 __host__ __device__ __forceinline__ void fft_br_inv(float2* z, const float2* __restrict__ tw, const X& x) {
     if constexpr (S >= 0) {
-        x.template pass<LOG2L, S - 3, 4, FFT_INV_DIF>(z, tw, nullptr);
+        x.template pass<LOG2L, S - 3, 4, FFT_INV_DIF>(z, tw, static_cast<const float2*>(nullptr));
         fft_br_inv<LOG2L, S - 4>(z, tw, x);
     }
 }
@@ -395,7 +479,7 @@ __host__ __device__ __forceinline__ void fft_br_fwd(float2* z, const float2* __r
         x.template pass<LOG2L, SB, R, FFT_MID_BR>(z, tw, G);
         fft_br_inv<LOG2L, SB - 1>(z, tw, x);
     } else {
-        x.template pass<LOG2L, SB, 4, FFT_FWD_DIT>(z, tw, nullptr);
+        x.template pass<LOG2L, SB, 4, FFT_FWD_DIT>(z, tw, static_cast<const float2*>(nullptr));
         fft_br_fwd<LOG2L, SB + 4>(z, tw, G, x);
     }
 }

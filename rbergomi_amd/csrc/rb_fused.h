@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "rb_device.h"
+#include "rb_types.h"
 
 namespace rb {
 
@@ -18,9 +19,8 @@ struct FusedUnit {
     float b;         // W1perp weight of the first-cell term
     float sc;        // sqrt(2H) N^-H
     int frag_off;    // offset of this unit's A-fragment table, in 16-byte entries
-    int p_off;       // offset of the unit's row tables, in floats.  Long-path kernel: one table
-                     // P_j = (j - off)^(2H), P_j at j.  GEMM kernel: per group of the unit (in
-                     // order, Np floats each) the row terms al P_j + be, at j - 1
+    int p_off;       // offset of the unit's row tables, in floats (GEMM kernel): per group of the
+                     // unit (in order, Np floats each) the row terms al P_j + be, at j - 1
     int g_begin, g_end;    // groups of this unit (contiguous)
     int pg_begin, pg_end;  // payoff groups (group, rho) of this unit (contiguous)
     int o_begin, o_end;    // options of this unit (contiguous)
@@ -237,32 +237,32 @@ inline int fused_greg(int gmax) {
 hipError_t launch_zero_int(int* p, int n, hipStream_t st);
 
 // ---------------------------------------------------------------- long paths (N > 1024)
-// One request priced by the single-launch FFT kernel (rb_fused_fft.hip).
+// One request on the FFT kernel (rb_fused_fft.hip): paths [p0, p0 + np) to their integrals.
 struct FftFusedArgs {
-    int N, log2L, nunits, out_size;
-    int mc;                      // 1 = plain Monte Carlo, 0 = Romano-Touzi
-    int pgu;                     // most payoff groups of one unit (LDS records per path)
-    int pairs_per_item;          // path pairs of one work item
-    long M, npairs, nitems;
     PhiloxKey key;
-    const FusedUnit* units;      // b, sc, p_off and the group / payoff-group / option ranges
+    long p0, np;
+    int N, nunits, nsplit;
+    int mc;                      // 1 = plain Monte Carlo, 0 = Romano-Touzi
+    const FusedUnit* units;      // b, sc and the group range
     const FusedGroup* groups;
-    const FusedPG* pgs;
-    const FusedOption* opts;
-    const float* ptab;           // per unit: P_j = (j - off)^(2H)
-    const float2* ghat;          // per unit [L]: FFT of (a, Gamma_1, ..., Gamma_{N-1}, 0, ...),
-                                 // bit-reversed order
-    const float2* tw;            // [L/2]: exp(-2 pi i k / L)
-    double* partial;             // [out_size][nitems][2]
-    int* counter;                // next work item (zeroed before the launch)
+    const float* ptab;           // per unit [L/2]: P_i = (i - off)^(2H), +inf at 0 and from N on
+    const float2* ghat;          // per unit [L]: spectrum of (a, Gamma_1, ..., Gamma_{N-1}), in the
+                                 // order of FftSpectrum
+    const float2* tw;            // [fused_fft_table]: exp(-2 pi i k / L), then the passes' tables
+    double* ints;                // [groups][np][2, plain MC 3]: Iv, Is, Ip
 };
-size_t fused_fft_lds_bytes(const FftFusedArgs& a);
-// quads per thread of the kernel instantiation that runs N: ceil(ceil(N/4) / 256) rounded up to
-// 1, 2, 4 or 8; its threads visit steps 0 .. 1024 QPT - 1
-inline int fused_fft_qpt(int N) {
-    const int q = ((N + 3) / 4 + 255) / 256;
-    return q <= 1 ? 1 : q <= 2 ? 2 : q <= 4 ? 4 : 8;
+int fused_fft_log2(int N);       // transform length 2^log2 >= 2N, at least 2^10
+// twiddles: L/2, and 8 2^sb for the passes at sb = log2L - 5, log2L - 9, ... > 0
+inline __host__ __device__ int fused_fft_table(int log2L) {
+    int n = 1 << (log2L - 1);
+    for (int sb = log2L - 5; sb > 0; sb -= 4) n += 8 << sb;
+    return n;
 }
-hipError_t launch_fused_fft(const FftFusedArgs& a, int grid, hipStream_t st);
+// tables on the device (off: 1 for the reference compensator, 0 for the exact one); gamma and tw64 are
+// scratch, L/2 doubles per unit and path64_fft_table(L/2) entries, or null where ghat comes from the host
+// (N > 4096)
+hipError_t launch_fused_fft_tables(const Unit* units, int nunits, int N, double off, double* gamma, double2* tw64,
+                                   float* ptab, float2* tw, float2* ghat, hipStream_t st);
+hipError_t launch_fused_fft(FftFusedArgs a, int cus, hipStream_t st);
 
 }  // namespace rb

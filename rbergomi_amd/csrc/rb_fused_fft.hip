@@ -1,342 +1,379 @@
-// rb_fused_fft.hip -- single-launch mixed-precision Romano-Touzi pricing by FFT convolution: for
-// long paths (N > 1024, where the Toeplitz GEMM's W1 tile no longer fits LDS), and for any
-// N <= 8192 at the FFT precision (the same kernel with one quad per thread below N = 1024).
+// rb_fused_fft.hip -- mixed-precision pricing by FFT convolution in one pass over the paths: for long
+// paths (N > 1024, where the Toeplitz GEMM's W1 tile no longer fits LDS), and for any N <= 8192 at the
+// FFT precision.
 //
-// A persistent workgroup takes work items (pairs_per_item pairs of paths) from an atomic
-// counter and runs the whole path of the reference for each pair without touching HBM:
-//   1. Philox4x32-10 W1 of both paths (FP32 Box-Muller, stream 0), kept in registers: thread t
-//      owns the 4-step quads q = t + 256 j of both paths (genGaussianMT,
-//      rBergLib/rBergomiMT.cpp:169-172).
-//   2. Per unit (H): z = W1_a + i W1_b zero-padded to L = 2^k >= 2N - 1 in LDS, radix-16 FFT
-//      (decimation in frequency), times FFT(a, Gamma_1, ..., Gamma_{N-1}) (the first-cell weight
-//      a folded in; bit-reversed order), inverse FFT (decimation in time): Gamma is real, so the
+// TP threads own a pair of paths, half of them each path: TP = L / 16 (512 at L = 2^14), L = 2^LOG2L >= 2 N:
+//   1. W1 of the thread's quads of steps of its path, Philox and FP32 Box-Muller (genGaussianMT,
+//      rBergLib/rBergomiMT.cpp:169-172), kept in registers.
+//   2. Per unit (distinct H): z = W1_a + i W1_b through the LDS transforms (rb_fft_lds.h, natural order),
+//      with the product by the spectrum of (a, Gamma_1, ..., Gamma_{N-1}) between them: Gamma is real, so the
 //      real and imaginary parts are the two paths' convolutions (updateWtilde's FFTW convolution,
-//      :83-109).  The transforms' top stages are done while z is written and read back.
-//   3. Wtilde = sc (Y + b W1perp) for the thread's steps, W1perp regenerated from the same
-//      counters (stream 1), written back to LDS in step order; then per (H, eta, T) group
-//      sqrt(v_i) = exp2(c1 Wtilde_{i-1} - al P_i - be) and the sums of v and sqrt(v) W1 over
-//      the thread's steps in FP32, over the workgroup in FP64 (scaleWtilde/updateV/intVdt/
-//      intRootVdW, :73-80, 163-167, 427-436).
-//   4. Per (path, group, rho) ln S', sigma; per option the conditioned Black-Scholes payoff in
-//      FP32 with the FP64 tail (payoff_mixed), summed in FP64 per option over the item's paths.
-// Plain Monte Carlo (computeIV_tensor's estimator, MC = true): a third sum sqrt(v) Wperp with
-// Wperp from stream 2, ln S_T = rho Is + sqrt(1 - rho^2) Ip - Iv / 2 and the payoff (S_T - K)^+
-// in FP64 (updateZ/updateS, rBergLib/rBergomiMT.cpp:111-137).
-// Outputs the same per-item option sums as the GEMM kernel, reduced by k_reduce_iv.
+//      :83-109).  Wtilde = sc (Y + b W1perp) for the thread's steps.
+//   3. Per (H, eta, T) group sqrt(v_i) = exp2(c1 Wtilde_{i-1} - al P_i - be) and the sums of v and
+//      sqrt(v) W1 in FP32 over up to eight quads of steps, then in FP64 (scaleWtilde/updateV/intVdt/
+//      intRootVdW, :73-80, 163-167, 427-436); plain MC adds sqrt(v) Wperp.  P = +inf at i = 0 and i >= N
+//      makes those terms exactly 0.
+//   4. ints[group][path]: the integrals (Iv, Is[, Ip]) in FP64, priced by the payoff kernel of
+//      rb_payoff64.hip in chunks of paths.
+//
+// What bounds it: vector issue (per thread of 16 steps and unit about 900 instructions of Gaussians, 1500 of
+// butterflies, 100 of each group: 0.55 ms of N = 4096's 0.76 below).  Sixteen points per thread keep
+// four waves per SIMD in registers (no spills to N = 2048, 19 beyond) and LDS (9 KB a wave); at N > 4096,
+// where one workgroup fills the LDS, two waves of thirty-two points each.  The form before it, one
+// pair per 256 threads with the payoffs of both paths priced between barriers by one thread per option
+// and the tables formed on the host, took, one maturity, N = 4096, M = 32768, 1.02 ms (now 0.76), N =
+// 2048, M = 65536 1.02 (0.53), plain MC 1.56 and 1.09 (0.82 and 0.57), N = 512, M = 200000 1.61 (0.39), and
+// its tables 1.3 ms of each request at N = 4096.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "rb_fft_lds.h"
 #include "rb_fused.h"
 #include "rb_kernels.h"
+#include "rb_lanes.h"
 
 namespace rb {
 
-constexpr int FFT_GR = 8;  // groups integrated per pass
-
-__device__ __forceinline__ double wave_sum64(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-constexpr int FFT_NS = 3;  // sums per (path, group) held in the reduction buffer
-
-size_t fused_fft_lds_bytes(const FftFusedArgs& a) {
-    return fft_lds_slots(a.log2L) * sizeof(float2) + size_t(4) * FFT_GR * 2 * FFT_NS * sizeof(double) +
-           size_t(2) * a.pgu * sizeof(PathPG) + size_t(a.out_size) * 2 * sizeof(double);
-}
-
-// QPT: quads per thread and path, ceil(ceil(N/4) / 256); LOG2L: the transform length,
-// L = 2^LOG2L >= 2N - 1 and at least 2^10 (LOG2L = 11 + log2 QPT for 1024 < N <= 8192; 10 or 11
-// for QPT = 1).
-template <int QPT, bool MC, int LOG2L>
-__global__ void __launch_bounds__(256, (QPT >= 8 || (MC && QPT >= 4)) ? 1 : 2) k_fused_fft(FftFusedArgs A) {
-    extern __shared__ float2 lds2[];
-    const int L = 1 << A.log2L, H2 = L >> 1;
-    float2* z = lds2;                                                      // [L + L/32], slot fpad(i)
-    double* red = reinterpret_cast<double*>(z + L + (L >> 5));             // [4][FFT_GR][2][FFT_NS]
-    PathPG* pgd = reinterpret_cast<PathPG*>(red + 4 * FFT_GR * 2 * FFT_NS);  // [2][pgu]
-    double* acc = reinterpret_cast<double*>(pgd + 2 * A.pgu);              // [out][2]
-    __shared__ int s_item;
-    __shared__ float s_w10[2], s_w20[2];  // W1, Wperp of both paths at step 0
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int N = A.N, nq = (N + 3) >> 2;
-    for (;;) {
-        if (tid == 0) s_item = atomicAdd(A.counter, 1);
-        __syncthreads();
-        const long item = s_item;
-        __syncthreads();
-        if (item >= A.nitems) break;
-        for (int o = tid; o < 2 * A.out_size; o += 256) acc[o] = 0.0;
-        const long pr0 = item * A.pairs_per_item;
-        const long pr1 = pr0 + A.pairs_per_item < A.npairs ? pr0 + A.pairs_per_item : A.npairs;
-        for (long pr = pr0; pr < pr1; ++pr) {
-            const long pth[2] = {2 * pr, 2 * pr + 1};
-            // ---- 1. W1 of both paths for this thread's quads (zero past N and past M)
-            float w1[2][QPT][4];
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-#pragma unroll
-                for (int j = 0; j < QPT; ++j) {
-                    const int q = tid + 256 * j;
-                    float zz[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (q < nq && pth[c] < A.M) normals4_f32(A.key, uint64_t(pth[c]), 0u, uint32_t(q), zz);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) w1[c][j][t] = 4 * q + t < N ? zz[t] : 0.f;
-                }
-            if (tid == 0) {
-                s_w10[0] = w1[0][0][0];
-                s_w10[1] = w1[1][0][0];
-                if constexpr (MC) {
-                    for (int c = 0; c < 2; ++c) {
-                        float zz[4] = {0.f, 0.f, 0.f, 0.f};
-                        if (pth[c] < A.M) normals4_f32(A.key, uint64_t(pth[c]), 2u, 0u, zz);
-                        s_w20[c] = zz[0];
-                    }
-                }
-            }
-            for (int u = 0; u < A.nunits; ++u) {
-                const FusedUnit U = A.units[u];
-                // ---- 2. z in natural order through the forward transform's top stage (its upper
-                //         half is the zero padding: z_i = x_i, z_{i + L/2} = x_i W_L^i), the
-                //         remaining stages, product, inverse transform but its top stage
-#pragma unroll
-                for (int j = 0; j < QPT; ++j) {
-                    const int q = tid + 256 * j;
-                    if (q < nq)
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            const int i = 4 * q + t;  // 4 nq <= L/2
-                            const float2 x = make_float2(w1[0][j][t], w1[1][j][t]);
-                            z[fpad(i)] = x;
-                            z[fpad(i + H2)] = cmulf(x, A.tw[i]);
-                        }
-                }
-                for (int i = 4 * nq + tid; i < H2; i += 256) {
-                    z[fpad(i)] = make_float2(0.f, 0.f);
-                    z[fpad(i + H2)] = make_float2(0.f, 0.f);
-                }
-                __syncthreads();
-                fft_convolve_r16<LOG2L>(z, A.tw, A.ghat + long(u) * L, FftWorkgroup{tid});
-                // ---- 3. Wtilde of the thread's steps (both paths), then back to LDS in step order
-                const float invL = 1.0f / float(L);
-                float wt[2][QPT][4];
-#pragma unroll
-                for (int j = 0; j < QPT; ++j) {
-                    const int q = tid + 256 * j;
-                    float zp[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-                    for (int c = 0; c < 2; ++c)
-                        if (q < nq && pth[c] < A.M) normals4_f32(A.key, uint64_t(pth[c]), 1u, uint32_t(q), zp[c]);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int i = 4 * q + t;
-                        float2 y = make_float2(0.f, 0.f);
-                        if (i < N) {  // the inverse top stage: z_i + conj(W_L^i) z_{i + L/2}
-                            const float2 lo = z[fpad(i)], hi = z[fpad(i + H2)], w = A.tw[i];
-                            const float2 p = cmulf(make_float2(w.x, -w.y), hi);
-                            y = make_float2(lo.x + p.x, lo.y + p.y);
-                        }
-                        wt[0][j][t] = U.sc * fmaf(y.x, invL, U.b * zp[0][t]);
-                        wt[1][j][t] = U.sc * fmaf(y.y, invL, U.b * zp[1][t]);
-                    }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int j = 0; j < QPT; ++j) {
-                    const int q = tid + 256 * j;
-                    if (q < nq)
-#pragma unroll
-                        for (int t = 0; t < 4; ++t)
-                            if (4 * q + t < N) z[fpad(4 * q + t)] = make_float2(wt[0][j][t], wt[1][j][t]);
-                }
-                __syncthreads();
-                // ---- 4. integrals of the unit's groups, FFT_GR groups per pass
-                const float* P = A.ptab + U.p_off;
-                for (int g0 = U.g_begin; g0 < U.g_end; g0 += FFT_GR) {
-                    const int gn = U.g_end - g0 < FFT_GR ? U.g_end - g0 : FFT_GR;
-                    float c1[FFT_GR], al[FFT_GR], be[FFT_GR];
-                    float fv[FFT_GR][2], fs[FFT_GR][2], fp[FFT_GR][2];
-#pragma unroll
-                    for (int gg = 0; gg < FFT_GR; ++gg) {
-                        c1[gg] = al[gg] = be[gg] = 0.f;
-                        fv[gg][0] = fv[gg][1] = fs[gg][0] = fs[gg][1] = fp[gg][0] = fp[gg][1] = 0.f;
-                        if (gg < gn) {
-                            c1[gg] = A.groups[g0 + gg].c1;
-                            al[gg] = A.groups[g0 + gg].al;
-                            be[gg] = A.groups[g0 + gg].be;
-                        }
-                    }
-                    if constexpr (MC) {
-                        // plain MC: steps outside, groups inside, since the Wperp Gaussians come
-                        // per quad (held across a group loop they raised the two-quad kernel's
-                        // spills from 0 to 27 VGPRs)
-#pragma unroll
-                        for (int j = 0; j < QPT; ++j) {
-                            const int q = tid + 256 * j;
-                            float wp[2][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-                            for (int c = 0; c < 2; ++c)
-                                if (q < nq && pth[c] < A.M) normals4_f32(A.key, uint64_t(pth[c]), 2u, uint32_t(q), wp[c]);
-#pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                const int i = 4 * q + t;  // v_i uses Wtilde_{i-1}; i = 0 is v_0 = xi
-                                if (i >= 1 && i < N) {
-                                    const float2 x = z[fpad(i - 1)];
-                                    const float pj = P[i];
-#pragma unroll
-                                    for (int gg = 0; gg < FFT_GR; ++gg) {
-                                        if (gg < gn) {
-                                            const float e = fmaf(al[gg], pj, be[gg]);
-                                            const float ra = __builtin_amdgcn_exp2f(fmaf(x.x, c1[gg], -e));
-                                            const float rb = __builtin_amdgcn_exp2f(fmaf(x.y, c1[gg], -e));
-                                            fv[gg][0] = fmaf(ra, ra, fv[gg][0]);
-                                            fs[gg][0] = fmaf(ra, w1[0][j][t], fs[gg][0]);
-                                            fv[gg][1] = fmaf(rb, rb, fv[gg][1]);
-                                            fs[gg][1] = fmaf(rb, w1[1][j][t], fs[gg][1]);
-                                            fp[gg][0] = fmaf(ra, wp[0][t], fp[gg][0]);
-                                            fp[gg][1] = fmaf(rb, wp[1][t], fp[gg][1]);
-                                        }
-                                    }
-                                }
-                            }
-                        }
-                    } else {
-                        // Romano-Touzi: groups outside (one uniform branch per group), steps inside
-                        // with no test:
-                        // P = +inf at i = 0 and at i >= N (al > 0) makes those terms exactly 0, and
-                        // i - 1 is clamped to a written slot.  Each group's sums still run over the
-                        // steps in the same order.
-#pragma unroll
-                        for (int gg = 0; gg < FFT_GR; ++gg) {
-                            if (gg < gn) {
-#pragma unroll
-                                for (int j = 0; j < QPT; ++j) {
-                                    const int q = tid + 256 * j;
-#pragma unroll
-                                    for (int t = 0; t < 4; ++t) {
-                                        const int i = 4 * q + t;  // v_i uses Wtilde_{i-1}; i = 0 is v_0 = xi
-                                        const float2 x = z[fpad(i > 0 ? i - 1 : 0)];
-                                        const float e = fmaf(al[gg], P[i], be[gg]);
-                                        const float ra = __builtin_amdgcn_exp2f(fmaf(x.x, c1[gg], -e));
-                                        const float rb = __builtin_amdgcn_exp2f(fmaf(x.y, c1[gg], -e));
-                                        fv[gg][0] = fmaf(ra, ra, fv[gg][0]);
-                                        fs[gg][0] = fmaf(ra, w1[0][j][t], fs[gg][0]);
-                                        fv[gg][1] = fmaf(rb, rb, fv[gg][1]);
-                                        fs[gg][1] = fmaf(rb, w1[1][j][t], fs[gg][1]);
-                                    }
-                                }
-                            }
-                        }
-                    }
-                    // FP64 over the workgroup: wave sums, then the four waves in order
-#pragma unroll
-                    for (int gg = 0; gg < FFT_GR; ++gg) {
-                        if (gg < gn) {
-#pragma unroll
-                            for (int c = 0; c < 2; ++c) {
-                                const double sv = wave_sum64(double(fv[gg][c]));
-                                const double ss = wave_sum64(double(fs[gg][c]));
-                                double sp = 0.0;
-                                if constexpr (MC) sp = wave_sum64(double(fp[gg][c]));
-                                if (lane == 0) {
-                                    red[((wave * FFT_GR + gg) * 2 + c) * FFT_NS + 0] = sv;
-                                    red[((wave * FFT_GR + gg) * 2 + c) * FFT_NS + 1] = ss;
-                                    red[((wave * FFT_GR + gg) * 2 + c) * FFT_NS + 2] = sp;
-                                }
-                            }
-                        }
-                    }
-                    __syncthreads();
-                    if (tid < 2 * gn) {
+// ---------------------------------------------------------------- tables
+// k^h to the nearest double, through a logarithm and an exponential of twice its length: the error of
+// a library power, 1e-12 in the spectrum of its differences, turns a rounding of the FP32 spectrum in one
+// request of two and moves its prices by 5e-10.
+struct Dd {
+    double hi, lo;
+};
+__device__ inline Dd dd_norm(double a, double b) {  // |a| >= |b|
 #pragma clang fp contract(off)
-                        const int gg = tid >> 1, c = tid & 1;
-                        const FusedGroup Gr = A.groups[g0 + gg];
-                        double a = Gr.xi, b = Gr.sxi * double(s_w10[c]);  // step 0: v_0 = xi
-                        double cp = MC ? Gr.sxi * double(s_w20[c]) : 0.0;
-                        for (int w = 0; w < 4; ++w) {
-                            a += red[((w * FFT_GR + gg) * 2 + c) * FFT_NS + 0];
-                            b += red[((w * FFT_GR + gg) * 2 + c) * FFT_NS + 1];
-                            if constexpr (MC) cp += red[((w * FFT_GR + gg) * 2 + c) * FFT_NS + 2];
-                        }
-                        const double Iv = Gr.dt * a, Is = Gr.sdt * b;
-                        if constexpr (MC) {
-                            // ln S_T = rho Is + sqrt(1 - rho^2) Ip - Iv / 2 (log-Euler, left point)
-                            const double Ip = Gr.sdt * cp;
-                            for (int pg = Gr.pg_begin; pg < Gr.pg_end; ++pg) {
-                                const double rho = A.pgs[pg].rho;
-                                PathPG rec;
-                                rec.lnS = rho * Is + sqrt(1.0 - rho * rho) * Ip - 0.5 * Iv;
-                                rec.sig = exp(rec.lnS);
-                                rec.S = float(rec.sig);
-                                rec.ik = rec.A = rec.sg = 0.f;
-                                pgd[c * A.pgu + (pg - U.pg_begin)] = rec;
-                            }
-                        }
-                        for (int pg = Gr.pg_begin; !MC && pg < Gr.pg_end; ++pg) {
-                            const double rho = A.pgs[pg].rho;
-                            PathPG rec;
-                            rec.sig = sqrt((1.0 - rho * rho) * Iv);
-                            rec.lnS = -0.5 * rho * rho * Iv + rho * Is;
-                            pathpg_f32(rec);
-                            pgd[c * A.pgu + (pg - U.pg_begin)] = rec;
-                        }
-                    }
-                    __syncthreads();
+    const double s = a + b;
+    return Dd{s, b - (s - a)};
+}
+__device__ inline Dd dd_mul(Dd a, Dd b) {
+#pragma clang fp contract(off)
+    const double p = a.hi * b.hi;
+    return dd_norm(p, fma(a.hi, b.hi, -p) + fma(a.hi, b.lo, a.lo * b.hi));
+}
+__device__ inline Dd dd_exp(Dd x) {  // 2^n (Taylor series of the rest over 64)^64
+#pragma clang fp contract(off)
+    constexpr double LN2_HI = 0.693147180559945286, LN2_LO = 2.31904681384629956e-17;
+    const double n = rint(x.hi / LN2_HI), p = n * LN2_HI;
+    const Dd d = dd_norm(x.hi - p, (x.lo - fma(n, LN2_HI, -p)) - n * LN2_LO);
+    const Dd r{d.hi * 0x1p-6, d.lo * 0x1p-6};
+    Dd e{1.0, 0.0};
+    for (int k = 9; k >= 1; --k) {  // 1 + r e / k
+        e = dd_mul(r, e);
+        const double q = e.hi / k;
+        e = dd_norm(q, (fma(-q, double(k), e.hi) + e.lo) / k);
+        const double s = 1.0 + e.hi;
+        e = dd_norm(s, (e.hi - (s - 1.0)) + e.lo);
+    }
+    for (int k = 0; k < 6; ++k) e = dd_mul(e, e);
+    return Dd{ldexp(e.hi, int(n)), ldexp(e.lo, int(n))};
+}
+__device__ inline double pow_nearest(double k, double h) {
+#pragma clang fp contract(off)
+    const double l = log(k);
+    const Dd e = dd_exp(Dd{-l, 0.0});
+    const Dd t = dd_mul(dd_norm(l, fma(k, e.hi, -1.0) + k * e.lo), Dd{h, 0.0});
+    return dd_exp(t).hi;
+}
+
+// gamma[u][i]: a, Gamma_1 .. Gamma_{N-1}; ptab[u][i] = P_i, +inf at 0 and from N on
+__global__ void k_fft32_tables(const Unit* __restrict__ units, int N, int tlen, double off, double* __restrict__ gamma,
+                               float* __restrict__ ptab) {
+#pragma clang fp contract(off)
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= tlen) return;
+    const Unit un = units[blockIdx.y];
+    const double h = un.H - 0.5 + 1.0;
+    double g = 0.0;
+    if (i == 0) g = un.a;
+    else if (i < N && gamma) g = (pow_nearest(i + 1.0, h) - pow_nearest(double(i), h)) / h;
+    if (gamma) gamma[long(blockIdx.y) * tlen + i] = g;
+    ptab[long(blockIdx.y) * tlen + i] = i >= 1 && i < N ? float(pow(double(i) - off, 2.0 * un.H)) : INFINITY;
+}
+
+// Twiddles: exp(-2 pi i k / L) for k < L/2, then the passes' tables (FftPassTable)
+__global__ void k_fft32_twiddles(int log2L, float2* __restrict__ tw) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, H2 = 1 << (log2L - 1);
+    if (i >= fused_fft_table(log2L)) return;
+    int k = i;
+    if (i >= H2) {
+        int sb = (log2L - 1) % 4 ? (log2L - 1) % 4 : 4, o = i - H2;
+        for (; o >= 8 << sb; sb += 4) o -= 8 << sb;
+        const int row = o >> sb, r = row < 2 ? row : row < 4 ? 2 : 3;
+        k = ((o & ((1 << sb) - 1)) + ((row - fft_pass_row(r)) << sb)) << (log2L - sb - r - 1);
+    }
+    double s, c;
+    sincospi(-double(k) / double(H2), &s, &c);
+    tw[i] = make_float2(float(c), float(s));
+}
+
+// ---------------------------------------------------------------- the path kernel
+template <int LOG2L>
+struct FftPair {
+    static constexpr int L = 1 << LOG2L;
+    static constexpr int TP = LOG2L <= 13 ? L / 16 : 512, HP = TP / 2;  // threads of a pair, of a path
+    static constexpr int NT = TP < 256 ? 256 : TP, PAIRS = NT / TP;
+    static constexpr int W = HP < 64 ? HP : 64, NW = HP / W;  // lanes and waves of a path
+    static constexpr int QT = L / 8 / HP;                     // quads of steps per thread
+    // A path's sums run in FP32 over the quads q, q + 256, ... (CQ of them), then in FP64
+    static constexpr int CQ = LOG2L <= 11 ? 1 : 1 << (LOG2L - 11);
+    // element i in slot i + i / 16: the accesses of every pass spread over the banks (i / 32, half of them
+    // two lanes to a bank)
+    static constexpr int PAD = 4, SLOTS = L + (L >> PAD);
+    __device__ static __forceinline__ int slot(int i) { return i + (i >> PAD); }
+    __device__ static __forceinline__ int quad(int s, int j) { return s + HP * (j / CQ) + 256 * (j % CQ); }
+    // waves per SIMD the registers are cut for
+    static constexpr int WAVES = LOG2L <= 13 ? 4 : 2;
+};
+
+// A pass of the transform by the TP threads of a pair (the schedules of rb_fft_lds.h)
+template <int TP, class Sync>
+struct FftPairPass {
+    int t;
+    Sync sync;
+    template <int LOG2L, int SB, int R, int KIND, class GT>
+    __device__ __forceinline__ void pass(float2* z, FftPassTable tw, GT G) const {
+        constexpr int NG = (1 << LOG2L) >> R;
+        static_assert(NG % TP == 0, "whole groups per thread");
+#pragma unroll 2
+        for (int u = 0; u < NG / TP; ++u) fft_group<LOG2L, SB, R, KIND, FftPair<LOG2L>::PAD>(z, tw, G, t + TP * u);
+        sync();
+    }
+};
+
+// The first pass of the forward transform: the top stage of a signal whose upper half is zero
+// (z_{i + L/2} = z_i W_L^i) and the four stages under it.
+template <int LOG2L, int TP, class Sync>
+__device__ __forceinline__ void fft_first_pass(float2* z, const float2* tw, int t, const Sync& sync) {
+    constexpr int SB = LOG2L - 5, span = 1 << SB, H2 = 1 << (LOG2L - 1), PAD = FftPair<LOG2L>::PAD;
+    const FftPassTable tab{tw + H2};
+    const int pos = t & (span - 1);
+    float2* p = z + FftPair<LOG2L>::slot(pos);
+    float2 x[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = p[k * span + ((k * span) >> PAD)];
+    auto upper = [&] {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = fft_mul<FFT_MUL_Y>(x[k], tw[pos + k * span]);
+    };
+    auto run = [&](int h) {
+        fft_stages_dif<LOG2L, SB, 4, false>(x, tab, pos, fft_first<LOG2L, SB, 4>(pos + h * span));
+        float2* o = p + h * (H2 + (H2 >> PAD));
+#pragma unroll
+        for (int k = 0; k < 16; ++k) o[k * span + ((k * span) >> PAD)] = x[k];
+    };
+    if constexpr (TP == 2 * span) {  // half of the threads to each half of the points
+        sync();                      // the lower half has been read
+        if (t >= span) upper();
+        run(t >= span ? 1 : 0);
+    } else {
+        static_assert(TP == span, "both halves of a group to a thread");
+        float2 y[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) y[k] = x[k];
+        run(0);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = y[k];
+        upper();
+        run(1);
+    }
+    sync();
+}
+
+// Grid (ceil(pairs / PAIRS), nsplit), block NT, dynamic LDS fused_fft_lds.
+template <int LOG2L, bool MC>
+__global__ void __launch_bounds__((FftPair<LOG2L>::NT), (FftPair<LOG2L>::WAVES)) k_fused_fft(FftFusedArgs A) {
+    using C = FftPair<LOG2L>;
+    using Sync = std::conditional_t<C::TP <= 64, WaveSync, BlockSync>;
+    constexpr int TP = C::TP, HP = C::HP, QT = C::QT, CQ = C::CQ, L = C::L, H2 = L / 2;
+    constexpr int NV = MC ? 3 : 2, V = MC ? 4 : 2;  // sums per path; values summed over the lanes
+    extern __shared__ double2 lds[];
+    double* red = reinterpret_cast<double*>(lds);  // [PAIRS][2][NW][V]
+    const int tid = threadIdx.x, lane = tid & 63, pair = tid / TP, t0 = tid % TP;
+    const int c = t0 / HP, s0 = t0 % HP;  // the thread's path of the pair
+    float2* z = reinterpret_cast<float2*>(red + C::PAIRS * 2 * C::NW * V) + pair * (C::SLOTS + L / 8);
+    float* last = reinterpret_cast<float*>(z + C::SLOTS) + c * (L / 8);  // [quads]: Wtilde of a quad's last step
+    red += (pair * 2 + c) * C::NW * V;
+    const Sync sync{};
+    const int N = A.N, nq = (N + 3) >> 2;
+    const long pr = long(blockIdx.x) * C::PAIRS + pair, p = 2 * pr + c;
+    // ---- 1. Gaussians of the thread's quads
+    auto gaussians = [&](uint32_t stream, int s, float(&w)[QT][4]) {
+#pragma unroll
+        for (int j = 0; j < QT; ++j) {
+            const int q = C::quad(s, j);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[j][r] = 0.f;
+            if (q < nq) normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(q), w[j]);
+        }
+    };
+    float w1[QT][4];
+    gaussians(0, s0, w1);
+#pragma unroll
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * C::quad(s0, j) + r >= N) w1[j][r] = 0.f;
+
+    const int u0 = int(long(A.nunits) * blockIdx.y / A.nsplit), u1 = int(long(A.nunits) * (blockIdx.y + 1) / A.nsplit);
+    for (int u = u0; u < u1; ++u) {
+        const FusedUnit U = A.units[u];
+        // the thread's place and the tables' address are hidden from the loop over the units: hoisted out
+        // of it, every pass's addresses and twiddles would stay in registers (60 to 100 spilled)
+        int t = t0, s = s0, hide = 0;
+        asm volatile("" : "+v"(t), "+v"(s), "+s"(hide));
+        const float2* tw = A.tw + hide;
+        // ---- 2. Wtilde of the thread's steps
+        if (u > u0) sync();  // the last unit's reads are done
+#pragma unroll
+        for (int j = 0; j < QT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) reinterpret_cast<float*>(z + C::slot(4 * C::quad(s, j) + r))[c] = w1[j][r];
+        sync();
+        fft_first_pass<LOG2L, TP>(z, tw, t, sync);
+        fft_nat_fwd<LOG2L, LOG2L - 6>(z, FftPassTable{tw + H2}, FftSpectrum{A.ghat + long(u) * L},
+                                        FftPairPass<TP, Sync>{t, sync});
+        asm volatile("" : "+v"(s));  // its slots are formed again after the transforms (24 fewer spilled)
+        // W1perp is drawn here, once per unit: held across the transforms, its registers would not leave
+        // four waves per SIMD
+        float x[QT][4];
+        gaussians(1, s, x);
+        constexpr float invL = 1.0f / float(L);
+        auto wtilde = [&](auto comp) {
+#pragma unroll
+            for (int j = 0; j < QT; ++j) {
+                const int i0 = 4 * C::quad(s, j);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {  // the inverse top stage: z_i + conj(W_L^i) z_{i + L/2}
+                    const float2 lo = z[C::slot(i0 + r)], hi = z[C::slot(i0 + r + H2)], w = tw[i0 + r];
+                    const float2 m = fft_mul<FFT_MUL_Y>(hi, make_float2(w.x, -w.y));
+                    const float y = decltype(comp)::value ? lo.y + m.y : lo.x + m.x;
+                    x[j][r] = U.sc * fmaf(y, invL, U.b * x[j][r]);
                 }
-                // ---- 5. payoffs of the unit's options for both paths (one thread per option)
-                for (int o = U.o_begin + tid; o < U.o_end; o += 256) {
-                    const FusedOption O = A.opts[o];
-                    const OptF of = opt_f32(O.lnK, O.K);
-                    double s1 = 0.0, s2 = 0.0;
-                    for (int c = 0; c < 2; ++c) {
-                        if (pth[c] >= A.M) continue;
-                        const PathPG& rec = pgd[c * A.pgu + (O.pg - U.pg_begin)];
-                        const double x = MC ? payoff_mc(rec, O.K) : payoff_mixed<true>(rec, of, O.lnK, O.K);
-                        s1 += x;
-                        s2 += x * x;
-                    }
-                    acc[2 * o + 0] += s1;
-                    acc[2 * o + 1] += s2;
-                }
-                __syncthreads();
+                last[C::quad(s, j)] = x[j][3];
             }
+        };
+        if (c == 0) wtilde(std::integral_constant<int, 0>());
+        else wtilde(std::integral_constant<int, 1>());
+        float w2[QT][4];
+        if constexpr (MC) gaussians(2, s, w2);
+        sync();
+        // v_i takes Wtilde_{i-1}: the quads move up by one step
+        float pj[QT][4];
+#pragma unroll
+        for (int j = 0; j < QT; ++j) {
+            const int q = C::quad(s, j);
+            const float4 p4 = *reinterpret_cast<const float4*>(A.ptab + long(u) * H2 + 4 * q);
+            pj[j][0] = p4.x;
+            pj[j][1] = p4.y;
+            pj[j][2] = p4.z;
+            pj[j][3] = p4.w;
+            x[j][3] = x[j][2];
+            x[j][2] = x[j][1];
+            x[j][1] = x[j][0];
+            x[j][0] = q > 0 ? last[q - 1] : 0.f;
         }
-        for (int o = tid; o < A.out_size; o += 256) {
-            const int I = A.opts[o].out;
-            A.partial[(long(I) * A.nitems + item) * 2 + 0] = acc[2 * o + 0];
-            A.partial[(long(I) * A.nitems + item) * 2 + 1] = acc[2 * o + 1];
+        // ---- 3. the unit's groups
+        for (int g = U.g_begin; g < U.g_end; ++g) {
+            const FusedGroup& G = A.groups[g];
+            const float c1 = G.c1, al = G.al, be = G.be;
+            double d[V];
+#pragma unroll
+            for (int k = 0; k < V; ++k) d[k] = 0.0;
+#pragma unroll
+            for (int j0 = 0; j0 < QT; j0 += CQ) {
+                float f0 = 0.f, f1 = 0.f, f2 = 0.f;
+#pragma unroll
+                for (int j = j0; j < j0 + CQ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float e = fmaf(al, pj[j][r], be);
+                        const float sv = __builtin_amdgcn_exp2f(fmaf(x[j][r], c1, -e));
+                        f0 = fmaf(sv, sv, f0);
+                        f1 = fmaf(sv, w1[j][r], f1);
+                        if constexpr (MC) f2 = fmaf(sv, w2[j][r], f2);
+                    }
+                d[0] += double(f0);
+                d[1] += double(f1);
+                if constexpr (MC) d[2] += double(f2);
+            }
+            // ---- 4. FP64 sums over the path's threads
+            int idx;
+            const double sum = lanes_sum<C::W, V>(d, lane, idx);
+            if (lane % (C::W / V) == 0) red[(s / C::W) * V + idx] = sum;
+            sync();
+            if (s == 0 && p < A.np) {
+                double v[NV];
+#pragma unroll
+                for (int k = 0; k < NV; ++k) {
+                    v[k] = 0.0;
+                    for (int w = 0; w < C::NW; ++w) v[k] += red[w * V + k];
+                }
+                // step 0: v_0 = xi
+                double* out = A.ints + (long(g) * A.np + p) * NV;
+                out[0] = G.dt * (G.xi + v[0]);
+                out[1] = G.sdt * (G.sxi * double(w1[0][0]) + v[1]);
+                if constexpr (MC) out[2] = G.sdt * (G.sxi * double(w2[0][0]) + v[2]);
+            }
+            sync();  // red may be written again
         }
-        __syncthreads();
     }
 }
 
-hipError_t launch_fused_fft(const FftFusedArgs& a, int grid, hipStream_t st) {
-    const size_t lds = fused_fft_lds_bytes(a);
-    const int qpt = fused_fft_qpt(a.N);
-    // the kernels are compiled for the transform length of their quad count
-    const int want = qpt == 1 ? (a.N <= 512 ? 10 : 11) : qpt == 2 ? 12 : qpt == 4 ? 13 : 14;
-    if (a.N < 1 || a.log2L != want) return hipErrorInvalidValue;
-    auto go = [&](auto kern) -> hipError_t {
-        if (lds > 65536) {
-            const hipError_t e = allow_lds(reinterpret_cast<const void*>(kern), lds);
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, st, a);
-        return hipGetLastError();
-    };
-    if (a.mc) {
-        if (qpt == 1) return a.log2L == 10 ? go(&k_fused_fft<1, true, 10>) : go(&k_fused_fft<1, true, 11>);
-        if (qpt <= 2) return go(&k_fused_fft<2, true, 12>);
-        if (qpt <= 4) return go(&k_fused_fft<4, true, 13>);
-        if (qpt <= 8) return go(&k_fused_fft<8, true, 14>);
-    } else {
-        if (qpt == 1) return a.log2L == 10 ? go(&k_fused_fft<1, false, 10>) : go(&k_fused_fft<1, false, 11>);
-        if (qpt <= 2) return go(&k_fused_fft<2, false, 12>);
-        if (qpt <= 4) return go(&k_fused_fft<4, false, 13>);
-        if (qpt <= 8) return go(&k_fused_fft<8, false, 14>);
+// ---------------------------------------------------------------- host side
+int fused_fft_log2(int N) {
+    int l = 10;
+    while ((1 << l) < 2 * N) ++l;
+    return l;
+}
+
+template <class Fn>
+static hipError_t with_log2(int l, Fn fn) {
+    switch (l) {
+        case 10: return fn(std::integral_constant<int, 10>());
+        case 11: return fn(std::integral_constant<int, 11>());
+        case 12: return fn(std::integral_constant<int, 12>());
+        case 13: return fn(std::integral_constant<int, 13>());
+        case 14: return fn(std::integral_constant<int, 14>());
+        default: return hipErrorInvalidValue;
     }
-    return hipErrorInvalidValue;
+}
+
+hipError_t launch_fused_fft_tables(const Unit* units, int nunits, int N, double off, double* gamma, double2* tw64,
+                                   float* ptab, float2* tw, float2* ghat, hipStream_t st) {
+    const int log2L = fused_fft_log2(N), tlen = 1 << (log2L - 1);
+    hipLaunchKernelGGL(k_fft32_tables, dim3(unsigned((tlen + 63) / 64), unsigned(nunits)), dim3(64), 0, st, units, N,
+                       tlen, off, gamma, ptab);
+    hipLaunchKernelGGL(k_fft32_twiddles, dim3(unsigned((fused_fft_table(log2L) + 255) / 256)), dim3(256), 0, st, log2L, tw);
+    if (gamma) {
+        const hipError_t e = launch_fft_spectrum_f32(gamma, nunits, N, tlen, log2L, tw64, ghat, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_fused_fft(FftFusedArgs a, int cus, hipStream_t st) {
+    if (a.np < 1 || a.N < 1 || a.N > 8192 || a.nunits < 1) return hipErrorInvalidValue;
+    return with_log2(fused_fft_log2(a.N), [&](auto l) -> hipError_t {
+        constexpr int LOG2L = decltype(l)::value;
+        using C = FftPair<LOG2L>;
+        const int V = a.mc ? 4 : 2;
+        const size_t lds = size_t(C::PAIRS) * (2 * C::NW * V * sizeof(double) + (C::SLOTS + C::L / 8) * sizeof(float2));
+        const long tiles = ((a.np + 1) / 2 + C::PAIRS - 1) / C::PAIRS;
+        // the units of a tile over as many workgroups as bring four to every CU
+        const long want = (4L * cus + tiles - 1) / tiles;
+        a.nsplit = int(want < a.nunits ? want : a.nunits);
+        auto go = [&](auto kern) -> hipError_t {
+            if (lds > 65536) {
+                const hipError_t e = allow_lds(reinterpret_cast<const void*>(kern), lds);
+                if (e != hipSuccess) return e;
+            }
+            hipLaunchKernelGGL(kern, dim3(unsigned(tiles), unsigned(a.nsplit)), dim3(C::NT), lds, st, a);
+            return hipGetLastError();
+        };
+        return a.mc ? go(&k_fused_fft<LOG2L, true>) : go(&k_fused_fft<LOG2L, false>);
+    });
 }
 
 }  // namespace rb

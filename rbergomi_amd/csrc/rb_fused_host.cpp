@@ -12,6 +12,8 @@
 // A request's results depend only on its own items, so they are bit-identical alone and in any
 // batch.
 #include "rb_fused_host.h"
+#include "rb_fft_lds.h"
+#include "rb_path64.h"
 
 #include <algorithm>
 #include <array>
@@ -152,7 +154,7 @@ void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride
     out.fg.clear();
     out.fpg.clear();
     out.fo.clear();
-    out.ptab.assign(size_t(nu) * Np, 0.f);
+    out.ptab.assign(size_t(nu) * Np, 0.f);  // Np = 0: no row tables
     const double log2e = 1.4426950408889634;
     const double off = req.comp == COMP_EXACT ? 0.0 : 1.0;
     pgmax = 1;
@@ -164,7 +166,7 @@ void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride
         U.sc = float(lay.units[u].sc);
         U.frag_off = u * frag_stride;
         U.p_off = u * Np;
-        for (int j = 1; j < req.N; ++j)
+        for (int j = 1; Np > 0 && j < req.N; ++j)
             out.ptab[size_t(u) * Np + j - pshift] = float(std::pow(double(j) - off, 2.0 * H));
         U.g_begin = int(out.fg.size());
         U.pg_begin = int(out.fpg.size());
@@ -818,30 +820,54 @@ void FftFused::release() {
     out.release();
     if (d_block) (void)hipFreeAsync(d_block, stream);
     d_block = nullptr;
-    d_fu = nullptr;
-    d_fg = nullptr;
-    d_fpg = nullptr;
-    d_fo = nullptr;
-    d_ptab = nullptr;
-    d_ghat = d_tw = nullptr;
+    d_payjobs = nullptr;
+    d_payopts = nullptr;
     d_partial = nullptr;
-    d_counter = nullptr;
-    d_row_off = d_row_n = d_row_M = nullptr;
     d_price = d_stat = d_iv = nullptr;
     d_ivopts = nullptr;
 }
 
-// P table of the long-path kernel: P_i at index i for the 1024 QPT steps its threads visit
-// (QPT quads of four steps per thread, QPT of the instantiation that runs N), +inf at i = 0 and
-// at i >= N so those terms vanish
-static void fft_ptab(const Request& req, const Layout& lay, FusedHostReq& tabs, int& pgmax, int& gmax) {
-    const int N = req.N, len = 1024 * fused_fft_qpt(N);
-    fused_tables(req, lay, len, 0, 0, tabs, pgmax, gmax);
-    for (size_t u = 0; u < lay.units.size(); ++u) {
-        tabs.ptab[u * len] = INFINITY;
-        for (int i = N; i < len; ++i) tabs.ptab[u * len + i] = INFINITY;
-    }
+// The request sizes the long-path kernel takes: a pair's signal with its pad, four waves' sums of
+// eight groups, the records of the unit with the most payoff groups and the sums of every option in
+// one workgroup's LDS.  (Its present form keeps the last two elsewhere; what it refuses is part of
+// the interface.)
+static int fft_request_fits(const FusedHostReq& tabs, int N, int nopt, size_t lds_limit, std::string& err) {
+    int log2L = 10;
+    while ((1 << log2L) < 2 * N - 1) ++log2L;
+    const size_t L = size_t(1) << log2L;
+    int pgu = 1;
+    for (const FusedUnit& U : tabs.fu) pgu = std::max(pgu, U.pg_end - U.pg_begin);
+    const size_t need = (L + L / 32) * sizeof(float2) + 4 * 8 * 2 * 3 * sizeof(double) + size_t(2) * pgu * sizeof(PathPG) +
+                        size_t(nopt) * 2 * sizeof(double);
+    if (need <= lds_limit) return ST_OK;
+    err = "long-path kernel needs " + std::to_string(need) + " bytes of LDS (N or the option count too large)";
+    return ST_ERR_LIMIT;
 }
+
+// Sizes of a request: paths per chunk, so that a chunk's integrals take about 4 MiB, and the block's
+// pieces in bytes
+struct FftSizes {
+    int ppt;
+    long nblk, chunk;
+    size_t ptab, ghat, tw, gamma, tw64, ints, partial;
+    FftSizes(const Request& req, int nunits, int ngroups, int nopt) {
+        const int N = req.N, ns = req.method == METHOD_MC ? 3 : 2;
+        const size_t L = size_t(1) << fused_fft_log2(N);
+        ppt = payoff_paths_per_thread(req.M, nopt);
+        const long pblk = 256L * ppt;
+        nblk = (req.M + pblk - 1) / pblk;
+        chunk = std::max<long>(1, (long(4) << 20) / (8L * ns * ngroups) / pblk) * pblk;
+        chunk = std::min(chunk, nblk * pblk);
+        ptab = nunits * (L / 2) * sizeof(float);
+        ghat = nunits * L * sizeof(float2);
+        tw = fused_fft_table(fused_fft_log2(N)) * sizeof(float2);
+        gamma = N <= 4096 ? nunits * (L / 2) * sizeof(double) : 0;
+        tw64 = N <= 4096 ? path64_fft_table(int(L / 2)) * sizeof(double2) : 0;
+        ints = size_t(ngroups) * chunk * ns * sizeof(double);
+        partial = size_t(nopt) * nblk * 2 * sizeof(double);
+    }
+    size_t total() const { return ptab + ghat + tw + gamma + tw64 + ints + partial; }
+};
 
 int FftFused::plan(const Request& req, const Layout& lay, size_t lds_limit, size_t& footprint, std::string& err) {
     const int N = req.N;
@@ -849,156 +875,129 @@ int FftFused::plan(const Request& req, const Layout& lay, size_t lds_limit, size
         err = "the long-path kernel covers 1024 < N <= 8192";
         return ST_ERR_LIMIT;
     }
-    int log2L = 10;  // L >= 2N - 1, at least 2^10 (the kernel's shortest transform)
-    while ((1 << log2L) < 2 * N - 1) ++log2L;
-    const size_t L = size_t(1) << log2L;
     FusedHostReq tabs;
     int pgmax = 1, gmax = 1;
-    fft_ptab(req, lay, tabs, pgmax, gmax);
-    FftFusedArgs a{};
-    a.log2L = log2L;
-    a.out_size = int(lay.options.size());
-    a.pgu = 1;
-    for (const FusedUnit& U : tabs.fu) a.pgu = std::max(a.pgu, U.pg_end - U.pg_begin);
-    if (fused_fft_lds_bytes(a) > lds_limit) {
-        err = "long-path kernel needs " + std::to_string(fused_fft_lds_bytes(a)) +
-              " bytes of LDS (N or the option count too large)";
-        return ST_ERR_LIMIT;
-    }
-    const long nitems = ((req.M + 1) / 2 + 31) / 32;
-    footprint = lay.units.size() * L * sizeof(float2) + L / 2 * sizeof(float2) + tabs.ptab.size() * sizeof(float) +
-                tabs.fo.size() * sizeof(FusedOption) + tabs.fpg.size() * sizeof(FusedPG) +
-                tabs.fg.size() * sizeof(FusedGroup) + tabs.fu.size() * sizeof(FusedUnit) +
-                lay.options.size() * (sizeof(Option) + 3 * sizeof(double) + 3 * sizeof(long) + size_t(nitems) * 16) + 16;
+    fused_tables(req, lay, 0, 0, 0, tabs, pgmax, gmax);
+    const int rc = fft_request_fits(tabs, N, int(lay.options.size()), lds_limit, err);
+    if (rc) return rc;
+    footprint = FftSizes(req, int(lay.units.size()), int(tabs.fg.size()), int(lay.options.size())).total() +
+                lay.options.size() * (sizeof(Option) + sizeof(PayOpt64) + sizeof(PayJob64)) +
+                tabs.fg.size() * sizeof(FusedGroup) + tabs.fu.size() * (sizeof(FusedUnit) + sizeof(Unit));
     return ST_OK;
 }
 
 int FftFused::build(const Request& req, const Layout& lay, int device, hipStream_t st, std::string& err) {
     release();
     stream = st;
-    const int N = req.N;
-    int log2L = 10;  // L >= 2N - 1, at least 2^10 (the kernel's shortest transform)
-    while ((1 << log2L) < 2 * N - 1) ++log2L;
-    const int L = 1 << log2L;
+    const int N = req.N, nunits = int(lay.units.size());
     if (((N + 3) / 4 + 255) / 256 > 8) {
         err = "the long-path kernel covers N <= 8192";
         return ST_ERR_LIMIT;
     }
     FusedHostReq tabs;
     int pgmax = 1, gmax = 1;
-    fft_ptab(req, lay, tabs, pgmax, gmax);
-    int pgu = 1;
-    for (const FusedUnit& U : tabs.fu) pgu = std::max(pgu, U.pg_end - U.pg_begin);
-    // twiddles and FFT(a, Gamma_1, ..., Gamma_{N-1}) per unit, in FP64, stored in FP32
-    std::vector<float2> tw(L / 2);
-    for (int k = 0; k < L / 2; ++k) {
-        const double ang = -2.0 * M_PI * double(k) / double(L);
-        tw[k] = make_float2(float(std::cos(ang)), float(std::sin(ang)));
-    }
-    std::vector<float2> gh(lay.units.size() * size_t(L));
-    for (size_t u = 0; u < lay.units.size(); ++u) {
-        std::vector<std::complex<double>> g(L, 0.0);
-        g[0] = lay.units[u].a;
-        for (int k = 1; k < N; ++k) g[k] = lay.gamma[u * N + k];
-        fft_host(g, -1);
-        // bit-reversed order: the spectrum's order between the device transforms
-        for (int k = 0; k < L; ++k) {
-            const int b = bit_reverse(k, log2L);
-            gh[u * L + k] = make_float2(float(g[b].real()), float(g[b].imag()));
-        }
-    }
-    FftFusedArgs& a = args;
-    a = FftFusedArgs{};
-    a.N = N;
-    a.log2L = log2L;
-    a.nunits = int(lay.units.size());
-    a.out_size = int(lay.options.size());
-    a.mc = req.method == METHOD_MC ? 1 : 0;
-    a.pgu = pgu;
-    a.pairs_per_item = 32;
-    a.M = req.M;
-    a.npairs = (req.M + 1) / 2;
-    a.nitems = (a.npairs + a.pairs_per_item - 1) / a.pairs_per_item;
-    a.key = philox_key(req.seed.data(), int(req.seed.size()));
-    total_out = a.out_size;
+    fused_tables(req, lay, 0, 0, 0, tabs, pgmax, gmax);
+    total_out = int(lay.options.size());
+    M = req.M;
+    mc = req.method == METHOD_MC;
     hipDeviceProp_t prop;
     RB_TRY(device_props(device, prop));
     keep_pool_cached(device);
-    const size_t lds = fused_fft_lds_bytes(a);
-    if (lds > prop.sharedMemPerBlock) {
-        err = "long-path kernel needs " + std::to_string(lds) + " bytes of LDS (N or the option count too large)";
-        return ST_ERR_LIMIT;
+    cus = prop.multiProcessorCount;
+    const int rc = fft_request_fits(tabs, N, total_out, prop.sharedMemPerBlock, err);
+    if (rc) return rc;
+    const FftSizes sz(req, nunits, int(tabs.fg.size()), total_out);
+    ppt = sz.ppt;
+    nblk = sz.nblk;
+    chunk = sz.chunk;
+    // beyond N = 4096 the FP64 transform of Gamma does not fit a workgroup's LDS: on the host
+    const int log2L = fused_fft_log2(N), L = 1 << log2L;
+    std::vector<float2> gh;
+    if (!sz.gamma) {
+        gh.resize(size_t(nunits) * L);
+        for (int u = 0; u < nunits; ++u) {
+            std::vector<std::complex<double>> g(L, 0.0);
+            const double h = lay.units[u].H - 0.5 + 1.0;
+            g[0] = lay.units[u].a;
+            for (int k = 1; k < N; ++k) g[k] = (std::pow(k + 1.0, h) - std::pow(double(k), h)) / h;
+            fft_host(g, -1);
+            for (int k = 0; k < L; ++k) {
+                const std::complex<double>& v = g[bit_reverse(k, log2L)];
+                gh[size_t(u) * L + fft_spectrum_slot(log2L, k)] = make_float2(float(v.real()), float(v.imag()));
+            }
+        }
     }
-    std::vector<long> row_off(a.out_size), row_n(a.out_size, a.nitems), row_M(a.out_size, a.M);
-    for (int I = 0; I < a.out_size; ++I) row_off[I] = long(I) * a.nitems * 2;
-    // one device block: the tables (one upload from pinned memory, not waited for), then the partial
-    // sums, the item counter and the results
+    std::vector<PayRow> rows;
+    for (const FusedOption& o : tabs.fo) {
+        const FusedPG& pg = tabs.fpg[o.pg];
+        rows.push_back(PayRow{pg.group, o.out, pg.rho, o.K, o.lnK});
+    }
+    std::stable_sort(rows.begin(), rows.end(), [](const PayRow& x, const PayRow& y) {
+        return x.group != y.group ? x.group < y.group : x.rho < y.rho;
+    });
+    std::vector<PayJob64> jobs;
+    std::vector<PayOpt64> opts;
+    payoff_jobs(rows, nblk, cus, jobs, opts);
+    npayjobs = int(jobs.size());
+    // one device block: the tables (one upload from pinned memory, not waited for), what the device
+    // forms from them, integrals, partial sums and results
     size_t off = 0;
     auto place = [&](size_t bytes) {
         const size_t o = off;
         off += (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
         return o;
     };
-    const size_t o_fu = place(tabs.fu.size() * sizeof(FusedUnit)), o_fg = place(tabs.fg.size() * sizeof(FusedGroup)),
-                 o_fpg = place(tabs.fpg.size() * sizeof(FusedPG)), o_fo = place(tabs.fo.size() * sizeof(FusedOption)),
-                 o_ptab = place(tabs.ptab.size() * sizeof(float)), o_gh = place(gh.size() * sizeof(float2)),
-                 o_tw = place(tw.size() * sizeof(float2)), o_roff = place(row_off.size() * sizeof(long)),
-                 o_rn = place(row_n.size() * sizeof(long)), o_rm = place(row_M.size() * sizeof(long)),
-                 o_ivo = place(lay.options.size() * sizeof(Option));
-    const size_t up_bytes = off;
-    const size_t res_bytes = size_t(a.out_size) * 3 * sizeof(double);
-    const size_t o_part = place(size_t(a.out_size) * a.nitems * 2 * sizeof(double)), o_cnt = place(sizeof(int)),
-                 o_out = place(to_host ? 1 : res_bytes);
+    const size_t o_un = place(nunits * sizeof(Unit)), o_fu = place(tabs.fu.size() * sizeof(FusedUnit)),
+                 o_fg = place(tabs.fg.size() * sizeof(FusedGroup)), o_ivo = place(total_out * sizeof(Option)),
+                 o_job = place(jobs.size() * sizeof(PayJob64)), o_opt = place(opts.size() * sizeof(PayOpt64)),
+                 o_gh = place(sz.ghat);
+    const size_t up_bytes = sz.gamma ? o_gh : off;
+    const size_t o_tw = place(sz.tw), o_tw64 = place(sz.tw64), o_gamma = place(sz.gamma), o_ptab = place(sz.ptab),
+                 o_ints = place(sz.ints), o_part = place(sz.partial);
+    const size_t res_bytes = size_t(total_out) * 3 * sizeof(double);
+    const size_t o_out = place(to_host ? 1 : res_bytes);
     RB_TRY(alloc_async(&d_block, off, st));
-    d_fu = reinterpret_cast<FusedUnit*>(d_block + o_fu);
-    d_fg = reinterpret_cast<FusedGroup*>(d_block + o_fg);
-    d_fpg = reinterpret_cast<FusedPG*>(d_block + o_fpg);
-    d_fo = reinterpret_cast<FusedOption*>(d_block + o_fo);
-    d_ptab = reinterpret_cast<float*>(d_block + o_ptab);
-    d_ghat = reinterpret_cast<float2*>(d_block + o_gh);
-    d_tw = reinterpret_cast<float2*>(d_block + o_tw);
-    d_row_off = reinterpret_cast<long*>(d_block + o_roff);
-    d_row_n = reinterpret_cast<long*>(d_block + o_rn);
-    d_row_M = reinterpret_cast<long*>(d_block + o_rm);
-    d_ivopts = reinterpret_cast<Option*>(d_block + o_ivo);
-    d_partial = reinterpret_cast<double*>(d_block + o_part);
-    d_counter = reinterpret_cast<int*>(d_block + o_cnt);
     unsigned char* h = up.reserve(up_bytes);
     d_price = reinterpret_cast<double*>(to_host ? reinterpret_cast<char*>(out.reserve(res_bytes)) : d_block + o_out);
     if (!h || !d_price) {
         err = "cannot allocate pinned host memory";
         return ST_ERR_NOMEM;
     }
-    d_iv = d_price + a.out_size;
-    d_stat = d_iv + a.out_size;
+    d_iv = d_price + total_out;
+    d_stat = d_iv + total_out;
+    d_ivopts = reinterpret_cast<Option*>(d_block + o_ivo);
+    d_payjobs = reinterpret_cast<PayJob64*>(d_block + o_job);
+    d_payopts = reinterpret_cast<PayOpt64*>(d_block + o_opt);
+    d_partial = reinterpret_cast<double*>(d_block + o_part);
     auto pack = [&](size_t o, const auto& v) {
         if (!v.empty()) std::memcpy(h + o, v.data(), v.size() * sizeof(v[0]));
     };
+    pack(o_un, lay.units);
     pack(o_fu, tabs.fu);
     pack(o_fg, tabs.fg);
-    pack(o_fpg, tabs.fpg);
-    pack(o_fo, tabs.fo);
-    pack(o_ptab, tabs.ptab);
-    pack(o_gh, gh);
-    pack(o_tw, tw);
-    pack(o_roff, row_off);
-    pack(o_rn, row_n);
-    pack(o_rm, row_M);
     pack(o_ivo, lay.options);
+    pack(o_job, jobs);
+    pack(o_opt, opts);
+    pack(o_gh, gh);
     RB_TRY(hipMemcpyAsync(d_block, h, up_bytes, hipMemcpyHostToDevice, st));
-    a.units = d_fu;
-    a.groups = d_fg;
-    a.pgs = d_fpg;
-    a.opts = d_fo;
-    a.ptab = d_ptab;
-    a.ghat = d_ghat;
-    a.tw = d_tw;
-    a.partial = d_partial;
-    a.counter = d_counter;
-    const size_t lds_cu = size_t(prop.maxSharedMemoryPerMultiProcessor ? prop.maxSharedMemoryPerMultiProcessor
-                                                                        : prop.sharedMemPerBlock);
-    const int per_cu = int(std::max<size_t>(1, std::min<size_t>(4, lds_cu / lds)));
-    grid = int(std::min<long>(a.nitems, long(prop.multiProcessorCount) * per_cu));
+    FftFusedArgs& a = args;
+    a = FftFusedArgs{};
+    a.key = philox_key(req.seed.data(), int(req.seed.size()));
+    a.N = N;
+    a.nunits = nunits;
+    a.mc = mc ? 1 : 0;
+    a.units = reinterpret_cast<FusedUnit*>(d_block + o_fu);
+    a.groups = reinterpret_cast<FusedGroup*>(d_block + o_fg);
+    a.ptab = reinterpret_cast<float*>(d_block + o_ptab);
+    a.ghat = reinterpret_cast<float2*>(d_block + o_gh);
+    a.tw = reinterpret_cast<float2*>(d_block + o_tw);
+    a.ints = reinterpret_cast<double*>(d_block + o_ints);
+    RB_TRY(launch_fused_fft_tables(reinterpret_cast<const Unit*>(d_block + o_un), nunits, N,
+                                   req.comp == COMP_EXACT ? 0.0 : 1.0,
+                                   sz.gamma ? reinterpret_cast<double*>(d_block + o_gamma) : nullptr,
+                                   sz.gamma ? reinterpret_cast<double2*>(d_block + o_tw64) : nullptr,
+                                   reinterpret_cast<float*>(d_block + o_ptab), reinterpret_cast<float2*>(d_block + o_tw),
+                                   reinterpret_cast<float2*>(d_block + o_gh), st));
     return ST_OK;
 }
 
@@ -1008,14 +1007,22 @@ int FftFused::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_t 
         if (timing) timing->mark(slot, nullptr, nullptr);
     };
     int s;
-    RB_TRY(launch_zero_int(d_counter, 1, st));
     if (kbeg) RB_TRY(hipEventRecord(kbeg, st));
-    s = timed(K_FUSED);
-    RB_TRY(launch_fused_fft(args, grid, st));
-    mark(s);
+    for (long p0 = 0; p0 < M; p0 += chunk) {
+        FftFusedArgs a = args;
+        a.p0 = p0;
+        a.np = std::min(chunk, M - p0);
+        s = timed(K_FUSED);
+        RB_TRY(launch_fused_fft(a, cus, st));
+        mark(s);
+        s = timed(K_PAYOFF);
+        RB_TRY(launch_payoff64(a.ints, a.np, ppt, d_payjobs, npayjobs, d_payopts, total_out, mc ? PAY_MC_MIX : PAY_RT_MIX,
+                               p0 / (256L * ppt), nblk, d_partial, nullptr, st));
+        mark(s);
+    }
     if (kend) RB_TRY(hipEventRecord(kend, st));
     s = timed(K_REDUCE);
-    RB_TRY(launch_reduce_iv(d_partial, ReduceRows{d_row_off, d_row_n, d_row_M, 0, 0}, d_ivopts, total_out, d_price,
+    RB_TRY(launch_reduce_iv(d_partial, ReduceRows{nullptr, nullptr, nullptr, nblk, M}, d_ivopts, total_out, d_price,
                             d_stat, d_iv, nullptr, st));
     mark(s);
     return ST_OK;

@@ -8,6 +8,7 @@
 
 #include "rb_fused.h"
 #include "rb_hostmem.h"
+#include "rb_payoff64.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -43,20 +44,14 @@ void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride
 // at the mixed precisions, any N <= 8192 at RB_PREC_FP32_FFT.
 struct FftFused {
     FftFusedArgs args{};
-    int grid = 0, total_out = 0;
+    int total_out = 0, cus = 256;
+    bool mc = false;
+    long M = 0, chunk = 0, nblk = 0;  // paths, paths per launch, payoff blocks
+    int ppt = 1, npayjobs = 0;
     hipStream_t stream = nullptr;
-    FusedUnit* d_fu = nullptr;
-    FusedGroup* d_fg = nullptr;
-    FusedPG* d_fpg = nullptr;
-    FusedOption* d_fo = nullptr;
-    float* d_ptab = nullptr;
-    float2* d_ghat = nullptr;
-    float2* d_tw = nullptr;
+    PayJob64* d_payjobs = nullptr;
+    PayOpt64* d_payopts = nullptr;
     double* d_partial = nullptr;
-    int* d_counter = nullptr;
-    long* d_row_off = nullptr;
-    long* d_row_n = nullptr;
-    long* d_row_M = nullptr;
     double* d_price = nullptr;
     double* d_stat = nullptr;
     double* d_iv = nullptr;

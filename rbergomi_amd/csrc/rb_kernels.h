@@ -67,6 +67,11 @@ hipError_t launch_volterra_fft(const double* Z, long zstride, long np, int N, in
                                const Unit* units, const float2* ghat, const float2* tw, double* Wt,
                                hipStream_t st);
 
+// Spectrum of gamma (tlen doubles per unit) by an FP64 transform of length 2^log2L <= 2^13, rounded to
+// FP32, and its FP64 twiddles (scratch, path64_fft_table entries) (rb_path64_fft.hip)
+hipError_t launch_fft_spectrum_f32(const double* gamma, int nunits, int N, int tlen, int log2L, double2* tw,
+                                   float2* ghat, hipStream_t st);
+
 // Sobol' Gaussians (quasi-Monte Carlo), same [path][stream][N] layout as the Philox ones
 hipError_t launch_normals_sobol_f64(const uint32_t* V, const uint32_t* shift, long p0, long np,
                                     int nstreams, int N, double* out, hipStream_t st);

@@ -25,7 +25,9 @@
 #include <type_traits>
 
 #include "rb_fft64.h"
+#include "rb_fft_lds.h"
 #include "rb_kernels.h"
+#include "rb_lanes.h"
 #include "rb_math64.h"
 #include "rb_path64.h"
 
@@ -66,18 +68,6 @@ __global__ void k_fft64_twiddles(double2* __restrict__ tab) {
     }
 }
 
-struct BlockSync {
-    __device__ __forceinline__ void operator()() const { __syncthreads(); }
-};
-// threads of one wave: LDS operations of a wave complete in order, so only the compiler is held
-struct WaveSync {
-    __device__ __forceinline__ void operator()() const {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-};
-
 // The spectrum of (gamma_0 .. gamma_{N-1}) / L of every unit, in the middle pass's register order:
 // element 16 t + k at [k][t].  Grid: units; block TP threads.
 template <int LOG2L>
@@ -98,6 +88,25 @@ __global__ void __launch_bounds__(Fft64<LOG2L>::TP) k_fft64_spectrum(const doubl
         ghat[(long(blockIdx.x) * 16 + k) * F::TP + t] = make_double2(x[k].x * s, x[k].y * s);
 }
 
+// The same unscaled and rounded to FP32, in the order of FftSpectrum, for the mixed-precision kernel
+// (rb_fused_fft.hip)
+template <int LOG2L>
+__global__ void __launch_bounds__(Fft64<LOG2L>::TP) k_fft64_spectrum_f32(const double* __restrict__ gamma, int N,
+                                                                          int tlen, const double2* __restrict__ tab,
+                                                                          float2* __restrict__ ghat) {
+    using F = Fft64<LOG2L>;
+    extern __shared__ double2 lds[];
+    const int t = threadIdx.x;
+    const double* g = gamma + long(blockIdx.x) * tlen;
+    for (int i = t; i < F::L / 2; i += F::TP) lds[fpad64(i)] = make_double2(i < N ? g[i] : 0.0, 0.0);
+    const Fft64Run<LOG2L, BlockSync> fft{lds, tab, t, BlockSync()};
+    double2 x[16];
+    fft.forward(x);
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+        ghat[long(blockIdx.x) * F::L + fft_spectrum_slot(LOG2L, 16 * t + k)] = make_float2(float(x[k].x), float(x[k].y));
+}
+
 // ---------------------------------------------------------------- the path kernel
 template <int LOG2L>
 struct Path64Fft {
@@ -109,28 +118,6 @@ struct Path64Fft {
 
 // LDS behind the transforms' slots, in doubles
 constexpr int P64F_MAXV = 8;  // values summed per group and pair
-
-// Sum v[0 .. V) over W lanes (V = 4 or 8 = 2^B): each of B steps hands half of the values to the
-// partner lane, so that a lane ends with one value of index `idx`, summed over all W lanes.
-template <int W, int V>
-__device__ __forceinline__ double lanes_sum(double (&v)[V], int lane, int& idx) {
-    int off = W / 2;
-    idx = 0;
-#pragma unroll
-    for (int n = V / 2; n >= 1; n >>= 1, off >>= 1) {
-        const bool hi = lane & off;
-#pragma unroll
-        for (int i = 0; i < n; ++i) {
-            const double send = hi ? v[i] : v[i + n], keep = hi ? v[i + n] : v[i];
-            v[i] = keep + __shfl_xor(send, off, 64);
-        }
-        idx = 2 * idx + (hi ? 1 : 0);
-    }
-    double s = v[0];
-#pragma unroll
-    for (; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-    return s;
-}
 
 template <int SRC>
 __device__ __forceinline__ void path64f_gauss(const Path64Args& A, const double2* lg, long p, int s, int q, double z[4]) {
@@ -390,6 +377,23 @@ hipError_t launch_path64_fft_tables(const double* gamma, int nunits, int N, int 
         hipLaunchKernelGGL((k_fft64_twiddles<LOG2L>), dim3((F::TABLE + 255) / 256), dim3(256), 0, st, tw);
         hipLaunchKernelGGL((k_fft64_spectrum<LOG2L>), dim3(unsigned(nunits)), dim3(F::TP), lds, st, gamma, N, tlen, tw,
                            ghat);
+        return hipGetLastError();
+    });
+}
+
+hipError_t launch_fft_spectrum_f32(const double* gamma, int nunits, int N, int tlen, int log2L, double2* tw,
+                                   float2* ghat, hipStream_t st) {
+    return with_log2(log2L, [&](auto l) -> hipError_t {
+        constexpr int LOG2L = decltype(l)::value;
+        using F = Fft64<LOG2L>;
+        const size_t lds = F::SLOTS * sizeof(double2);
+        if (lds > 65536) {
+            const hipError_t e = allow_lds(reinterpret_cast<const void*>(&k_fft64_spectrum_f32<LOG2L>), lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL((k_fft64_twiddles<LOG2L>), dim3((F::TABLE + 255) / 256), dim3(256), 0, st, tw);
+        hipLaunchKernelGGL((k_fft64_spectrum_f32<LOG2L>), dim3(unsigned(nunits)), dim3(F::TP), lds, st, gamma, N, tlen,
+                           tw, ghat);
         return hipGetLastError();
     });
 }

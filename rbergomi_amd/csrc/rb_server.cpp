@@ -104,7 +104,7 @@ int plan_job(const rb_request* q, int precision, int method, int comp, Job& j, s
     int rc = request_of(q, precision, method, comp, j.req, err);
     if (rc) return rc;
     const Request& r = j.req;
-    j.lay = make_layout(r);
+    j.lay = make_layout(r, r.N <= 1024);  // the long-path kernel forms Gamma itself
     j.price = q->price;
     j.iv = q->iv;
     j.stat = q->stat;

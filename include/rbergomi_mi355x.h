@@ -391,8 +391,9 @@ int rb_probe_copy(long bytes, int reps, double* avg_ms);
  * the fused kernels is priced with these. */
 int rb_probe_issue(double* ns_per_inst, int* simds);
 /* The split-precision kernels' per-path payoff for given (ln S', sigma, K) -> out[i], and its
- * Mills-ratio approximation at z[i] -> mills[i] (n values).  form 0: the fused GEMM kernel's
- * (deep out-of-the-money tail through erfcx), 1: the long-path kernel's (through erfc). */
+ * Mills-ratio approximation at z[i] -> mills[i] (n values).  form: 0 or 1, the fused
+ * GEMM kernel's and the long-path kernel's, which are one (deep out of the money in FP64, through
+ * Mills ratios). */
 int rb_probe_payoff(const double* lnS, const double* sig, const double* K, int n, double* out,
                     const float* z, float* mills, int form);
 /* Per-path integrals (Ivdt, IsvdW) of option I from Z: out[2*(m*out_size + I) + {0,1}] */

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "rb_device.h"
+#include "rb_math64.h"
 #include "rb_types.h"
 
 namespace rb {
@@ -154,11 +155,9 @@ __device__ __forceinline__ float mills_f32(float z) { return mills_den(fmaf(z, 0
 // selects (no divergent branch in the strike loop).  In FP32 from the record's scaled fields
 // (u = s d, s = sqrt(log2(e) / 2)): u2 = A - ln K ik, u1 = u2 + sg, E = exp2(LK - u2^2), and
 // the Mills-ratio denominators 1 + |u| / (3 s).  Deep out of the money (d1 < -8,
-// Phi(d1) < 7e-16) the normal CDFs are evaluated in FP64, in one of two forms of the same value:
-// Phi(e) = exp(-e^2/2) erfcx(-e/sqrt 2) / 2 with S' exp(-e1^2/2) = K exp(-e2^2/2), one
-// exponential (the default: fewer instructions), or S' Phi(e1) - K Phi(e2) through erfc
-// (LOWREG: fewer live registers, for the long-path kernel, which holds its Gaussians in
-// registers; the erfcx form raised its register spills from 51 to 121 at N = 4096).
+// Phi(d1) < 7e-16) the payoff is evaluated in FP64 as S' phi(e1) (M(-e1) - M(-e2)), the Mills ratios
+// by mills_pair: some 80 FP64 instructions on the lanes of a wave that reach it, against 130 with two
+// library erfcx and 250 with two erfc.
 // Multiply-adds are written out (no implicit contraction), so every kernel instantiation that
 // inlines this computes the same bits.
 // the FP32 part; deep: d1 < -8, where the caller takes payoff_deep instead
@@ -176,23 +175,26 @@ __device__ __forceinline__ double payoff_f32(const PathPG& q, const OptF& o, boo
     return double(u2 >= 0.f ? x_itm : (u1 >= 0.f ? x_mid : x_otm));
 }
 
-// the FP64 deep out-of-the-money form
-template <bool LOWREG = false>
-__device__ __forceinline__ double payoff_deep(const PathPG& q, double lnK, double K) {
+// the FP64 deep out-of-the-money form (e2 < e1 < -8; beyond 1000 the exponential is 0)
+__device__ __forceinline__ double payoff_deep(const PathPG& q, double lnK) {
 #pragma clang fp contract(off)
     const double e1 = (q.lnS - lnK) / q.sig + 0.5 * q.sig, e2 = e1 - q.sig;
-    if constexpr (LOWREG)
-        return exp(q.lnS) * phi_f64(e1) - K * phi_f64(e2);
-    else
-        return 0.5 * exp(q.lnS - 0.5 * e1 * e1) *
-               (erfcx(-0.7071067811865476 * e1) - erfcx(-0.7071067811865476 * e2));
+    // the coefficients are read here, by scalar loads: as literals they are hoisted out of the
+    // caller's loops into scalar registers it does not have (60 to 130 spilled)
+    using ConstD = const __attribute__((address_space(4))) double*;
+    ConstD c = (ConstD)MILLS_POLY;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(c));
+#endif
+    double m1, m2;
+    mills_pair(fmin(-e1, 1000.0), fmin(-e2, 1000.0), m1, m2, c);
+    return 0.3989422804014327 * exp(q.lnS - 0.5 * e1 * e1) * (m1 - m2);
 }
 
-template <bool LOWREG = false>
-__device__ __forceinline__ double payoff_mixed(const PathPG& q, const OptF& o, double lnK, double K) {
+__device__ __forceinline__ double payoff_mixed(const PathPG& q, const OptF& o, double lnK) {
     bool deep;
     const double x = payoff_f32(q, o, deep);
-    return deep ? payoff_deep<LOWREG>(q, lnK, K) : x;
+    return deep ? payoff_deep(q, lnK) : x;
 }
 
 // plain Monte Carlo payoff (S_T - K)^+ in FP64 (S_T in the sig slot)

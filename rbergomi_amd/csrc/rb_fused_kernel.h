@@ -614,7 +614,7 @@ __global__ void __launch_bounds__(256, UPW >= 8 ? 1 : 2) k_fused(FusedBatchArgs 
                             double s1 = 0.0, s2 = 0.0;
                             for (int pl = 0; pl < np; ++pl) {
                                 const double x = MC ? payoff_mc(pgd[pl * A.pgmax + pgl], O.K)
-                                                    : payoff_mixed(pgd[pl * A.pgmax + pgl], of, O.lnK, O.K);
+                                                    : payoff_mixed(pgd[pl * A.pgmax + pgl], of, O.lnK);
                                 s1 += x;
                                 s2 += x * x;
                             }
@@ -634,7 +634,7 @@ __global__ void __launch_bounds__(256, UPW >= 8 ? 1 : 2) k_fused(FusedBatchArgs 
                             double s1 = 0.0, s2 = 0.0;
                             for (int pl = sl; pl < np; pl += S) {
                                 const double x = MC ? payoff_mc(pgd[pl * A.pgmax + pgl], O.K)
-                                                    : payoff_mixed(pgd[pl * A.pgmax + pgl], of, O.lnK, O.K);
+                                                    : payoff_mixed(pgd[pl * A.pgmax + pgl], of, O.lnK);
                                 s1 += x;
                                 s2 += x * x;
                             }

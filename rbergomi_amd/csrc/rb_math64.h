@@ -223,16 +223,17 @@ static constexpr double MILLS_POLY[23] = {
     0x1.73593d9b065c3p-31, 0x1.77b6c9a1ffe4dp-29};
 
 // The Mills ratios of x, y in [0, 1e4], two independent chains on one reciprocal
-__host__ __device__ __forceinline__ void mills_pair(double x, double y, double& mx, double& my) {
+template <class P = const double*>
+__host__ __device__ __forceinline__ void mills_pair(double x, double y, double& mx, double& my, P c = MILLS_POLY) {
     constexpr double k = 4.5;
     const double dx = x + k, dy = y + k, inv = rcp_pos(dx * dy);
     const double ix = inv * dy, iy = inv * dx;
     const double u = (x - k) * ix, w = (y - k) * iy;
-    double a = MILLS_POLY[22], b = MILLS_POLY[22];
+    double a = c[22], b = c[22];
 #pragma unroll
     for (int i = 21; i >= 0; --i) {
-        a = fma(a, u, MILLS_POLY[i]);
-        b = fma(b, w, MILLS_POLY[i]);
+        a = fma(a, u, c[i]);
+        b = fma(b, w, c[i]);
     }
     mx = a * ix;
     my = b * iy;

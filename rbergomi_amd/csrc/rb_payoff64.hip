@@ -57,7 +57,7 @@ struct PayRtMix {  // mixed-precision Romano-Touzi (Iv, Is)
         pathpg_f32(q);
     }
     __device__ __forceinline__ double pay(const double*, const PayOpt64& o) const {
-        return payoff_mixed<true>(q, opt_f32(o.lnK, o.K), o.lnK, o.K);
+        return payoff_mixed(q, opt_f32(o.lnK, o.K), o.lnK);
     }
 };
 struct PayMcMix {  // plain MC (Iv, Is, Ip): ln S_T = rho Is + sqrt(1 - rho^2) Ip - Iv / 2

@@ -66,7 +66,7 @@ __global__ void k_probe_payoff(const double* __restrict__ lnS, const double* __r
     pathpg_f32(q);
     const double lnK = log(K[i]);
     const OptF of = opt_f32(lnK, K[i]);
-    out[i] = form ? payoff_mixed<true>(q, of, lnK, K[i]) : payoff_mixed<false>(q, of, lnK, K[i]);
+    out[i] = payoff_mixed(q, of, lnK);  // one form serves both kernels
     mills_out[i] = mills_f32(z[i]);
 }
 

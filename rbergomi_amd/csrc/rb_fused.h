@@ -130,6 +130,7 @@ struct FusedBatchArgs {
     int wpart_d;                 // LDS: cross-wave partials, in doubles
     int pgd_n;                   // LDS: per-(path, payoff group) records of one group chunk
     int acc_d;                   // LDS: option sums (largest request in LDS mode), in doubles
+    int per_cu;                  // workgroups per CU of the launch (k_fused's WG at four row blocks per wave)
 };
 
 // Mills ratio M(z) = (1 - Phi(z)) / phi(z) for z >= 0, as M = t P(t), t = 1/(1 + z/3), with P a

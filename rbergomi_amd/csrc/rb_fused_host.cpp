@@ -395,9 +395,10 @@ static hipError_t batch_alloc(DevArena* ar, T** p, size_t n, hipStream_t st) {
 }
 
 size_t fused_batch_lds(const std::vector<const FusedHostReq*>& reqs, size_t lds_cu, FusedBatchArgs* a, int* cap) {
-    int bf = 0, wp = 0, pg = 0, ac = 0, ns = 2;
+    int bf = 0, wp = 0, pg = 0, ac = 0, ns = 2, upw = 1;
     for (const FusedHostReq* q : reqs) {
         const FusedReq& r = q->r;
+        upw = std::max(upw, q->upw);
         ns = r.mc ? 3 : 2;
         bf = std::max(bf, r.PB * r.NK * r.chunk_u4);
         wp = std::max(wp, 4 * r.gchunk * 32 * ns);
@@ -405,12 +406,17 @@ size_t fused_batch_lds(const std::vector<const FusedHostReq*>& reqs, size_t lds_
         ac = std::max(ac, r.acc_in_lds ? 2 * r.out_size : 0);
     }
     const size_t stat = sizeof(FusedReq) + 16;  // the kernel's static record and item index
-    const size_t half = lds_cu / 2;
+    const size_t half = lds_cu / 2, third = lds_cu / 3;
     const size_t rest = size_t(bf) * 16 + size_t(pg) * sizeof(PathPG) + size_t(ac) * 8 + stat;
     int c_cap = 0;
-    if (rest + size_t(wp) * 8 > half) {
-        for (int c = FUSED_GREG; c >= 1 && c_cap == 0; --c)
-            if (rest + size_t(4 * c * 32 * ns) * 8 <= half) c_cap = c;
+    // chunks of half a pass's groups or more if that lets a third workgroup onto the CU (N = 512, FP16,
+    // eight groups 2.09 -> 1.95 ms, N = 320, BF16, five groups 1.29 -> 1.20), of any size if it lets a second
+    for (const size_t share : {third, half}) {
+        if (share == third && upw > 4) continue;  // its registers do not fit three times
+        if (rest + size_t(wp) * 8 <= share || c_cap > 0) break;
+        const int c_min = share == third ? (wp / (4 * 32 * ns) + 1) / 2 : 1;
+        for (int c = FUSED_GREG; c >= c_min && c_cap == 0; --c)
+            if (rest + size_t(4 * c * 32 * ns) * 8 <= share) c_cap = c;
         if (c_cap > 0) {
             wp = 0;
             for (const FusedHostReq* q : reqs) wp = std::max(wp, 4 * std::min(q->r.gchunk, c_cap) * 32 * ns);
@@ -594,8 +600,8 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
     hipDeviceProp_t prop;
     RB_TRY(device_props(device, prop));
     if (!arena) keep_pool_cached(device);
-    // Two workgroups per CU need at most half the CU's LDS each, the static request record
-    // included; fused_batch_lds cuts the cross-wave partials' chunk of groups when that helps.
+    // Two or three workgroups per CU need at most half or a third of the CU's LDS each, the static request
+    // record included; fused_batch_lds cuts the cross-wave partials' chunk of groups when that helps.
     const size_t lds_cu = size_t(prop.maxSharedMemoryPerMultiProcessor ? prop.maxSharedMemoryPerMultiProcessor
                                                                         : prop.sharedMemPerBlock);
     int cap = 0;
@@ -764,8 +770,13 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
     args.item_req = d_item_req;
     args.item_local = d_item_local;
     args.counter = d_counter;
-    const int per_cu = int(std::max<size_t>(1, std::min<size_t>(2, lds_cu / lds_total)));
-    grid = int(std::min<long>(args.total_items, long(prop.multiProcessorCount) * per_cu));
+    // Three workgroups per CU where their LDS fits (and their registers: up to four row blocks per
+    // wave).  Vector instructions of two waves per SIMD do not issue back to back: N = 512, M = 2^22, FP16,
+    // five groups 6.51 -> 6.00 ms, M = 2^20, one group 1.24 -> 1.06, plain MC, two groups 1.13 -> 1.00,
+    // N = 256, five groups 0.95 -> 0.81, 48 server requests 22.9 -> 20.6.  Where only two fit the
+    // registers of three cost (N = 512, eight groups 2.08 -> 2.31, BF16, five groups 1.79 -> 1.93).
+    args.per_cu = int(std::max<size_t>(1, std::min<size_t>(upw <= 4 ? 3 : 2, lds_cu / lds_total)));
+    grid = int(std::min<long>(args.total_items, long(prop.multiProcessorCount) * args.per_cu));
     // pageable sources: the host tables die with this call
     if (!staged) RB_TRY(hipStreamSynchronize(st));
     return ST_OK;

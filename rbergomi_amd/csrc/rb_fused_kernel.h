@@ -174,9 +174,10 @@ __device__ __forceinline__ double half_sum_f64(double v) {
     return v;
 }
 
-// GR: groups integrated per pass over the accumulators (at most FUSED_GREG)
-template <int MODE, int UPW, bool MC, int GR>
-__global__ void __launch_bounds__(256, UPW >= 8 ? 1 : 2) k_fused(FusedBatchArgs B) {
+// GR: groups integrated per pass over the accumulators (at most FUSED_GREG).  WG: workgroups per CU
+// (waves per SIMD) the registers are cut for.
+template <int MODE, int UPW, bool MC, int GR, int WG>
+__global__ void __launch_bounds__(256, WG) k_fused(FusedBatchArgs B) {
     static_assert(GR <= FUSED_GREG, "pgmax is sized for windows of FUSED_GREG groups");
     constexpr int NS = MC ? 3 : 2;                        // sums per (path, group)
     typedef SplitT<MODE> S;
@@ -496,19 +497,28 @@ __global__ void __launch_bounds__(256, UPW >= 8 ? 1 : 2) k_fused(FusedBatchArgs 
                             // lane's 16 row terms of a group are four aligned float4 loads, those
                             // of the next group issued before this group's rows (two buffers by
                             // the parity of the group); slots past gn reload the last group's.
-                            float qv[2][16];
-                            load_rows16(Qr, qv[0]);
+                            // With three waves per SIMD one buffer, read at the group's start, and
+                            // the groups one after the other: their rows interleaved hold every
+                            // group's row terms at once (36 to 111 registers spilled, now 0 to
+                            // 61), and the other waves fill the gaps (N = 512, M = 2^22, five
+                            // groups: 6.24 -> 6.00 ms; with two waves interleaved 6.51).
+                            constexpr bool SEQ = WG == 3;
+                            float qv[SEQ ? 1 : 2][16];
+                            if constexpr (!SEQ) load_rows16(Qr, qv[0]);
 #pragma unroll
                             for (int gg = 0; gg < GR; ++gg) {
-                                if (gg + 1 < GR)
+                                if constexpr (SEQ)
+                                    load_rows16(Qr + (gg < gn ? gg : gn - 1) * A.Np, qv[0]);
+                                else if (gg + 1 < GR)
                                     load_rows16(Qr + (gg + 1 < gn ? gg + 1 : gn - 1) * A.Np, qv[(gg + 1) & 1]);
 #pragma unroll
                                 for (int r = 0; r < 16; ++r) {
-                                    const float rr = __builtin_amdgcn_exp2f(fmaf(acc[s][r], c1[gg], -qv[gg & 1][r]));
+                                    const float rr = __builtin_amdgcn_exp2f(fmaf(acc[s][r], c1[gg], -qv[SEQ ? 0 : gg & 1][r]));
                                     fv[gg] = fmaf(rr, rr, fv[gg]);
                                     fs[gg] = fmaf(rr, wv[r], fs[gg]);
                                     if constexpr (MC) fp[gg] = fmaf(rr, wq[r], fp[gg]);
                                 }
+                                if constexpr (SEQ) __builtin_amdgcn_sched_barrier(0);
                             }
                             if constexpr (!MC) {
 #pragma unroll
@@ -681,32 +691,34 @@ __global__ void __launch_bounds__(256, UPW >= 8 ? 1 : 2) k_fused(FusedBatchArgs 
 
 size_t fused_lds_bytes(const FusedBatchArgs& b);
 
-template <int MODE, int UPW, bool MC, int GR>
+template <int MODE, int UPW, bool MC, int GR, int WG>
 static hipError_t launch_t(const FusedBatchArgs& a, int grid, hipStream_t st) {
     const size_t lds = fused_lds_bytes(a);
     if (lds > 65536) {
-        const hipError_t e = allow_lds(reinterpret_cast<const void*>(&k_fused<MODE, UPW, MC, GR>), lds);
+        const hipError_t e = allow_lds(reinterpret_cast<const void*>(&k_fused<MODE, UPW, MC, GR, WG>), lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_fused<MODE, UPW, MC, GR>), dim3(grid), dim3(256), lds, st, a);
+    hipLaunchKernelGGL((k_fused<MODE, UPW, MC, GR, WG>), dim3(grid), dim3(256), lds, st, a);
     return hipGetLastError();
+}
+
+template <int MODE, bool MC, int GR>
+static hipError_t launch_u(int upw, const FusedBatchArgs& a, int grid, hipStream_t st) {
+    switch (upw) {
+        case 1: return launch_t<MODE, 1, MC, GR, 3>(a, grid, st);
+        case 2: return launch_t<MODE, 2, MC, GR, 3>(a, grid, st);
+        case 4: return a.per_cu == 3 ? launch_t<MODE, 4, MC, GR, 3>(a, grid, st) : launch_t<MODE, 4, MC, GR, 2>(a, grid, st);
+        case 8: return launch_t<MODE, 8, MC, GR, 1>(a, grid, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 template <bool MC, int GR>
 static hipError_t launch_mu(int mode, int upw, const FusedBatchArgs& a, int grid, hipStream_t st) {
-    switch (mode * 16 + upw) {
-        case 1: return launch_t<0, 1, MC, GR>(a, grid, st);
-        case 2: return launch_t<0, 2, MC, GR>(a, grid, st);
-        case 4: return launch_t<0, 4, MC, GR>(a, grid, st);
-        case 8: return launch_t<0, 8, MC, GR>(a, grid, st);
-        case 17: return launch_t<1, 1, MC, GR>(a, grid, st);
-        case 18: return launch_t<1, 2, MC, GR>(a, grid, st);
-        case 20: return launch_t<1, 4, MC, GR>(a, grid, st);
-        case 24: return launch_t<1, 8, MC, GR>(a, grid, st);
-        case 33: return launch_t<2, 1, MC, GR>(a, grid, st);
-        case 34: return launch_t<2, 2, MC, GR>(a, grid, st);
-        case 36: return launch_t<2, 4, MC, GR>(a, grid, st);
-        case 40: return launch_t<2, 8, MC, GR>(a, grid, st);
+    switch (mode) {
+        case 0: return launch_u<0, MC, GR>(upw, a, grid, st);
+        case 1: return launch_u<1, MC, GR>(upw, a, grid, st);
+        case 2: return launch_u<2, MC, GR>(upw, a, grid, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -340,11 +340,16 @@ int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHos
     a.mc = req.method == METHOD_MC ? 1 : 0;
     a.M = req.M;
     a.ntiles = (req.M + a.TP - 1) / a.TP;
-    // work items of at most 1024 paths, and at least 256 per request where its tiles allow, so a
-    // small request alone still spreads over the chip (N = 64, M = 2^16: 64 items of 1024 paths
-    // took 0.170 ms, 256 items of 256 paths 0.089 ms).  The item size depends on the request
-    // only, so its sums are added in the same order alone and in any batch.
-    a.tiles_per_item = int(std::max<long>(1, std::min<long>(1024 / a.TP, (a.ntiles + 255) / 256)));
+    // Work items of at most 1024 paths, and 1024 or more per request where its tiles allow: three
+    // workgroups on each CU take 768, and a request of some hundred items would leave a launch
+    // of its own with one or two each (N = 512, M = 2^18, five maturities: 256 items 0.72 ms, 1024 items
+    // 0.43, 2048 items 0.46; N = 365, M = 3e5, plain MC, BF16: 293 items 0.72, 938 items 0.49), but
+    // beyond 256 items no less than 2^14 path steps each (a call of N = 64, M = 2^16: 256 items 0.108 ms, 512
+    // items 0.118).  The item size depends on the request only, so its sums are added in the same order
+    // alone and in any batch.
+    const long steps = long(N) * a.TP;
+    const long least = std::min((a.ntiles + 255) / 256, ((1L << 14) + steps - 1) / steps);
+    a.tiles_per_item = int(std::max<long>(1, std::min<long>(1024 / a.TP, std::max((a.ntiles + 1023) / 1024, least))));
     a.nitems = (a.ntiles + a.tiles_per_item - 1) / a.tiles_per_item;
     a.items_big = a.nitems;
     a.tiles_small = a.tiles_per_item;

@@ -553,7 +553,7 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
         p64.ptab = d_p64tab + size_t(nunits) * p64.tlen;
         RB_TRY(launch_path64_tables(d_units, int(nunits), N, p64.tlen, r.comp == COMP_EXACT ? 0.0 : 1.0, d_p64tab,
                                     d_p64tab + size_t(nunits) * p64.tlen, stream));
-        if (path64_uses_fft(N)) {
+        if (path64_fft) {
             p64.tw = d_p64fft;
             p64.ghat = d_p64fft + path64_fft_table(N);
             RB_TRY(launch_path64_fft_tables(p64.gamma, int(nunits), N, p64.tlen, d_p64fft,
@@ -575,7 +575,7 @@ void Plan::begin_timing() {
     else if (conv_fft)
         times[K_VOLTERRA].name = "k_volterra_fft";
     else if (path64)
-        times[K_VOLTERRA].name = path64_uses_fft(req.N) ? "k_path64_fft" : "k_path64";
+        times[K_VOLTERRA].name = path64_fft ? "k_path64_fft" : "k_path64";
     else if (volterra_conv_mfma(req.N, lds_limit))
         times[K_VOLTERRA].name = "k_volterra_mfma_long_f64";
 }
@@ -632,7 +632,7 @@ int Plan::integrals(uint64_t p0, long np, bool from_z, int signs, std::string& e
         a.zstride = long(nstreams) * req.N;
         a.ints = d_ints;
         a.ints2 = d_ints2;
-        if (path64_uses_fft(req.N)) {
+        if (path64_fft) {
             path64_fft_shape(a, cus);
             RB_LAUNCH(K_VOLTERRA, launch_path64_fft(a, stream));
         } else {
@@ -879,7 +879,8 @@ void Plan::init_path64() {
     upload(&d_p64groups, groups);
     upload(&d_p64jobs, jobs);
     dalloc(&d_p64tab, size_t(2) * nunits * p64.tlen);
-    if (path64_uses_fft(N)) dalloc(&d_p64fft, path64_fft_table(N) + (size_t(nunits) << path64_fft_log2(N)));
+    path64_fft = path64_uses_fft(N, int(nunits), int(groups.size()), req.method == METHOD_MC);
+    if (path64_fft) dalloc(&d_p64fft, path64_fft_table(N) + (size_t(nunits) << path64_fft_log2(N)));
 }
 
 hipError_t Plan::conv(long np, long zstride) {

@@ -161,6 +161,7 @@ struct Plan {
     long* d_count = nullptr;      // [options] their totals
     // single-pass FP64 path (hybrid scheme, FP64): no Gaussians or Wtilde in HBM unless the caller's
     bool path64 = false;
+    bool path64_fft = false;  // by transforms (path64_uses_fft)
     Path64Args p64{};             // tables and launch shape; the paths are set per chunk
     Path64Group* d_p64groups = nullptr;
     Path64Job* d_p64jobs = nullptr;

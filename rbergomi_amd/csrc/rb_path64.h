@@ -71,10 +71,10 @@ void path64_shape(Path64Args& a, int cus);
 size_t path64_lds_bytes(const Path64Args& a);
 hipError_t launch_path64(const Path64Args& a, hipStream_t st);
 
-// The transform kernel (N <= 4096, and whether it is taken for N): length 2^log2 >= 2N, twiddle and spectrum tables (path64_fft_table
+// The transform kernel (N <= 4096, and whether it is taken): length 2^log2 >= 2N, twiddle and spectrum tables (path64_fft_table
 // and L entries per unit), LDS
 constexpr int PATH64_FFT_MAX_N = 4096, PATH64_FFT_MIN_LOG2 = 9;
-bool path64_uses_fft(int N);
+bool path64_uses_fft(int N, int units, int groups, bool mc);
 int path64_fft_log2(int N);
 void path64_fft_shape(Path64Args& a, int cus);
 size_t path64_fft_table(int N);

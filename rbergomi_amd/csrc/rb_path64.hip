@@ -1,5 +1,5 @@
 // rb_path64.hip -- the FP64 path in one pass: from Gaussians to the integrals of every group, with
-// nothing per step in HBM (N <= 384; rb_path64_fft.hip beyond).
+// nothing per step in HBM (N <= 384 where products are cheaper than transforms, path64_uses_fft; rb_path64_fft.hip else).
 //
 // A workgroup owns a tile of 16 PT paths (PT = 1, 2 or 4 sub-tiles of 16):
 //   1. W1 of the tile, k-major in LDS: Philox and Box-Muller in place (genGaussianMT,

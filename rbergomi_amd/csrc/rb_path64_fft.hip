@@ -313,11 +313,21 @@ int path64_fft_log2(int N) {
     return l;
 }
 
-// Measured per 1.6e8 paths*steps, Romano-Touzi / plain MC (ms), products on the matrix cores against
-// transforms: N = 256 1.19 / 1.46 against 1.11 / 1.55 (L = 512), N = 300 1.36 / 1.60 against 2.00 / 2.78
-// (L = 1024), N = 400 1.64 / 1.93 against 1.51 / 2.10, N = 512 1.87 / 2.16 against 1.19 / 1.66: the
-// products grow with N, the transforms with L / N, and they cross at about 3/4 of L = 1024.
-bool path64_uses_fft(int N) { return N > 384; }
+// Time of 8e7 paths*steps in microseconds, of the transforms and of the products on the matrix cores, as
+// fitted to plans of 104 <= N <= 512: Gaussians, then per unit a transform (the same for every N of a length)
+// or a product (growing with N), then per group.  Romano-Touzi, one unit and group, measured at N = 224,
+// 256, 304, 360, 384: transforms 627, 559, 904, 771, 727, products 613, 628, 707, 808, 842; one
+// unit, five groups at 256, 384: 788, 1042 against 864, 1029; three units at 176, 200, 256, 304, 336: 1607, 1420,
+// 1126, 1894, 1718 against 1304, 1565, 1596, 1879, 2000; plain MC, one unit at 224, 256, 384: 831, 731, 942
+// against 721, 768, 971.  Beyond N = 384 products lose even where transforms fill their length least (N = 400,
+// plain MC, five groups: 1548 against 1350).
+bool path64_uses_fft(int N, int units, int groups, bool mc) {
+    if (N > 384) return true;
+    const double u = units, g = groups, r = double(1 << path64_fft_log2(N)) / 2 / N;
+    const double fft = r * (mc ? 386 + 262 * u + 83 * g : 276 + 226 * u + 57 * g);
+    const double mm = (mc ? 225 : 115) + u * (110 + 1.37 * N) + 60 * g;
+    return fft < mm;
+}
 
 template <class Fn>
 static hipError_t with_log2(int l, Fn fn) {

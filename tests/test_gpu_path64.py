@@ -100,3 +100,19 @@ def test_extreme_coefficients_stay_finite_where_the_model_is(rb):
     assert np.max(np.abs(iv - 0.2)) < 1e-10
     price, _, _ = rb.price_v2(0.04, [0.1], [400.0], [-0.5], np.ones(3), K, 37, 50, [1])
     assert np.all(np.isfinite(price))
+
+
+# either side of the choice between products and transforms, which depends on units and groups: transforms of
+# length 512 (N <= 256), products and transforms up to N = 384
+@pytest.mark.parametrize("units,mats,N", [(1, 1, 231), (1, 1, 256), (2, 2, 224), (3, 1, 193), (4, 1, 255), (1, 5, 256),
+                                          (1, 1, 336), (1, 1, 368), (1, 8, 384), (3, 3, 340)])
+def test_choice_of_kernel(rb, orc, units, mats, N):
+    xi, (H, eta, rho, T, K) = 0.04, _params(units, mats, N)
+    for method in (0, 1):
+        M = 131
+        print("path64 choice N=%d units=%d mats=%d method=%d" % (N, units, mats, method), flush=True)
+        Z = orc.normals_philox([11, N], 0, M, 2 + method, N)
+        fn = orc.payoff_mc_samples if method else orc.payoff_rt_samples
+        price, stat = orc.price_stat(fn(xi, H, eta, rho, T, K, N, Z))
+        p, _, s = rb.price_v2(xi, H, eta, rho, T, K, N, M, [11, N], precision=rb.PREC_FP64, method=method)
+        assert np.max(np.abs(p - price)) < 1e-12 and np.max(np.abs(s - stat)) < 1e-12

@@ -19,7 +19,7 @@
 // plain MC, none or 4 for Romano-Touzi; with the passes' twiddles hoisted out of the loop over the jobs
 // 40 to 100, and N = 512 took 1.19 ms per 1.6e8 path steps where it takes 1.08, N = 4096 2.23, now 1.72),
 // and its 17 KB of LDS per wave the CU's.  N = 2048, M = 16384, one maturity: 3.05 (k_normals,
-// k_volterra_mfma_long, k_scan) -> 0.29 ms; 1.2e11 paths*steps/s at N = 1024 and 2048.
+// k_volterra_mfma_long, k_scan) -> 0.25 ms; 1.3e11 paths*steps/s at N = 1024 and 2048.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -154,28 +154,56 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
 
     const int N = A.N, nq = (N + 3) >> 2;
     const long pr = long(blockIdx.x) * C::PAIRS + pair, pa = 2 * pr;
-    // ---- 1. Gaussians through LDS (the loop stays rolled): W1 in place for the transform, the other
-    // streams through the upper half
+    // ---- 1. Gaussians.  At two waves per SIMD a quad's chains of dependent FP64 instructions (a logarithm,
+    // a root, a sine) leave the unit idle unless other quads' fill the waits: Romano-Touzi forms the
+    // quads of both paths and both streams together (N = 256, M = 655360: one quad at a time 1155 us a call, two
+    // paths' 1093, all four 1051; five groups at N = 512, M = 2^19: 2891, 2820, 2713).  Plain MC has no registers
+    // for that: its loop takes two paths' at a time, rolled, and its values go through LDS, W1 in place for the
+    // transform, the other streams through the upper half, or 16 to 60 registers are spilled.
     double2 w1[2][4], wp[2][4], w2[MC ? 2 : 1][4];
-    auto gaussians = [&](int s, int at, double2(&w)[2][4]) {
-#pragma unroll 1
-        for (int i = 0; i < 4; ++i) {
-            const int c = i & 1, q = t + TP * (i >> 1);
-            double g[4] = {0.0, 0.0, 0.0, 0.0};
-            if (q < nq) path64f_gauss<SRC>(A, lg, pa + c, s, q, g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) reinterpret_cast<double*>(z + fpad64(at + 4 * q + r))[c] = g[r];
+    auto quad = [&](int s, int q, double2(&w)[4]) {
+        double g[4] = {0.0, 0.0, 0.0, 0.0}, h[4] = {0.0, 0.0, 0.0, 0.0};
+        if (q < nq) {
+            path64f_gauss<SRC>(A, lg, pa, s, q, g);
+            path64f_gauss<SRC>(A, lg, pa + 1, s, q, h);
         }
-        WaveSync()();  // the thread's own values
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) w[j][r] = z[fpad64(at + 4 * (t + TP * j) + r)];
-        WaveSync()();
+        for (int r = 0; r < 4; ++r) w[r] = make_double2(g[r], h[r]);
     };
-    gaussians(0, 0, w1);
-    gaussians(1, L / 2, wp);
-    if constexpr (MC) gaussians(2, L / 2, w2);
+    if constexpr (MC) {
+        auto gaussians = [&](int s, int at, double2(&w)[2][4]) {
+#pragma unroll 1
+            for (int j = 0; j < 2; ++j) {
+                double2 v[4];
+                quad(s, t + TP * j, v);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) z[fpad64(at + 4 * (t + TP * j) + r)] = v[r];
+            }
+            WaveSync()();  // the thread's own values
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[j][r] = z[fpad64(at + 4 * (t + TP * j) + r)];
+            WaveSync()();
+        };
+        gaussians(0, 0, w1);
+        gaussians(1, L / 2, wp);
+        gaussians(2, L / 2, w2);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int q = t + TP * j;
+            double g[4][4] = {};
+            if (q < nq)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) path64f_gauss<SRC>(A, lg, pa + (k & 1), k >> 1, q, g[k]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                w1[j][r] = z[fpad64(4 * q + r)] = make_double2(g[0][r], g[1][r]);
+                wp[j][r] = make_double2(g[2][r], g[3][r]);
+            }
+        }
+    }
     // the first value of the next quad of each of the thread's quads
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -317,7 +345,7 @@ int path64_fft_log2(int N) {
 // fitted to plans of 104 <= N <= 512: Gaussians, then per unit a transform (the same for every N of a length)
 // or a product (growing with N), then per group.  Romano-Touzi, one unit and group, measured at N = 224,
 // 256, 304, 360, 384: transforms 627, 559, 904, 771, 727, products 613, 628, 707, 808, 842; one
-// unit, five groups at 256, 384: 788, 1042 against 864, 1029; three units at 176, 200, 256, 304, 336: 1607, 1420,
+// unit, five groups at 256, 384: 788, 1042 against 864, 1029 (transforms since take 40 less); three units at 176, 200, 256, 304, 336: 1607, 1420,
 // 1126, 1894, 1718 against 1304, 1565, 1596, 1879, 2000; plain MC, one unit at 224, 256, 384: 831, 731, 942
 // against 721, 768, 971.  Beyond N = 384 products lose even where transforms fill their length least (N = 400,
 // plain MC, five groups: 1548 against 1350).

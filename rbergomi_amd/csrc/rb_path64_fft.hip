@@ -19,7 +19,7 @@
 // plain MC, none or 4 for Romano-Touzi; with the passes' twiddles hoisted out of the loop over the jobs
 // 40 to 100, and N = 512 took 1.19 ms per 1.6e8 path steps where it takes 1.08, N = 4096 2.23, now 1.72),
 // and its 17 KB of LDS per wave the CU's.  N = 2048, M = 16384, one maturity: 3.05 (k_normals,
-// k_volterra_mfma_long, k_scan) -> 0.25 ms; 1.3e11 paths*steps/s at N = 1024 and 2048.
+// k_volterra_mfma_long, k_scan) -> 0.27 ms; 1.3e11 paths*steps/s at N = 1024 and 2048.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -158,27 +158,16 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
     // a root, a sine) leave the unit idle unless other quads' fill the waits: Romano-Touzi forms the
     // quads of both paths and both streams together (N = 256, M = 655360: one quad at a time 1155 us a call, two
     // paths' 1093, all four 1051; five groups at N = 512, M = 2^19: 2891, 2820, 2713).  Plain MC has no registers
-    // for that: its loop takes two paths' at a time, rolled, and its values go through LDS, W1 in place for the
-    // transform, the other streams through the upper half, or 16 to 60 registers are spilled.
+    // for the values: its loops are rolled and the values go through LDS, W1 in place for the transform, the
+    // other streams through the upper half, or 16 to 60 registers are spilled (five groups at N = 512, M = 2^22: a quad at a
+    // time 27.4 ms, two 26.8, the first two streams together 26.5).
     double2 w1[2][4], wp[2][4], w2[MC ? 2 : 1][4];
-    auto quad = [&](int s, int q, double2(&w)[4]) {
-        double g[4] = {0.0, 0.0, 0.0, 0.0}, h[4] = {0.0, 0.0, 0.0, 0.0};
-        if (q < nq) {
-            path64f_gauss<SRC>(A, lg, pa, s, q, g);
-            path64f_gauss<SRC>(A, lg, pa + 1, s, q, h);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) w[r] = make_double2(g[r], h[r]);
-    };
     if constexpr (MC) {
-        auto gaussians = [&](int s, int at, double2(&w)[2][4]) {
-#pragma unroll 1
-            for (int j = 0; j < 2; ++j) {
-                double2 v[4];
-                quad(s, t + TP * j, v);
+        auto put = [&](int at, int j, const double2(&v)[4]) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) z[fpad64(at + 4 * (t + TP * j) + r)] = v[r];
-            }
+            for (int r = 0; r < 4; ++r) z[fpad64(at + 4 * (t + TP * j) + r)] = v[r];
+        };
+        auto get = [&](int at, double2(&w)[2][4]) {
             WaveSync()();  // the thread's own values
 #pragma unroll
             for (int j = 0; j < 2; ++j)
@@ -186,9 +175,37 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
                 for (int r = 0; r < 4; ++r) w[j][r] = z[fpad64(at + 4 * (t + TP * j) + r)];
             WaveSync()();
         };
-        gaussians(0, 0, w1);
-        gaussians(1, L / 2, wp);
-        gaussians(2, L / 2, w2);
+#pragma unroll 1
+        for (int j = 0; j < 2; ++j) {
+            const int q = t + TP * j;
+            double g[4][4] = {};
+            if (q < nq)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) path64f_gauss<SRC>(A, lg, pa + (k & 1), k >> 1, q, g[k]);
+            double2 v[4], u[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] = make_double2(g[0][r], g[1][r]);
+                u[r] = make_double2(g[2][r], g[3][r]);
+            }
+            put(0, j, v);
+            put(L / 2, j, u);
+        }
+        get(0, w1);
+        get(L / 2, wp);
+#pragma unroll 1
+        for (int j = 0; j < 2; ++j) {
+            const int q = t + TP * j;
+            double g[2][4] = {};
+            if (q < nq)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) path64f_gauss<SRC>(A, lg, pa + k, 2, q, g[k]);
+            double2 v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = make_double2(g[0][r], g[1][r]);
+            put(L / 2, j, v);
+        }
+        get(L / 2, w2);
     } else {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {

@@ -198,14 +198,22 @@ __global__ void __launch_bounds__((FftPair<LOG2L>::NT), (FftPair<LOG2L>::WAVES))
     const Sync sync{};
     const int N = A.N, nq = (N + 3) >> 2;
     const long pr = long(blockIdx.x) * C::PAIRS + pair, p = 2 * pr + c;
-    // ---- 1. Gaussians of the thread's quads
+    // ---- 1. Gaussians of the thread's quads, two at a time where the whole wave needs both: their chains of
+    // dependent instructions fill each other's waits (one at a time, N = 4096, M = 32768: 698 us a call, now 689;
+    // N = 2048, M = 60003, two maturities 551 -> 544; drawn for lanes that need one only, N = 1100 lost 3%)
     auto gaussians = [&](uint32_t stream, int s, float(&w)[QT][4]) {
 #pragma unroll
-        for (int j = 0; j < QT; ++j) {
-            const int q = C::quad(s, j);
+        for (int j = 0; j < QT; j += 2) {
+            const int q = C::quad(s, j), qn = C::quad(s, j + 1);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[j][r] = 0.f;
-            if (q < nq) normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(q), w[j]);
+            for (int r = 0; r < 4; ++r) w[j][r] = w[j + 1][r] = 0.f;
+            if (__all(qn < nq)) {
+                normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(q), w[j]);
+                normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(qn), w[j + 1]);
+            } else {
+                if (q < nq) normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(q), w[j]);
+                if (qn < nq) normals4_f32(A.key, uint64_t(A.p0 + p), stream, uint32_t(qn), w[j + 1]);
+            }
         }
     };
     float w1[QT][4];

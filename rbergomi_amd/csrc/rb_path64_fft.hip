@@ -17,7 +17,7 @@
 // triangular product on the matrix cores (which keep the vector unit) takes N / 2.  A thread's 16
 // points and 16 steps of each stream fill the registers of two waves per SIMD (4 to 26 spilled for
 // plain MC, none or 4 for Romano-Touzi; with the passes' twiddles hoisted out of the loop over the jobs
-// 40 to 100, and N = 512 took 1.19 ms per 1.6e8 path steps where it takes 1.08, N = 4096 2.23, now 1.72),
+// 40 to 100, and N = 512 took 1.19 ms per 1.6e8 path steps where it then took 1.08, N = 4096 2.23 and 1.72),
 // and its 17 KB of LDS per wave the CU's.  N = 2048, M = 16384, one maturity: 3.05 (k_normals,
 // k_volterra_mfma_long, k_scan) -> 0.27 ms; 1.3e11 paths*steps/s at N = 1024 and 2048.
 #include <hip/hip_runtime.h>
@@ -360,16 +360,18 @@ int path64_fft_log2(int N) {
 
 // Time of 8e7 paths*steps in microseconds, of the transforms and of the products on the matrix cores, as
 // fitted to plans of 104 <= N <= 512: Gaussians, then per unit a transform (the same for every N of a length)
-// or a product (growing with N), then per group.  Romano-Touzi, one unit and group, measured at N = 224,
-// 256, 304, 360, 384: transforms 627, 559, 904, 771, 727, products 613, 628, 707, 808, 842; one
-// unit, five groups at 256, 384: 788, 1042 against 864, 1029 (transforms since take 40 less); three units at 176, 200, 256, 304, 336: 1607, 1420,
+// or a product (growing with N), then per group.  Measured, transforms against products: Romano-Touzi, one
+// unit and group at N = 224, 256, 304, 360, 384: 627, 559, 904, 771, 727 against 613, 628, 707, 808, 842; one
+// unit, five groups at 256, 384: 788, 1042 against 864, 1029; three units at 176, 200, 256, 304, 336: 1607, 1420,
 // 1126, 1894, 1718 against 1304, 1565, 1596, 1879, 2000; plain MC, one unit at 224, 256, 384: 831, 731, 942
-// against 721, 768, 971.  Beyond N = 384 products lose even where transforms fill their length least (N = 400,
-// plain MC, five groups: 1548 against 1350).
+// against 721, 768, 971.  Since Romano-Touzi's transforms form four quads of Gaussians together they take 48 r
+// less (r: padded over real length); whole calls at N = 224, 360: 619, 759 against 627, 836, three groups at 360 934
+// against 991, five at 380 1012 against 1067.  Beyond N = 384 products lose even where transforms fill their
+// length least (N = 400, plain MC, five groups: 1548 against 1350).
 bool path64_uses_fft(int N, int units, int groups, bool mc) {
     if (N > 384) return true;
     const double u = units, g = groups, r = double(1 << path64_fft_log2(N)) / 2 / N;
-    const double fft = r * (mc ? 386 + 262 * u + 83 * g : 276 + 226 * u + 57 * g);
+    const double fft = r * (mc ? 386 + 262 * u + 83 * g : 228 + 226 * u + 57 * g);
     const double mm = (mc ? 225 : 115) + u * (110 + 1.37 * N) + 60 * g;
     return fft < mm;
 }

@@ -482,6 +482,10 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     // one path per payoff thread in the turbo-charged estimator, whose own payoff kernel sums 256
     ppt = r.turbo ? 1 : payoff_paths_per_thread(r.M, nopt);
     const long pblk = 256L * ppt;
+    if (path64) {
+        path64_fft = path64_uses_fft(N, int(nunits), int(ngroups), r.method == METHOD_MC);
+        ch = std::min(ch, path64_fft ? path64_fft_max_paths(N) : path64_max_paths(N));
+    }
     ch = std::max(pblk, ch / pblk * pblk);
     const long Mr = (r.M + pblk - 1) / pblk * pblk;
     chunk = std::min(ch, Mr);
@@ -879,7 +883,6 @@ void Plan::init_path64() {
     upload(&d_p64groups, groups);
     upload(&d_p64jobs, jobs);
     dalloc(&d_p64tab, size_t(2) * nunits * p64.tlen);
-    path64_fft = path64_uses_fft(N, int(nunits), int(groups.size()), req.method == METHOD_MC);
     if (path64_fft) dalloc(&d_p64fft, path64_fft_table(N) + (size_t(nunits) << path64_fft_log2(N)));
 }
 

@@ -70,6 +70,10 @@ int path64_greg(int groups_of_largest_unit, int signs);
 void path64_shape(Path64Args& a, int cus);
 size_t path64_lds_bytes(const Path64Args& a);
 hipError_t launch_path64(const Path64Args& a, hipStream_t st);
+// Paths one launch takes: HIP has no grid of 2^32 threads or more a dimension, and the product kernel spends up to
+// 512 threads on 16 paths, the transform kernel 32 on a path (N <= 512) to 256 (N > 2048).  Larger requests go
+// in chunks.
+long path64_max_paths(int N);
 
 // The transform kernel (N <= 4096, and whether it is taken): length 2^log2 >= 2N, twiddle and spectrum tables (path64_fft_table
 // and L entries per unit), LDS
@@ -77,6 +81,7 @@ constexpr int PATH64_FFT_MAX_N = 4096, PATH64_FFT_MIN_LOG2 = 9;
 bool path64_uses_fft(int N, int units, int groups, bool mc);
 int path64_fft_log2(int N);
 void path64_fft_shape(Path64Args& a, int cus);
+long path64_fft_max_paths(int N);
 size_t path64_fft_table(int N);
 hipError_t launch_path64_fft_tables(const double* gamma, int nunits, int N, int tlen, double2* tw, double2* ghat,
                                     hipStream_t st);

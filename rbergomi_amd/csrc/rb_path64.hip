@@ -110,6 +110,9 @@ void path64_shape(Path64Args& a, int cus) {
     if (path64_lds_bytes(a) > P64_LDS_CU / 3 && path64_blocks(a.N) >= 8) a.threads = 512;
 }
 
+// tiles by the larger of the two workgroup sizes
+long path64_max_paths(int N) { return ((1L << 32) - 1) / 512 * 16 * path64_subtiles(N); }
+
 // groups per job: the smallest instantiated count that holds a unit's groups, 8 at most
 int path64_greg(int most, int signs) { return signs == 2 || most <= 2 ? 2 : most <= 4 ? 4 : 8; }
 
@@ -347,7 +350,7 @@ __global__ void __launch_bounds__(NT, 4) k_path64(Path64Args A) {
 hipError_t launch_path64(const Path64Args& a, hipStream_t st) {
     const size_t lds = path64_lds_bytes(a);
     const int per = 16 * path64_subtiles(a.N);
-    if (a.np < 1 || a.njobs < 1 || a.nsplit < 1 || a.N > PATH64_MFMA_MAX_N || a.tlen != (a.N + 15) / 16 * 16)
+    if (a.np < 1 || a.njobs < 1 || a.nsplit < 1 || a.N > PATH64_MFMA_MAX_N || a.np > path64_max_paths(a.N) || a.tlen != (a.N + 15) / 16 * 16)
         return hipErrorInvalidValue;
     const dim3 grid(unsigned((a.np + per - 1) / per), unsigned(a.nsplit));
     auto go = [&](auto kern) -> hipError_t {

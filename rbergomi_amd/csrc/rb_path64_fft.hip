@@ -400,6 +400,16 @@ void path64_fft_shape(Path64Args& a, int cus) {
     a.nsplit = int(want < a.njobs ? want : a.njobs);
 }
 
+long path64_fft_max_paths(int N) {
+    long n = 0;
+    (void)with_log2(path64_fft_log2(N), [&](auto l) {
+        using C = Path64Fft<decltype(l)::value>;
+        n = ((1L << 32) - 1) / C::NT * 2 * C::PAIRS;
+        return hipSuccess;
+    });
+    return n;
+}
+
 size_t path64_fft_table(int N) {
     size_t n = 0;
     (void)with_log2(path64_fft_log2(N), [&](auto l) {
@@ -456,7 +466,8 @@ hipError_t launch_fft_spectrum_f32(const double* gamma, int nunits, int N, int t
 }
 
 hipError_t launch_path64_fft(const Path64Args& a, hipStream_t st) {
-    if (a.np < 1 || a.njobs < 1 || a.nsplit < 1 || a.N > PATH64_FFT_MAX_N) return hipErrorInvalidValue;
+    if (a.np < 1 || a.njobs < 1 || a.nsplit < 1 || a.N > PATH64_FFT_MAX_N || a.np > path64_fft_max_paths(a.N))
+        return hipErrorInvalidValue;
     return with_log2(path64_fft_log2(a.N), [&](auto l) -> hipError_t {
         constexpr int LOG2L = decltype(l)::value;
         using C = Path64Fft<LOG2L>;

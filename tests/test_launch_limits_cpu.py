@@ -1,0 +1,39 @@
+"""Launches of the FP64 path at path counts that one grid does not hold, planned by the built library on the
+recording runtime (recording.py), which refuses a grid as HIP does (gridDim * blockDim of 2^32 or more): every
+path is launched once, in chunks whose payoff blocks are whole."""
+import pytest
+
+import recording
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    return recording.build(tmp_path_factory.mktemp("recording"))
+
+
+CODE = """
+for method in (rb.METHOD_RT, rb.METHOD_MC):
+    for N in (1, 17, 33, 64, 128, 200, 256, 300, 360, 384, 385, 512, 513, 1024, 1025, 2048, 2049, 4096):
+        for M in ((1 << 24) + 1, 1000000007):
+            p = rb.Plan(0.04, [0.1], [1.9], [-0.7], [1.0], [1.0], N, M, [1], method=method)
+            p.run()
+            p.close()
+            at = 0
+            for name, f in launches("k_path64"):
+                if "np" not in f:
+                    continue
+                assert f["p0"] == at and f["grid"] * f["block"] < 2 ** 32, (N, M, name, f)
+                at += f["np"]
+                assert at == M or f["np"] % 1024 == 0, (N, M, name, f)
+            assert at == M, (N, M, at)
+# the mirrored paths of the turbo-charged estimator, with its pilot paths in a launch of their own
+for N in (200, 4096):
+    M, pilot = 300000000, 1000000
+    rb.price_rows_turbo([0.04], [0.1], [1.9], [-0.7], [1.0], [1.0], N, M, [1], m_control=pilot)
+    assert sum(f["np"] for _, f in launches("k_path64") if "np" in f) == M + pilot
+print("ok")
+"""
+
+
+def test_every_path_is_launched_within_the_grid(lib):
+    assert recording.run(lib, CODE).strip().endswith("ok")

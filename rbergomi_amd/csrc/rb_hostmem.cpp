@@ -42,7 +42,9 @@ unsigned char* Pinned::reserve(size_t bytes) {
         }
     }
     void* p = nullptr;
-    if (hipHostMalloc(&p, want, hipHostMallocPortable) != hipSuccess) {
+    // coherent whatever HIP_HOST_COHERENT says: kernels write results here, and the host reads them after an event
+    // or a stream alone
+    if (hipHostMalloc(&p, want, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }

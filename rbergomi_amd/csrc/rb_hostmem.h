@@ -11,7 +11,7 @@
 
 namespace rb {
 
-// A pinned host block of at least the bytes asked for, from the pool (blocks are powers of two from
+// A pinned, coherent host block of at least the bytes asked for, from the pool (blocks are powers of two from
 // 64 KiB; up to 64 MiB of idle blocks are kept), returned to it with the object.
 class Pinned {
   public:

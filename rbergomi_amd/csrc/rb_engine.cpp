@@ -311,47 +311,52 @@ void ws_free(void* p) {
 }
 
 // A plan's device buffers are one workspace block, with everything to upload at its front: one
-// allocation and one copy per plan.
+// allocation and, for tables of up to PINNED_TABLES, one copy per plan.
+static size_t align256(size_t n) { return (n + 255) / 256 * 256; }
+
 template <class T>
 void Plan::dalloc(T** p, size_t n) {
     mem.push_back({reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(T)});
 }
 
 template <class T>
-void Plan::upload(T** p, const std::vector<T>& v) {
-    const size_t at = (up.size() + 255) / 256 * 256;
-    up.resize(at + v.size() * sizeof(T));
-    if (!v.empty()) std::memcpy(up.data() + at, v.data(), v.size() * sizeof(T));
-    up_at.push_back({reinterpret_cast<void**>(p), at});
+void Plan::upload(T** p, std::vector<T> v) {
+    const auto held = std::make_shared<const std::vector<T>>(std::move(v));
+    const size_t at = align256(up_bytes);
+    up_bytes = at + held->size() * sizeof(T);
+    up.push_back({reinterpret_cast<void**>(p), held, held->data(), held->size() * sizeof(T), at});
 }
 
 int Plan::commit(std::string& err) {
-    size_t total = (up.size() + 255) / 256 * 256;
-    for (const auto& m : mem) total += (m.second + 255) / 256 * 256;
+    // tables and results share a pinned block (the copy reads it and the last kernel writes it without
+    // the host waiting); it is the plan's, and the plan waits for its stream before it goes.  Larger tables
+    // are copied from where they are, and without pinned memory the results are too
+    const size_t n = lay.options.size();
+    size_t total = align256(up_bytes);
+    const size_t front = up_bytes <= PINNED_TABLES ? total : 0;
+    unsigned char* h = host.reserve(front + 3 * n * sizeof(double));
+    if (!h) dalloc(&d_price, 3 * n);
+    for (const auto& m : mem) total += align256(m.second);
     RB_TRY(ws_alloc(&d_block, total));
     char* base = static_cast<char*>(d_block);
-    for (const auto& u : up_at) *u.first = base + u.second;
-    size_t at = (up.size() + 255) / 256 * 256;
+    for (const Table& t : up) *t.p = base + t.at;
+    size_t at = align256(up_bytes);
     for (const auto& m : mem) {
         *m.first = base + at;
-        at += (m.second + 255) / 256 * 256;
+        at += align256(m.second);
     }
-    // tables and results share a pinned block (the copy reads it and the last kernel writes it without
-    // the host waiting); it is the plan's, and the plan waits for its stream before it goes
-    const size_t res = (up.size() + 255) / 256 * 256;
-    unsigned char* h = host.reserve(res + 3 * lay.options.size() * sizeof(double));
-    if (!h) {
-        err = "cannot allocate pinned host memory";
-        return ST_ERR_NOMEM;
+    if (h) d_price = reinterpret_cast<double*>(h + front);
+    d_stat = d_price + n;
+    d_iv = d_stat + n;
+    const bool packed = h && front > 0;
+    for (const Table& t : up) {
+        if (t.bytes == 0) continue;
+        if (packed) std::memcpy(h + t.at, t.src, t.bytes);
+        else RB_TRY(hipMemcpyAsync(base + t.at, t.src, t.bytes, hipMemcpyHostToDevice, stream));
     }
-    d_price = reinterpret_cast<double*>(h + res);
-    d_stat = d_price + lay.options.size();
-    d_iv = d_stat + lay.options.size();
-    if (!up.empty()) {
-        std::memcpy(h, up.data(), up.size());
-        RB_TRY(hipMemcpyAsync(base, h, up.size(), hipMemcpyHostToDevice, stream));
-    }
-    std::vector<char>().swap(up);
+    if (packed && up_bytes > 0) RB_TRY(hipMemcpyAsync(base, h, up_bytes, hipMemcpyHostToDevice, stream));
+    if (!packed) RB_TRY(hipStreamSynchronize(stream));  // the tables go now
+    up.clear();
     return ST_OK;
 }
 
@@ -528,12 +533,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     if (r.scheme == SCHEME_CHOLESKY) {
         // host factor per unit (distinct H), then one upload
         std::vector<double> all, L;
+        all.reserve(lay.units.size() * 2 * size_t(N) * N);
         for (const Unit& un : lay.units) {
             rc = chol_factor(un.H, N, L, err);
             if (rc) return rc;
             all.insert(all.end(), L.begin(), L.end());
         }
-        upload(&d_chol, all);
+        upload(&d_chol, std::move(all));
     }
     if (need_z) dalloc(&d_Z, size_t(chunk) * nstreams * N);
     if (!path64) dalloc(&d_Wt, size_t(nunits) * chunk * N);
@@ -807,7 +813,7 @@ int Plan::init_fft(std::string& err) {
         for (int k = 0; k < L; ++k) gh[u * L + k] = make_float2(float(a[k].real()), float(a[k].imag()));
     }
     upload(&d_tw, tw);
-    upload(&d_ghat, gh);
+    upload(&d_ghat, std::move(gh));
     return ST_OK;
 }
 
@@ -916,14 +922,15 @@ int Plan::turbo_results(double* alpha, double* Q, long* exceptions, std::string&
 int Plan::results(double* price, double* iv, double* stat, std::string& err) {
     RB_TRY(hipStreamSynchronize(stream));
     if (fused) {
-        fused_batch->fetch(0, price, iv, stat);
+        RB_TRY(fused_batch->fetch(0, price, iv, stat));
     } else if (fused_fft) {
-        fused_fft->fetch(price, iv, stat);
+        RB_TRY(fused_fft->fetch(price, iv, stat));
     } else {
         const size_t n = lay.options.size();
-        if (price) std::copy_n(d_price, n, price);
-        if (stat) std::copy_n(d_stat, n, stat);
-        if (iv) std::copy_n(d_iv, n, iv);
+        const bool pinned = host.data() != nullptr;
+        RB_TRY(fetch_results(price, d_price, n, pinned));
+        RB_TRY(fetch_results(stat, d_stat, n, pinned));
+        RB_TRY(fetch_results(iv, d_iv, n, pinned));
     }
     return ST_OK;
 }

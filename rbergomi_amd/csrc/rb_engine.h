@@ -122,14 +122,20 @@ struct Plan {
     int nstreams = 2;        // Gaussian blocks per path: W1, W1perp (+ Wperp for plain MC)
     // the block that holds every device buffer below, and what its front is filled from
     void* d_block = nullptr;
-    std::vector<std::pair<void**, size_t>> mem;    // buffers and their bytes
-    std::vector<std::pair<void**, size_t>> up_at;  // uploaded tables and their places in `up`
-    std::vector<char> up;
-    Pinned host;                                   // `up` on its way to the device, and the results
+    std::vector<std::pair<void**, size_t>> mem;  // buffers and their bytes
+    struct Table {
+        void** p;
+        std::shared_ptr<const void> hold;        // keeps src
+        const void* src;
+        size_t bytes, at;                        // its place in the block
+    };
+    std::vector<Table> up;                       // uploaded tables
+    size_t up_bytes = 0;
+    Pinned host;                                 // tables on their way to the device, and the results
     template <class T>
     void dalloc(T** p, size_t n);
     template <class T>
-    void upload(T** p, const std::vector<T>& v);
+    void upload(T** p, std::vector<T> v);
     int commit(std::string& err);
     // device tables
     Unit* d_units = nullptr;
@@ -145,7 +151,8 @@ struct Plan {
     double* d_Wt = nullptr;       // [units][chunk][N]
     double* d_ints = nullptr;     // [groups][chunk][2]
     double* d_partial = nullptr;  // [options][nblk][2]
-    // results, in the plan's pinned host memory: the reduction writes them there
+    // results, in the plan's pinned host memory: the reduction writes them there (in the block where no pinned
+    // memory could be had)
     double* d_price = nullptr;
     double* d_stat = nullptr;
     double* d_iv = nullptr;

@@ -693,7 +693,9 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
                  o_reqs = place(R.size() * sizeof(FusedReq)), o_cnt = place(sizeof(int));
     const size_t up_bytes = off;
     const size_t res_bytes = std::max<size_t>(1, size_t(total_out) * 3 * sizeof(double));
-    const size_t o_part = place(size_t(poff) * sizeof(double)), o_out = place(to_host ? 1 : res_bytes);
+    // results in the block where no pinned memory can be had
+    double* host_out = to_host ? reinterpret_cast<double*>(out.reserve(res_bytes)) : nullptr;
+    const size_t o_part = place(size_t(poff) * sizeof(double)), o_out = place(host_out ? 1 : res_bytes);
     RB_TRY(batch_alloc(arena, &d_block, off, st));
     d_fu = reinterpret_cast<FusedUnit*>(d_block + o_fu);
     d_fg = reinterpret_cast<FusedGroup*>(d_block + o_fg);
@@ -711,11 +713,7 @@ int FusedBatch::build(const std::vector<const FusedHostReq*>& reqs, int mode_, i
     d_counter = reinterpret_cast<int*>(d_block + o_cnt);
     counter_dirty = false;
     d_partial = reinterpret_cast<double*>(d_block + o_part);
-    d_price = reinterpret_cast<double*>(to_host ? reinterpret_cast<char*>(out.reserve(res_bytes)) : d_block + o_out);
-    if (!d_price) {
-        err = "cannot allocate pinned host memory";
-        return ST_ERR_NOMEM;
-    }
+    d_price = host_out ? host_out : reinterpret_cast<double*>(d_block + o_out);
     d_iv = d_price + total_out;
     d_stat = d_price + 2 * size_t(total_out);
     for (FusedReq& r : R) {
@@ -810,11 +808,13 @@ int FusedBatch::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_
     return ST_OK;
 }
 
-void FusedBatch::fetch(int q, double* price, double* iv, double* stat) const {
+hipError_t FusedBatch::fetch(int q, double* price, double* iv, double* stat) const {
     const long a = out_off[q], b = out_off[q + 1];
-    if (price) std::copy(d_price + a, d_price + b, price);
-    if (iv) std::copy(d_iv + a, d_iv + b, iv);
-    if (stat) std::copy(d_stat + a, d_stat + b, stat);
+    const bool pinned = out.data() != nullptr;
+    hipError_t e = fetch_results(price, d_price + a, size_t(b - a), pinned);
+    if (!e) e = fetch_results(iv, d_iv + a, size_t(b - a), pinned);
+    if (!e) e = fetch_results(stat, d_stat + a, size_t(b - a), pinned);
+    return e;
 }
 
 int FusedBatch::results(int q, double* price, double* iv, double* stat, hipStream_t st,
@@ -971,14 +971,17 @@ int FftFused::build(const Request& req, const Layout& lay, int device, hipStream
     const size_t o_tw = place(sz.tw), o_tw64 = place(sz.tw64), o_gamma = place(sz.gamma), o_ptab = place(sz.ptab),
                  o_ints = place(sz.ints), o_part = place(sz.partial);
     const size_t res_bytes = size_t(total_out) * 3 * sizeof(double);
-    const size_t o_out = place(to_host ? 1 : res_bytes);
+    // results in the block where no pinned memory can be had, and large tables from pageable memory
+    double* host_out = to_host ? reinterpret_cast<double*>(out.reserve(res_bytes)) : nullptr;
+    const size_t o_out = place(host_out ? 1 : res_bytes);
     RB_TRY(alloc_async(&d_block, off, st));
-    unsigned char* h = up.reserve(up_bytes);
-    d_price = reinterpret_cast<double*>(to_host ? reinterpret_cast<char*>(out.reserve(res_bytes)) : d_block + o_out);
-    if (!h || !d_price) {
-        err = "cannot allocate pinned host memory";
-        return ST_ERR_NOMEM;
+    unsigned char* h = up_bytes <= PINNED_TABLES ? up.reserve(up_bytes) : nullptr;
+    std::vector<unsigned char> pageable;
+    if (!h) {
+        pageable.resize(up_bytes);
+        h = pageable.data();
     }
+    d_price = host_out ? host_out : reinterpret_cast<double*>(d_block + o_out);
     d_iv = d_price + total_out;
     d_stat = d_iv + total_out;
     d_ivopts = reinterpret_cast<Option*>(d_block + o_ivo);
@@ -996,6 +999,7 @@ int FftFused::build(const Request& req, const Layout& lay, int device, hipStream
     pack(o_opt, opts);
     pack(o_gh, gh);
     RB_TRY(hipMemcpyAsync(d_block, h, up_bytes, hipMemcpyHostToDevice, st));
+    if (!pageable.empty()) RB_TRY(hipStreamSynchronize(st));
     FftFusedArgs& a = args;
     a = FftFusedArgs{};
     a.key = philox_key(req.seed.data(), int(req.seed.size()));
@@ -1044,10 +1048,12 @@ int FftFused::launch(hipStream_t st, std::string& err, Plan* timing, hipEvent_t 
     return ST_OK;
 }
 
-void FftFused::fetch(double* price, double* iv, double* stat) const {
-    if (price) std::copy_n(d_price, total_out, price);
-    if (iv) std::copy_n(d_iv, total_out, iv);
-    if (stat) std::copy_n(d_stat, total_out, stat);
+hipError_t FftFused::fetch(double* price, double* iv, double* stat) const {
+    const bool pinned = out.data() != nullptr;
+    hipError_t e = fetch_results(price, d_price, total_out, pinned);
+    if (!e) e = fetch_results(iv, d_iv, total_out, pinned);
+    if (!e) e = fetch_results(stat, d_stat, total_out, pinned);
+    return e;
 }
 
 int autotune_fused(const Request& shape, const std::vector<int>& Ns, int mode, int device,

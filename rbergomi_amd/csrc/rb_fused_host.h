@@ -71,7 +71,7 @@ struct FftFused {
     int launch(hipStream_t st, std::string& err, Plan* timing = nullptr, hipEvent_t kbeg = nullptr,
                hipEvent_t kend = nullptr);
     // the results of the last launch (to_host), after the caller has waited for it
-    void fetch(double* price, double* iv, double* stat) const;
+    hipError_t fetch(double* price, double* iv, double* stat) const;
 };
 
 // Tile shape (path blocks per tile) per (padded N, operand mode, plain MC): an autotuned entry,
@@ -170,7 +170,7 @@ struct FusedBatch {
     int launch(hipStream_t st, std::string& err, Plan* timing = nullptr, hipEvent_t kbeg = nullptr,
                hipEvent_t kend = nullptr);
     // the results of request q from the last launch (to_host), after the caller has waited for it
-    void fetch(int q, double* price, double* iv, double* stat) const;
+    hipError_t fetch(int q, double* price, double* iv, double* stat) const;
     // enqueue the copies of request q's results (not to_host; the caller synchronizes the stream)
     int results(int q, double* price, double* iv, double* stat, hipStream_t st, std::string& err);
 };

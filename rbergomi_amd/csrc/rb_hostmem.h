@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <algorithm>
+
 namespace rb {
 
 // A pinned, coherent host block of at least the bytes asked for, from the pool (blocks are powers of two from
@@ -28,6 +30,20 @@ class Pinned {
     unsigned char* p_ = nullptr;
     size_t bytes_ = 0;
 };
+
+// Tables of more bytes than this go to the device from the pageable memory they were made in, which the
+// caller waits for: pinned memory is held for a plan's life and rounded up to a power of two (the exact sampler's
+// factors are 134 MB for every H at N = 2048).
+constexpr size_t PINNED_TABLES = size_t(4) << 20;
+
+// n results a kernel wrote, in a pinned block or, where none could be had, in device memory; the caller has
+// waited for the kernel
+inline hipError_t fetch_results(double* to, const double* from, size_t n, bool pinned) {
+    if (!to || n == 0) return hipSuccess;
+    if (!pinned) return hipMemcpy(to, from, n * sizeof(double), hipMemcpyDeviceToHost);
+    std::copy_n(from, n, to);
+    return hipSuccess;
+}
 
 // A non-blocking stream of the current device; up to 32 idle ones are kept
 hipError_t stream_get(hipStream_t* st);

@@ -208,16 +208,17 @@ bool rb_server::reap(std::unique_lock<std::mutex>& lk) {
         }
         for (size_t i = 0; i < F.jobs.size(); ++i) {
             Job& j = *F.jobs[i];
-            if (q == hipSuccess) {
-                if (F.batch) F.batch->fetch(int(i), j.price, j.iv, j.stat);
-                else F.fft->fetch(j.price, j.iv, j.stat);
+            const hipError_t got = q != hipSuccess ? q
+                                   : F.batch       ? F.batch->fetch(int(i), j.price, j.iv, j.stat)
+                                                   : F.fft->fetch(j.price, j.iv, j.stat);
+            if (got == hipSuccess) {
                 j.status = ST_OK;
                 latencies.push_back(std::chrono::duration<double, std::milli>(now - j.t_submit).count());
                 path_steps += double(j.req.M) * j.req.N;
                 conv_flops += j.conv_flops;
             } else {
                 j.status = ST_ERR_DEVICE;
-                j.err = std::string("batch execution failed on the device: ") + hipGetErrorString(q);
+                j.err = std::string("batch execution failed on the device: ") + hipGetErrorString(got);
             }
             j.t_done = now;
             j.done = true;
@@ -463,11 +464,11 @@ int rb_batch::run(std::string& err) {
     for (size_t r = 0; r < runs.size(); ++r)
         for (int k = runs[r].first; k < runs[r].second; ++k) {
             const Job& j = *jobs[short_idx[k]];
-            fused[r]->fetch(k - runs[r].first, j.price, j.iv, j.stat);
+            RB_TRY_SRV(fused[r]->fetch(k - runs[r].first, j.price, j.iv, j.stat));
         }
     for (size_t l = 0; l < long_idx.size(); ++l) {
         const Job& j = *jobs[long_idx[l]];
-        longs[l]->fetch(j.price, j.iv, j.stat);
+        RB_TRY_SRV(longs[l]->fetch(j.price, j.iv, j.stat));
     }
     return ST_OK;
 }

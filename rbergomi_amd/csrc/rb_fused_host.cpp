@@ -216,7 +216,7 @@ void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride
 }
 
 int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHostReq& out,
-                       std::string& err, int pb) {
+                       std::string& err, int pb, size_t bytes) {
     const int N = req.N;
     const int Np = (N + 31) / 32 * 32;
     if (Np > 1024) {
@@ -346,28 +346,33 @@ int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHos
     // 0.43, 2048 items 0.46; N = 365, M = 3e5, plain MC, BF16: 293 items 0.72, 938 items 0.49), but
     // beyond 256 items no less than 2^14 path steps each (a call of N = 64, M = 2^16: 256 items 0.108 ms, 512
     // items 0.118).  The item size depends on the request only, so its sums are added in the same order
-    // alone and in any batch.
-    const long steps = long(N) * a.TP;
-    const long least = std::min((a.ntiles + 255) / 256, ((1L << 14) + steps - 1) / steps);
-    a.tiles_per_item = int(std::max<long>(1, std::min<long>(1024 / a.TP, std::max((a.ntiles + 1023) / 1024, least))));
-    a.nitems = (a.ntiles + a.tiles_per_item - 1) / a.tiles_per_item;
-    a.items_big = a.nitems;
-    a.tiles_small = a.tiles_per_item;
-    // a request of 4096 or more items is in practice a launch of its own: its last eighth of
-    // tiles goes in items of an eighth of the size, handed out last (cheapest first in the
-    // batch's order), so the workgroups finish together rather than one large item apart
-    // (N = 512, M = 2^22, Romano-Touzi: 7.05 -> 6.70 ms with every item of 256 paths; plain
-    // Monte Carlo, with no data-dependent branch, was even without it)
-    if (a.nitems >= 4096 && a.tiles_per_item >= 8) {
-        a.tiles_small = a.tiles_per_item / 8;
-        a.items_big = (a.ntiles - a.ntiles / 8) / a.tiles_per_item;
-        const long rest = a.ntiles - a.items_big * a.tiles_per_item;
-        a.nitems = a.items_big + (rest + a.tiles_small - 1) / a.tiles_small;
-    }
+    // alone and in any batch; only where the partial sums of so many items (16 bytes per option and
+    // item) do not fit the memory there is, 256 items have to do.
+    auto items = [&](long most) {
+        const long steps = long(N) * a.TP;
+        const long least = std::min((a.ntiles + 255) / 256, ((1L << 14) + steps - 1) / steps);
+        a.tiles_per_item = int(std::max<long>(1, std::min<long>(1024 / a.TP, std::max((a.ntiles + most - 1) / most, least))));
+        a.nitems = (a.ntiles + a.tiles_per_item - 1) / a.tiles_per_item;
+        a.items_big = a.nitems;
+        a.tiles_small = a.tiles_per_item;
+        // a request of 4096 or more items is in practice a launch of its own: its last eighth of
+        // tiles goes in items of an eighth of the size, handed out last (cheapest first in the
+        // batch's order), so the workgroups finish together rather than one large item apart
+        // (N = 512, M = 2^22, Romano-Touzi: 7.05 -> 6.70 ms with every item of 256 paths; plain
+        // Monte Carlo, with no data-dependent branch, was even without it)
+        if (a.nitems >= 4096 && a.tiles_per_item >= 8) {
+            a.tiles_small = a.tiles_per_item / 8;
+            a.items_big = (a.ntiles - a.ntiles / 8) / a.tiles_per_item;
+            const long rest = a.ntiles - a.items_big * a.tiles_per_item;
+            a.nitems = a.items_big + (rest + a.tiles_small - 1) / a.tiles_small;
+        }
+    };
     a.key = philox_key(req.seed.data(), int(req.seed.size()));
     a.gchunk = std::min(gmax, FUSED_GREG);
     out.gmax = gmax;
     out.ivopts = lay.options;
+    items(1024);
+    if (FusedBatch::footprint({&out}) > bytes) items(256);
     // cost of one item (relative): RNG + integrals ~ N * groups, GEMM ~ N^2 / 64, payoffs ~ options
     out.item_cost = double(a.tiles_per_item * a.TP) *
                     (double(N) * (2.0 + 2.0 * a.mc + gmax) + double(Np) * Np / 64.0 * nu + 4.0 * a.out_size);

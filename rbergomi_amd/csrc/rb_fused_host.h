@@ -32,9 +32,10 @@ struct FusedHostReq {
     std::vector<Option> ivopts;  // per output I: K, T for the implied vols
 };
 
-// pb: path blocks of 32 per tile (1, 2 or 4); 0 takes fused_pb_choice
+// pb: path blocks of 32 per tile (1, 2 or 4); 0 takes fused_pb_choice.  bytes: device memory the request's
+// owner can give it (its footprint may still need more)
 int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHostReq& out,
-                       std::string& err, int pb = 0);
+                       std::string& err, int pb = 0, size_t bytes = SIZE_MAX);
 
 // Units, groups, payoff groups, options and P_j tables (Np entries per unit) of a request
 void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride, int pshift, FusedHostReq& out,

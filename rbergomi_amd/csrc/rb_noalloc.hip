@@ -77,9 +77,9 @@ extern "C" int rb_price_noalloc(double xi, const double* H, const double* eta, c
     if (N > 1024) return fail(RB_ERR_LIMIT, "rb_price_noalloc covers N <= 1024 (the fused Toeplitz-GEMM kernel)");
     const Layout lay = make_layout(r);
     FusedHostReq fh;
-    rc = plan_fused_request(r, lay, mode, fh, err);
-    if (rc) return fail(rc, err);
     // every carved buffer is rounded up to 256 bytes: at most 19 buffers
+    rc = plan_fused_request(r, lay, mode, fh, err, 0, NOALLOC_SCRATCH_BYTES - 19 * 256);
+    if (rc) return fail(rc, err);
     const size_t need = FusedBatch::footprint({&fh}) + 19 * 256;
     if (need > NOALLOC_SCRATCH_BYTES)
         return fail(RB_ERR_LIMIT, "request needs about " + std::to_string(need >> 20) + " MiB of device scratch, above the " +

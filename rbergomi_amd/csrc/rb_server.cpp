@@ -96,7 +96,8 @@ int request_of(const rb_request* q, int precision, int method, int comp, Request
     return validate(r, err);
 }
 
-int plan_job(const rb_request* q, int precision, int method, int comp, Job& j, std::string& err) {
+// bytes: the device memory a job may take at most
+int plan_job(const rb_request* q, int precision, int method, int comp, size_t bytes, Job& j, std::string& err) {
     if (!q->price || !q->stat) {
         err = "null output arrays";
         return ST_ERR_ARG;
@@ -118,7 +119,7 @@ int plan_job(const rb_request* q, int precision, int method, int comp, Job& j, s
         j.long_path = true;
         return FftFused::plan(r, j.lay, lds_block, j.footprint, err);
     }
-    rc = plan_fused_request(r, j.lay, fused_mode_of(precision), j.fh, err);
+    rc = plan_fused_request(r, j.lay, fused_mode_of(precision), j.fh, err, 0, bytes);
     if (rc) return rc;
     // alone it must fit one workgroup's LDS; batches are closed before a request that would push
     // their combined LDS over the limit
@@ -378,7 +379,7 @@ struct rb_batch {
         out.clear();
         for (int i = 0; i < n; ++i) {
             out.emplace_back(new Job());
-            const int rc = plan_job(&reqs[i], cfg.precision, cfg.method, cfg.compensator, *out.back(), err);
+            const int rc = plan_job(&reqs[i], cfg.precision, cfg.method, cfg.compensator, SIZE_MAX, *out.back(), err);
             if (rc) {
                 err = "request " + std::to_string(i) + ": " + err;
                 return rc;
@@ -693,7 +694,7 @@ int rb_server_submit(rb_server* s, const rb_request* req, long* ticket) {
     std::unique_ptr<Job> j(new Job());
     j->t_submit = Clock::now();
     std::string err;
-    const int rc = plan_job(req, s->cfg.precision, s->method, s->comp, *j, err);
+    const int rc = plan_job(req, s->cfg.precision, s->method, s->comp, size_t(s->cfg.max_device_bytes), *j, err);
     if (rc) {
         set_last_error(err);
         return rc;

@@ -37,3 +37,34 @@ print("ok")
 
 def test_every_path_is_launched_within_the_grid(lib):
     assert recording.run(lib, CODE).strip().endswith("ok")
+
+
+# requests whose partial sums, 16 bytes per option and work item, fill a bounded memory
+BOUNDED = """
+from rbergomi_amd.serving import Request, Server
+opts = np.linspace(0.05, 1.0, 5), np.linspace(0.8, 1.2, 100)
+T, K = np.repeat(opts[0], 100), np.tile(opts[1], 5)
+H, eta, rho = np.linspace(0.05, 0.4, 10), np.full(10, 1.9), np.full(10, -0.7)
+# 5000 options: 20 MB of sums in 256 items, 80 MB in 1024, of 64 MiB
+rb.price_noalloc(0.04, H, eta, rho, T, K, 64, 1 << 18, [1])
+# the same request in a server of 32 MiB
+s = Server(max_device_bytes=32 << 20)
+s.wait(s.submit(Request(0.04, H, eta, rho, T, K, 64, 1 << 18, [1])))
+for M in (1 << 30, 1 << 24):  # 4096 items and more
+    try:
+        rb.price_noalloc(0.04, H, eta, rho, T, K, 64, M, [1])
+        assert False
+    except rb.RbError as e:
+        assert e.code == 5
+    try:
+        s.submit(Request(0.04, H, eta, rho, T, K, 64, M, [1]))
+        assert False
+    except rb.RbError as e:
+        assert e.code == 5
+s.close()
+print("ok")
+"""
+
+
+def test_partial_sums_fit_bounded_memory(lib):
+    assert recording.run(lib, BOUNDED).strip().endswith("ok")

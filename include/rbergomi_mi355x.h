@@ -184,7 +184,8 @@ int rb_plan_create_rows(const double* xi, const double* H, const double* eta, co
  * (X + alpha Y)/2 on (W1, W1perp) and on (-W1, -W1perp), with q_max (the reference's Qmax, 10000)
  * in place of Q where Q <= Iv; price = mean - alpha E[Y].  stat is the standard error of the
  * pair-averaged payoff.  alpha, Q (per row) and exceptions (Q <= Iv evaluations per row) may be
- * NULL.  Requires m_control <= the paths of one chunk (about 6 GB of staged buffers). */
+ * NULL.  Requires m_control <= the paths of which 6 GB hold the Gaussians, Volterra processes and
+ * integrals. */
 int rb_price_rows_turbo(const double* xi, const double* H, const double* eta, const double* rho,
                         const double* T, const double* K, int rows, int N, long M,
                         const uint64_t* seed, int seed_size, long m_control, double q_max,

@@ -495,10 +495,13 @@ int Plan::init(const Request& r, hipStream_t st, bool quadrature, std::string& e
     const long Mr = (r.M + pblk - 1) / pblk * pblk;
     chunk = std::min(ch, Mr);
     if (r.turbo) {
-        // the pilot paths are priced as one chunk (two-pass covariances over all of them)
+        // the pilot paths are priced as one chunk (two-pass covariances over all of them), of which the interface
+        // allows as many as 6 GB hold with their Gaussians and Volterra processes beside the integrals
         const long mc = ((r.m_control + 255) / 256) * 256;
-        if (mc > ch) {
-            err = "m_control above the paths one chunk holds (" + std::to_string(ch) + ")";
+        const long fit = long(6.0e9 / (8.0 * N * (nstreams + nunits) + 32.0 * ngroups)) / 256 * 256;
+        const long most = std::min(ch, std::max(256L, fit));
+        if (mc > most) {
+            err = "m_control above the paths one chunk holds (" + std::to_string(most) + ")";
             return ST_ERR_LIMIT;
         }
         chunk = std::max(chunk, mc);

@@ -28,7 +28,7 @@ for method in (rb.METHOD_RT, rb.METHOD_MC):
             assert at == M, (N, M, at)
 # the mirrored paths of the turbo-charged estimator, with its pilot paths in a launch of their own
 for N in (200, 4096):
-    M, pilot = 300000000, 1000000
+    M, pilot = 300000000, 50000
     rb.price_rows_turbo([0.04], [0.1], [1.9], [-0.7], [1.0], [1.0], N, M, [1], m_control=pilot)
     assert sum(f["np"] for _, f in launches("k_path64") if "np" in f) == M + pilot
 print("ok")
@@ -68,3 +68,22 @@ print("ok")
 
 def test_partial_sums_fit_bounded_memory(lib):
     assert recording.run(lib, BOUNDED).strip().endswith("ok")
+
+
+PILOTS = """
+row = [0.04], [0.1], [1.9], [-0.7], [1.0], [1.0]
+for N in (64, 256, 1024, 4096):
+    fit = int(6e9 / (24 * N + 32)) // 256 * 256
+    rb.price_rows_turbo(*row, N, 1000, [1], m_control=fit)
+    try:
+        rb.price_rows_turbo(*row, N, 1000, [1], m_control=fit + 1)
+        assert False
+    except rb.RbError as e:
+        assert e.code == 5
+print("ok")
+"""
+
+
+def test_pilot_paths_of_the_turbo_estimator_are_limited(lib):
+    """rb_price_rows_turbo's m_control: 6 GB of two streams, one process and two pairs of integrals a path."""
+    assert recording.run(lib, PILOTS).strip().endswith("ok")

@@ -848,20 +848,19 @@ void FftFused::release() {
     d_ivopts = nullptr;
 }
 
-// The request sizes the long-path kernel takes: a pair's signal with its pad, four waves' sums of
-// eight groups, the records of the unit with the most payoff groups and the sums of every option in
-// one workgroup's LDS.  (Its present form keeps the last two elsewhere; what it refuses is part of
-// the interface.)
-static int fft_request_fits(const FusedHostReq& tabs, int N, int nopt, size_t lds_limit, std::string& err) {
+// The request sizes of the long-path kernel, a limit of the interface: 16 bytes an option and 64 a (group, rho)
+// of the H with the most, beside 8.25 a point of the transform, in 160 KiB less 1.5 (from the time when one
+// workgroup's LDS held them; nothing in the present kernel needs it).
+static int fft_request_fits(const FusedHostReq& tabs, int N, int nopt, std::string& err) {
     int log2L = 10;
     while ((1 << log2L) < 2 * N - 1) ++log2L;
-    const size_t L = size_t(1) << log2L;
+    const long L = 1L << log2L, room = 160 * 1024 - 1536 - 8 * (L + L / 32);
     int pgu = 1;
     for (const FusedUnit& U : tabs.fu) pgu = std::max(pgu, U.pg_end - U.pg_begin);
-    const size_t need = (L + L / 32) * sizeof(float2) + 4 * 8 * 2 * 3 * sizeof(double) + size_t(2) * pgu * sizeof(PathPG) +
-                        size_t(nopt) * 2 * sizeof(double);
-    if (need <= lds_limit) return ST_OK;
-    err = "long-path kernel needs " + std::to_string(need) + " bytes of LDS (N or the option count too large)";
+    if (64L * pgu + 16L * nopt <= room) return ST_OK;
+    err = "too many options for a request of N = " + std::to_string(N) + " on the long-path kernel: 16 for each of its " +
+          std::to_string(nopt) + " options and 64 for each of the " + std::to_string(pgu) +
+          " (maturity, eta, rho) of its largest H may come to " + std::to_string(room);
     return ST_ERR_LIMIT;
 }
 
@@ -890,7 +889,7 @@ struct FftSizes {
     size_t total() const { return ptab + ghat + tw + gamma + tw64 + ints + partial; }
 };
 
-int FftFused::plan(const Request& req, const Layout& lay, size_t lds_limit, size_t& footprint, std::string& err) {
+int FftFused::plan(const Request& req, const Layout& lay, size_t& footprint, std::string& err) {
     const int N = req.N;
     if (N <= 1024 || ((N + 3) / 4 + 255) / 256 > 8) {
         err = "the long-path kernel covers 1024 < N <= 8192";
@@ -899,7 +898,7 @@ int FftFused::plan(const Request& req, const Layout& lay, size_t lds_limit, size
     FusedHostReq tabs;
     int pgmax = 1, gmax = 1;
     fused_tables(req, lay, 0, 0, 0, tabs, pgmax, gmax);
-    const int rc = fft_request_fits(tabs, N, int(lay.options.size()), lds_limit, err);
+    const int rc = fft_request_fits(tabs, N, int(lay.options.size()), err);
     if (rc) return rc;
     footprint = FftSizes(req, int(lay.units.size()), int(tabs.fg.size()), int(lay.options.size())).total() +
                 lay.options.size() * (sizeof(Option) + sizeof(PayOpt64) + sizeof(PayJob64)) +
@@ -925,7 +924,7 @@ int FftFused::build(const Request& req, const Layout& lay, int device, hipStream
     RB_TRY(device_props(device, prop));
     keep_pool_cached(device);
     cus = prop.multiProcessorCount;
-    const int rc = fft_request_fits(tabs, N, total_out, prop.sharedMemPerBlock, err);
+    const int rc = fft_request_fits(tabs, N, total_out, err);
     if (rc) return rc;
     const FftSizes sz(req, nunits, int(tabs.fg.size()), total_out);
     ppt = sz.ppt;

@@ -117,7 +117,7 @@ int plan_job(const rb_request* q, int precision, int method, int comp, size_t by
     if (r.N > 1024) {
         // long paths: one request per launch of the FFT kernel
         j.long_path = true;
-        return FftFused::plan(r, j.lay, lds_block, j.footprint, err);
+        return FftFused::plan(r, j.lay, j.footprint, err);
     }
     rc = plan_fused_request(r, j.lay, fused_mode_of(precision), j.fh, err, 0, bytes);
     if (rc) return rc;

@@ -87,3 +87,26 @@ print("ok")
 def test_pilot_paths_of_the_turbo_estimator_are_limited(lib):
     """rb_price_rows_turbo's m_control: 6 GB of two streams, one process and two pairs of integrals a path."""
     assert recording.run(lib, PILOTS).strip().endswith("ok")
+
+
+OPTIONS = """
+from rbergomi_amd.serving import Request, Server
+s = Server()
+for N, L in ((1025, 4096), (4096, 8192), (8192, 16384)):
+    most = (160 * 1024 - 1536 - 8 * (L + L // 32) - 64) // 16
+    for n in (most, most + 1):
+        one = 0.04, [0.1], [1.9], [-0.7], np.full(n, 1.0), np.linspace(0.5, 1.5, n), N, 1000, [1]
+        for call in (lambda: rb.price_v2(*one, precision=rb.PREC_SPLIT_FP16), lambda: s.wait(s.submit(Request(*one)))):
+            try:
+                call()
+                assert n == most
+            except rb.RbError as e:
+                assert n == most + 1 and e.code == 5 and "LDS" not in str(e) and str(n) in str(e), e
+s.close()
+print("ok")
+"""
+
+
+def test_options_of_a_long_path_request_are_limited(lib):
+    """A limit of the interface, and the message says so."""
+    assert recording.run(lib, OPTIONS).strip().endswith("ok")

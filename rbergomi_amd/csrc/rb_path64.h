@@ -34,6 +34,18 @@ constexpr double P64_PAD = 1e40, P64_AL_MIN = 1e-30, P64_AL_MAX = 1e250;
 
 enum Path64Source { P64_PHILOX = 0, P64_MEMORY = 1 };
 
+// A caller's Gaussians may be anything.  What infinities and NaN do stays with their path and their steps, as
+// it does in the direct sum: W1perp of the last step, which the model does not use, has no effect
+// (`used`: the step has a successor), and an infinite exponent gives 0 or infinity, where exp2_32 would make NaN of it.
+__host__ __device__ __forceinline__ double path64_caller_x(double x, bool used) {
+    constexpr double BIG = 1e200;
+    x = x > BIG ? BIG : x < -BIG ? -BIG : x;  // NaN stays
+    return used ? x : 0.0;
+}
+// W1 beyond this (no Gaussian is) is not put through a transform, which would spread it over its path's other
+// steps and the pair's other path
+constexpr double P64_WILD = 64.0;
+
 struct Path64Args {
     PhiloxKey key;
     long p0;               // Philox counter of the launch's path 0

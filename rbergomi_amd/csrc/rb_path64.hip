@@ -269,6 +269,7 @@ __global__ void __launch_bounds__(NT, 4) k_path64(Path64Args A) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 x[r] = fma(b, z[r], acc0[r] + acc1[r]);
+                if constexpr (SRC == P64_MEMORY) x[r] = path64_caller_x(x[r], 4 * q + r < N - 1);
                 w[r] = W[(4 * q + 1 + r) * 16];
                 pj[r] = P[4 * q + r];
             }

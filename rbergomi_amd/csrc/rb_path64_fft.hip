@@ -230,6 +230,15 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
         }
     if (t == 0) E[2 * C::NW] = E[C::EDGES + 2 * C::NW] = make_double2(0.0, 0.0);
     sync();
+    bool direct = false;  // by the direct sum: a caller's W1 beyond P64_WILD in the workgroup
+    if constexpr (SRC == P64_MEMORY) {
+        bool wild = false;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wild |= !(fabs(w1[j][r].x) <= P64_WILD && fabs(w1[j][r].y) <= P64_WILD);
+        direct = __syncthreads_or(wild);
+    }
     double2 n1[2], n2[MC ? 2 : 1];
     auto next = [&](const double2(&w)[2][4], int at, double2* n) {
 #pragma unroll
@@ -259,7 +268,21 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
         asm volatile("" : "+s"(hide));
         const double2* tw = A.tw + hide;
         const Fft64Run<LOG2L, Sync> fft{z, tw, t, sync};
-        {
+        if (SRC == P64_MEMORY && direct) {
+            sync();
+            const double* gam = A.gamma + long(job.unit) * A.tlen;
+#pragma unroll 1
+            for (int e = 0; e < 8; ++e) {
+                const int i = 4 * (t + TP * (e >> 2)) + (e & 3);
+                double2 y = make_double2(0.0, 0.0);
+                for (int k = 0; k <= i && k < N; ++k) {
+                    const double g = gam[k];
+                    const double2 v = z[fpad64(i - k)];
+                    y = make_double2(fma(g, v.x, y.x), fma(g, v.y, y.y));
+                }
+                z[fpad64(L / 2 + i)] = y;  // the thread's own: nothing else is read there
+            }
+        } else {
             double2 x[16];
             fft.forward(x);
             const double2* gh = A.ghat + long(job.unit) * L + t;
@@ -278,8 +301,12 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
             const int q = t + TP * j;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const double2 y = z[fpad64(4 * q + r)];
+                const double2 y = z[fpad64((SRC == P64_MEMORY && direct ? L / 2 : 0) + 4 * q + r)];
                 x[j][r] = make_double2(fma(b, wp[j][r].x, y.x), fma(b, wp[j][r].y, y.y));
+                if constexpr (SRC == P64_MEMORY) {
+                    x[j][r].x = path64_caller_x(x[j][r].x, 4 * q + r < N - 1);
+                    x[j][r].y = path64_caller_x(x[j][r].y, 4 * q + r < N - 1);
+                }
                 pj[j][r] = 4 * q + r < A.tlen ? A.ptab[long(job.unit) * A.tlen + 4 * q + r] : P64_PAD;
             }
         }

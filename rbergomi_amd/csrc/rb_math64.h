@@ -243,6 +243,20 @@ __host__ __device__ __forceinline__ void mills_pair(double x, double y, double& 
 struct PathRt64 {
     double lnS, S, sig, isig;
 };
+__host__ __device__ __forceinline__ PathRt64 path_rt64(double Iv, double Is, double rho) {
+    PathRt64 q;
+    q.sig = sqrt((1.0 - rho * rho) * Iv);
+    q.isig = 1.0 / q.sig;
+    q.lnS = -0.5 * rho * rho * Iv + rho * Is;
+    q.S = exp(q.lnS);
+    // S' beyond the largest double (a caller's Gaussians): the payoff is infinite, which rt_payoff64 gives for
+    // d1 = -1, d2 = 1 and makes NaN of with d1 at its end (infinity times a phi of 0)
+    if (q.S > 1.7976931348623157e308) {
+        q.lnS = q.isig = 0.0;
+        q.sig = -2.0;
+    }
+    return q;
+}
 
 // Romano-Touzi payoff C_BS(S', K, 1, sigma) (rBergLib/rBergomiMT.cpp:383-388, BlackScholes.cpp:22-26)
 // = S' Phi(d1) - K Phi(d2).  With K phi(d2) = S' phi(d1) both tails come from one exponential and

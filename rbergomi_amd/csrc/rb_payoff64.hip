@@ -33,10 +33,7 @@ struct PayRt64 {  // FP64 Romano-Touzi (Iv, Is)
     static constexpr bool TAB = true;
     PathRt64 q;
     __device__ __forceinline__ void set(const double* v, double rho) {
-        q.sig = sqrt((1.0 - rho * rho) * v[0]);
-        q.isig = 1.0 / q.sig;
-        q.lnS = -0.5 * rho * rho * v[0] + rho * v[1];
-        q.S = exp(q.lnS);
+        q = path_rt64(v[0], v[1], rho);
     }
     __device__ __forceinline__ double pay(const double* e2, const PayOpt64& o) const { return rt_payoff64(e2, q, o.K, o.lnK); }
 };

@@ -30,10 +30,12 @@ def test_other_paths_and_unused_steps_are_not_touched(rb, orc, N, method):
     Z[12, 1, k] = -np.inf        # W1perp of one step: that step has no variance
     Z[14, 1, N - 1] = np.nan     # W1perp of the last step is not used
     Z[17, 1, N - 1] = np.inf
+    Z[18, 0, 0] = -1e7           # S' beyond the largest double: an infinite payoff
     fn = orc.payoff_mc_samples if method else orc.payoff_rt_samples
     got = rb.payoff_samples_v2(xi, H, eta, rho, T, K, N, Z, method=method)
     ref = fn(xi, H, eta, rho, T, K, N, Z)
-    lost = [2, 5, 8, 11]
+    assert np.all(ref[18] == np.inf) and np.all(got[18] == np.inf)
+    lost = [2, 5, 8, 11, 18]
     kept = [p for p in range(len(Z)) if p not in lost]
     assert np.all(np.isfinite(ref[kept]))
     assert np.max(np.abs(got[kept] - ref[kept])) < 1e-12

@@ -99,16 +99,25 @@ static constexpr double LOG_TAB[128] = {
 constexpr int EXP2_N = 32, LOG_N = 64;
 constexpr double EXP2_SCALE = 46.166241308446828384;  // 32 log2(e): exp(x) = 2^(x EXP2_SCALE / 32)
 
+// A whole number as an integer, the nearest end of the range beyond it and 0 for NaN.  C++ leaves int(n)
+// undefined there, and every step past a path's last one comes with an exponent of -1e10 and less; the instruction
+// is the one int(n) would be, by name (-fno-strict-float-cast-overflow puts six more around it).
+__host__ __device__ __forceinline__ int whole_i32(double n) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    int k;
+    asm("v_cvt_i32_f64 %0, %1" : "=v"(k) : "v"(n));
+    return k;
+#else
+    return n >= 2147483647.0 ? 2147483647 : n > -2147483648.0 ? int(n) : n <= -2147483648.0 ? -2147483647 - 1 : 0;
+#endif
+}
+
 // 2^(y / 32): y = n + f with n whole and |f| <= 1/2, 2^(n/32) from the table and an exponent
 // shift, 2^(f/32) = 1 + f q(f) with q of degree 4 (relative error 9e-17).  y beyond the exponent
-// range gives 0 or infinity (the conversion to an integer saturates); NaN stays NaN.
+// range gives 0 or infinity (the conversion to an integer saturates); NaN and infinities give NaN.
 __host__ __device__ __forceinline__ double exp2_32(const double* T, double y) {
     const double n = rint(y), f = y - n;
-#if defined(__HIP_DEVICE_COMPILE__)
-    const int k = int(n);
-#else
-    const int k = n > 1e6 ? 1000000 : n > -1e6 ? int(n) : -1000000;
-#endif
+    const int k = whole_i32(n);
     double q = fma(0x1.5d8789d24d3fep-35, f, 0x1.3b2b276cebac8p-27);
     q = fma(q, f, 0x1.c6b08d70b74e4p-20);
     q = fma(q, f, 0x1.ebfbdff8098e8p-13);

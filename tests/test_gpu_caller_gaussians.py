@@ -32,7 +32,7 @@ def test_other_paths_and_unused_steps_are_not_touched(rb, orc, N, method):
     Z[17, 1, N - 1] = np.inf
     Z[18, 0, 0] = -1e7           # S' beyond the largest double: an infinite payoff
     fn = orc.payoff_mc_samples if method else orc.payoff_rt_samples
-    got = rb.payoff_samples_v2(xi, H, eta, rho, T, K, N, Z, method=method)
+    got, _, _ = rb.payoff_samples_v2(xi, H, eta, rho, T, K, N, Z, method=method)
     ref = fn(xi, H, eta, rho, T, K, N, Z)
     assert np.all(ref[18] == np.inf) and np.all(got[18] == np.inf)
     lost = [2, 5, 8, 11, 18]
@@ -42,6 +42,6 @@ def test_other_paths_and_unused_steps_are_not_touched(rb, orc, N, method):
     if method == 0:
         assert not np.any(np.isfinite(got[[2, 5, 11]]))
     # the same values as without the lost paths' (the transform of a clean pair is not the direct sum: 1e-12)
-    calm = rb.payoff_samples_v2(xi, H, eta, rho, T, K, N, clean, method=method)
+    calm, _, _ = rb.payoff_samples_v2(xi, H, eta, rho, T, K, N, clean, method=method)
     same = [p for p in kept if p not in (12, 14, 17)]
     assert np.max(np.abs(got[same] - calm[same])) < 1e-12

@@ -209,9 +209,10 @@ __device__ __forceinline__ void fft_dif_inv_r4_t(float2* z, const float2* __rest
 // ---- convolution of two paths with radix-16 passes, L = 2^10..2^14 (FP32).  The stages run in
 // passes over groups of 16 points held in registers (3-5 LDS passes and barriers per transform
 // instead of 6-7 for radix 4), and the pass either side of the spectral product runs as one.
-// Element i0 + k span of a group sits in slot fpad(i0) + k span + (k span) / 32 for every
-// power-of-two span.  Two orders:
-//  - natural (fft_convolve_r16): forward by decimation in frequency from natural order, inverse
+// Element i0 + k span of a group sits in slot i0 + i0 / 2^PAD + k span + (k span) / 2^PAD for every
+// power-of-two span (PAD 5, as fpad, in the staged kernel, 4 in the long-path kernel).  Two orders:
+//  - natural (the long-path kernel; fft_convolve_r16 is the same passes with the plain table, which only a
+//    host run walks): forward by decimation in frequency from natural order, inverse
 //    by decimation in time back to natural order, the spectrum and G in bit-reversed order
 //    between them.  The top stage (distance L/2) of each transform is left to the caller:
 //    forward while the input is written (its upper half is the zero padding, so the stage gives
@@ -243,6 +244,16 @@ __host__ __device__ __forceinline__ float2 fft_tw(FftPassTable tw, int pos, int 
     } else {
         return tw.tab[fft_pass_off(SB) + ((fft_pass_row(r) + m) << SB) + pos];
     }
+}
+
+// Entry i of that table, plain and by pass, is exp(-2 pi i k / L): its k
+__host__ __device__ __forceinline__ int fft_twiddle_power(int log2L, int i) {
+    const int H2 = 1 << (log2L - 1);
+    if (i < H2) return i;
+    int sb = (log2L - 1) % 4 ? (log2L - 1) % 4 : 4, o = i - H2;
+    for (; o >= 8 << sb; sb += 4) o -= 8 << sb;
+    const int row = o >> sb, r = row < 2 ? row : row < 4 ? 2 : 3;
+    return ((o & ((1 << sb) - 1)) + ((row - fft_pass_row(r)) << sb)) << (log2L - sb - r - 1);
 }
 
 // a w.  Each part is one rounded product and one FMA; which product is rounded first is free, and
@@ -459,6 +470,31 @@ template <int LOG2L, class TW, class GT, class X>
 __host__ __device__ __forceinline__ void fft_convolve_r16(float2* z, TW tw, GT G, const X& x) {
     static_assert(LOG2L >= 10 && LOG2L <= 14, "transform lengths 2^10 .. 2^14");
     fft_nat_fwd<LOG2L, LOG2L - 2>(z, tw, G, x);
+}
+
+// The first pass of the forward transform where its table is ordered by pass: the top stage of a signal whose upper
+// half is zero (z_{i + L/2} = z_i W_L^i) and the four stages under it.  Group pos < 2^(LOG2L - 5) has the points
+// pos + k 2^(LOG2L - 5), k < 16, of the lower half, and as many of the upper; tw: the plain table, then the passes'.
+template <int LOG2L, int PAD>
+__host__ __device__ __forceinline__ void fft_first_load(float2 (&x)[16], const float2* z, int pos) {
+    constexpr int span = 1 << (LOG2L - 5);
+    const float2* p = z + (pos + (pos >> PAD));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = p[k * span + ((k * span) >> PAD)];
+}
+template <int LOG2L>
+__host__ __device__ __forceinline__ void fft_first_upper(float2 (&x)[16], const float2* tw, int pos) {
+    constexpr int span = 1 << (LOG2L - 5);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = fft_mul<FFT_MUL_Y>(x[k], tw[pos + k * span]);
+}
+template <int LOG2L, int PAD>
+__host__ __device__ __forceinline__ void fft_first_store(float2 (&x)[16], float2* z, const float2* tw, int pos, int h) {
+    constexpr int SB = LOG2L - 5, span = 1 << SB, H2 = 1 << (LOG2L - 1);
+    fft_stages_dif<LOG2L, SB, 4, false>(x, FftPassTable{tw + H2}, pos, fft_first<LOG2L, SB, 4>(pos + h * span));
+    float2* o = z + (pos + (pos >> PAD)) + h * (H2 + (H2 >> PAD));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) o[k * span + ((k * span) >> PAD)] = x[k];
 }
 
 // ---- bit-reversed order: forward passes from stage 0 up, the middle one at the top

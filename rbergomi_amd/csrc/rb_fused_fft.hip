@@ -96,15 +96,8 @@ __global__ void k_fft32_tables(const Unit* __restrict__ units, int N, int tlen, 
 __global__ void k_fft32_twiddles(int log2L, float2* __restrict__ tw) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, H2 = 1 << (log2L - 1);
     if (i >= fused_fft_table(log2L)) return;
-    int k = i;
-    if (i >= H2) {
-        int sb = (log2L - 1) % 4 ? (log2L - 1) % 4 : 4, o = i - H2;
-        for (; o >= 8 << sb; sb += 4) o -= 8 << sb;
-        const int row = o >> sb, r = row < 2 ? row : row < 4 ? 2 : 3;
-        k = ((o & ((1 << sb) - 1)) + ((row - fft_pass_row(r)) << sb)) << (log2L - sb - r - 1);
-    }
     double s, c;
-    sincospi(-double(k) / double(H2), &s, &c);
+    sincospi(-double(fft_twiddle_power(log2L, i)) / double(H2), &s, &c);
     tw[i] = make_float2(float(c), float(s));
 }
 
@@ -142,41 +135,25 @@ struct FftPairPass {
     }
 };
 
-// The first pass of the forward transform: the top stage of a signal whose upper half is zero
-// (z_{i + L/2} = z_i W_L^i) and the four stages under it.
+// The first pass of the forward transform by the TP threads of a pair (fft_first_load and what follows)
 template <int LOG2L, int TP, class Sync>
 __device__ __forceinline__ void fft_first_pass(float2* z, const float2* tw, int t, const Sync& sync) {
-    constexpr int SB = LOG2L - 5, span = 1 << SB, H2 = 1 << (LOG2L - 1), PAD = FftPair<LOG2L>::PAD;
-    const FftPassTable tab{tw + H2};
+    constexpr int span = 1 << (LOG2L - 5), PAD = FftPair<LOG2L>::PAD;
     const int pos = t & (span - 1);
-    float2* p = z + FftPair<LOG2L>::slot(pos);
     float2 x[16];
-#pragma unroll
-    for (int k = 0; k < 16; ++k) x[k] = p[k * span + ((k * span) >> PAD)];
-    auto upper = [&] {
-#pragma unroll
-        for (int k = 0; k < 16; ++k) x[k] = fft_mul<FFT_MUL_Y>(x[k], tw[pos + k * span]);
-    };
-    auto run = [&](int h) {
-        fft_stages_dif<LOG2L, SB, 4, false>(x, tab, pos, fft_first<LOG2L, SB, 4>(pos + h * span));
-        float2* o = p + h * (H2 + (H2 >> PAD));
-#pragma unroll
-        for (int k = 0; k < 16; ++k) o[k * span + ((k * span) >> PAD)] = x[k];
-    };
+    fft_first_load<LOG2L, PAD>(x, z, pos);
     if constexpr (TP == 2 * span) {  // half of the threads to each half of the points
         sync();                      // the lower half has been read
-        if (t >= span) upper();
-        run(t >= span ? 1 : 0);
+        if (t >= span) fft_first_upper<LOG2L>(x, tw, pos);
+        fft_first_store<LOG2L, PAD>(x, z, tw, pos, t >= span ? 1 : 0);
     } else {
         static_assert(TP == span, "both halves of a group to a thread");
         float2 y[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) y[k] = x[k];
-        run(0);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) x[k] = y[k];
-        upper();
-        run(1);
+        fft_first_store<LOG2L, PAD>(x, z, tw, pos, 0);
+        fft_first_upper<LOG2L>(y, tw, pos);
+        fft_first_store<LOG2L, PAD>(y, z, tw, pos, 1);
     }
     sync();
 }

@@ -76,8 +76,8 @@ struct Path64Args {
 hipError_t launch_path64_tables(const Unit* units, int nunits, int N, int tlen, double off, double* gamma,
                                 double* ptab, hipStream_t st);
 
-// The matrix-core kernel (N <= 512 by its LDS and registers): groups per job, launch shape, LDS
-constexpr int PATH64_MFMA_MAX_N = 512;
+// The matrix-core kernel (up to where path64_uses_fft may choose it): groups per job, launch shape, LDS
+constexpr int PATH64_MFMA_MAX_N = 384;
 int path64_greg(int groups_of_largest_unit, int signs);
 void path64_shape(Path64Args& a, int cus);
 size_t path64_lds_bytes(const Path64Args& a);

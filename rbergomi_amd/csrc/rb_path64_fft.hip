@@ -396,7 +396,7 @@ int path64_fft_log2(int N) {
 // against 991, five at 380 1012 against 1067.  Beyond N = 384 products lose even where transforms fill their
 // length least (N = 400, plain MC, five groups: 1548 against 1350).
 bool path64_uses_fft(int N, int units, int groups, bool mc) {
-    if (N > 384) return true;
+    if (N > PATH64_MFMA_MAX_N) return true;
     const double u = units, g = groups, r = double(1 << path64_fft_log2(N)) / 2 / N;
     const double fft = r * (mc ? 386 + 262 * u + 83 * g : 228 + 226 * u + 57 * g);
     const double mm = (mc ? 225 : 115) + u * (110 + 1.37 * N) + 60 * g;

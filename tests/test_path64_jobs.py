@@ -62,3 +62,35 @@ def test_prices_match_the_oracle(orc, kernel, threads, perp, units, mats, N, M, 
     if N == 500:  # the same paths as a caller's Gaussians
         _, pr2, st2 = rb.payoff_samples_v2(*args, N, Z, method=method)
         assert np.max(np.abs(pr2 - pr)) < 1e-12 and np.max(np.abs(st2 - st)) < 1e-12
+
+
+# the long-path mixed-precision kernel's loop over units: transforms of 2^10 to 2^14 points (at the FFT precision below
+# N = 1025), threads of a pair 64 to 512
+UNITS = [(500, 9000), (1000, 4300), (1500, 2100), (3000, 1300), (6000, 1300)]
+H3, ETA3, RHO3 = [0.07, 0.21, 0.4], [1.9, 1.1, 0.7], [-0.9, -0.6, -0.3]
+
+
+def test_unit_cases_have_workgroups_of_several_units(tmp_path):
+    lib = recording.build(tmp_path)
+    out = recording.run(lib, """
+for N, M in %r:
+    rb.price_v2(0.04, %r, %r, %r, [1.0], [1.0], N, M, [1], precision=rb.PREC_FP32_FFT)
+    (name, f), = launches("k_fused_fft")
+    print(f["grid_y"] < 3, name, f)
+""" % (UNITS, H3, ETA3, RHO3))
+    assert [x.split()[0] for x in out.splitlines()] == ["True"] * len(UNITS), out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("N,M", UNITS)
+def test_units_of_one_workgroup_price_as_alone(N, M, method):
+    """The paths of a call do not depend on its parameter sets, so every set's prices are the same bits alone."""
+    import rbergomi_amd as rb
+    T, K = np.array([0.4, 1.1]), np.array([0.95, 1.05])
+    kw = dict(precision=rb.PREC_FP32_FFT, method=method)
+    print("units N=%d M=%d method=%d" % (N, M, method), flush=True)
+    price, _, stat = rb.price_v2(0.04, H3, ETA3, RHO3, T, K, N, M, [3, N], **kw)
+    for h in range(3):
+        p, _, s = rb.price_v2(0.04, H3[h:h + 1], ETA3[h:h + 1], RHO3[h:h + 1], T, K, N, M, [3, N], **kw)
+        assert np.array_equal(p, price[2 * h:2 * h + 2]) and np.array_equal(s, stat[2 * h:2 * h + 2])

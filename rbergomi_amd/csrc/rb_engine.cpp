@@ -639,7 +639,7 @@ int Plan::integrals(uint64_t p0, long np, bool from_z, int signs, std::string& e
         a.key = key;
         a.p0 = long(p0);
         a.np = np;
-        a.src = from_z ? P64_MEMORY : P64_PHILOX;
+        a.src = !from_z ? P64_PHILOX : req.gauss >= 1 ? P64_MEMORY : P64_CALLER;
         a.signs = signs;
         a.Z = d_Z;
         a.zstride = long(nstreams) * req.N;

@@ -32,11 +32,14 @@ struct Path64Job {
 // on the steps before (P <= 8192^2)
 constexpr double P64_PAD = 1e40, P64_AL_MIN = 1e-30, P64_AL_MAX = 1e250;
 
-enum Path64Source { P64_PHILOX = 0, P64_MEMORY = 1 };
+// P64_MEMORY: Gaussians a kernel of the package left in Z (Sobol' points); P64_CALLER: a caller's
+enum Path64Source { P64_PHILOX = 0, P64_MEMORY = 1, P64_CALLER = 2 };
 
 // A caller's Gaussians may be anything.  What infinities and NaN do stays with their path and their steps, as
 // it does in the direct sum: W1perp of the last step, which the model does not use, has no effect
 // (`used`: the step has a successor), and an infinite exponent gives 0 or infinity, where exp2_32 would make NaN of it.
+// The guards are compiled for P64_CALLER only: they cost the transform kernel 5 to 27% of its time (N = 256, M =
+// 31250: 58 -> 68 us), which a caller's call, most of it the copy of its Gaussians, does not notice.
 __host__ __device__ __forceinline__ double path64_caller_x(double x, bool used) {
     constexpr double BIG = 1e200;
     x = x > BIG ? BIG : x < -BIG ? -BIG : x;  // NaN stays
@@ -57,7 +60,7 @@ struct Path64Args {
     int greg;              // groups per job at most (path64_greg)
     int mc, signs;         // plain MC; 2: the mirrored path's integrals too (ints2)
     int cache_perp;        // W1perp of the tile kept in LDS for the jobs after the first
-    const double* Z;       // P64_MEMORY: path p at Z + p zstride, blocks of N values
+    const double* Z;       // P64_MEMORY, P64_CALLER: path p at Z + p zstride, blocks of N values
     long zstride;
     const Unit* units;
     const double* gamma;   // [units][tlen]: a, Gamma_1 .. Gamma_{N-1}, 0 ..

@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(NT, 4) k_path64(Path64Args A) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 x[r] = fma(b, z[r], acc0[r] + acc1[r]);
-                if constexpr (SRC == P64_MEMORY) x[r] = path64_caller_x(x[r], 4 * q + r < N - 1);
+                if constexpr (SRC == P64_CALLER) x[r] = path64_caller_x(x[r], 4 * q + r < N - 1);
                 w[r] = W[(4 * q + 1 + r) * 16];
                 pj[r] = P[4 * q + r];
             }
@@ -362,15 +362,22 @@ hipError_t launch_path64(const Path64Args& a, hipStream_t st) {
         hipLaunchKernelGGL(kern, grid, dim3(unsigned(a.threads)), lds, st, a);
         return hipGetLastError();
     };
-    const bool mem = a.src == P64_MEMORY;
     auto pick = [&](auto greg, auto threads) -> hipError_t {
         constexpr int GREG = decltype(greg)::value, NT = decltype(threads)::value;
-        if (a.mc) return mem ? go(&k_path64<P64_MEMORY, true, 1, GREG, NT>) : go(&k_path64<P64_PHILOX, true, 1, GREG, NT>);
-        return mem ? go(&k_path64<P64_MEMORY, false, 1, GREG, NT>) : go(&k_path64<P64_PHILOX, false, 1, GREG, NT>);
+        auto from = [&](auto src) {
+            constexpr int SRC = decltype(src)::value;
+            return a.mc ? go(&k_path64<SRC, true, 1, GREG, NT>) : go(&k_path64<SRC, false, 1, GREG, NT>);
+        };
+        switch (a.src) {
+            case P64_PHILOX: return from(std::integral_constant<int, P64_PHILOX>());
+            case P64_MEMORY: return from(std::integral_constant<int, P64_MEMORY>());
+            case P64_CALLER: return from(std::integral_constant<int, P64_CALLER>());
+            default: return hipErrorInvalidValue;
+        }
     };
     auto sized = [&](auto threads) -> hipError_t {
         if (a.signs == 2) {
-            if (mem || a.mc || a.greg != 2) return hipErrorInvalidValue;
+            if (a.src != P64_PHILOX || a.mc || a.greg != 2) return hipErrorInvalidValue;
             return go(&k_path64<P64_PHILOX, false, 2, 2, decltype(threads)::value>);
         }
         if (a.greg == 2) return pick(std::integral_constant<int, 2>(), threads);

@@ -231,7 +231,7 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
     if (t == 0) E[2 * C::NW] = E[C::EDGES + 2 * C::NW] = make_double2(0.0, 0.0);
     sync();
     bool direct = false;  // by the direct sum: a caller's W1 beyond P64_WILD in the workgroup
-    if constexpr (SRC == P64_MEMORY) {
+    if constexpr (SRC == P64_CALLER) {
         bool wild = false;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -268,7 +268,7 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
         asm volatile("" : "+s"(hide));
         const double2* tw = A.tw + hide;
         const Fft64Run<LOG2L, Sync> fft{z, tw, t, sync};
-        if (SRC == P64_MEMORY && direct) {
+        if (SRC == P64_CALLER && direct) {
             sync();
             const double* gam = A.gamma + long(job.unit) * A.tlen;
 #pragma unroll 1
@@ -301,9 +301,9 @@ __global__ void __launch_bounds__((Path64Fft<LOG2L>::NT), 2) k_path64_fft(Path64
             const int q = t + TP * j;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const double2 y = z[fpad64((SRC == P64_MEMORY && direct ? L / 2 : 0) + 4 * q + r)];
+                const double2 y = z[fpad64((SRC == P64_CALLER && direct ? L / 2 : 0) + 4 * q + r)];
                 x[j][r] = make_double2(fma(b, wp[j][r].x, y.x), fma(b, wp[j][r].y, y.y));
-                if constexpr (SRC == P64_MEMORY) {
+                if constexpr (SRC == P64_CALLER) {
                     x[j][r].x = path64_caller_x(x[j][r].x, 4 * q + r < N - 1);
                     x[j][r].y = path64_caller_x(x[j][r].y, 4 * q + r < N - 1);
                 }
@@ -509,10 +509,18 @@ hipError_t launch_path64_fft(const Path64Args& a, hipStream_t st) {
             hipLaunchKernelGGL(kern, grid, dim3(C::NT), lds, st, a);
             return hipGetLastError();
         };
-        const bool mem = a.src == P64_MEMORY;
-        if (a.signs == 2) return mem || a.mc ? hipErrorInvalidValue : go(&k_path64_fft<LOG2L, P64_PHILOX, false, 2>);
-        if (a.mc) return mem ? go(&k_path64_fft<LOG2L, P64_MEMORY, true, 1>) : go(&k_path64_fft<LOG2L, P64_PHILOX, true, 1>);
-        return mem ? go(&k_path64_fft<LOG2L, P64_MEMORY, false, 1>) : go(&k_path64_fft<LOG2L, P64_PHILOX, false, 1>);
+        if (a.signs == 2)
+            return a.src != P64_PHILOX || a.mc ? hipErrorInvalidValue : go(&k_path64_fft<LOG2L, P64_PHILOX, false, 2>);
+        auto from = [&](auto src) {
+            constexpr int SRC = decltype(src)::value;
+            return a.mc ? go(&k_path64_fft<LOG2L, SRC, true, 1>) : go(&k_path64_fft<LOG2L, SRC, false, 1>);
+        };
+        switch (a.src) {
+            case P64_PHILOX: return from(std::integral_constant<int, P64_PHILOX>());
+            case P64_MEMORY: return from(std::integral_constant<int, P64_MEMORY>());
+            case P64_CALLER: return from(std::integral_constant<int, P64_CALLER>());
+            default: return hipErrorInvalidValue;
+        }
     });
 }
 

@@ -347,7 +347,7 @@ int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHos
     // beyond 256 items no less than 2^14 path steps each (a call of N = 64, M = 2^16: 256 items 0.108 ms, 512
     // items 0.118).  The item size depends on the request only, so its sums are added in the same order
     // alone and in any batch; only where the partial sums of so many items (16 bytes per option and
-    // item) do not fit the memory there is, 256 items have to do.
+    // item) bring its memory above `bytes`, 256 items have to do.
     auto items = [&](long most) {
         const long steps = long(N) * a.TP;
         const long least = std::min((a.ntiles + 255) / 256, ((1L << 14) + steps - 1) / steps);

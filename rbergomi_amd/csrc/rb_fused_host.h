@@ -32,10 +32,14 @@ struct FusedHostReq {
     std::vector<Option> ivopts;  // per output I: K, T for the implied vols
 };
 
-// pb: path blocks of 32 per tile (1, 2 or 4); 0 takes fused_pb_choice.  bytes: device memory the request's
-// owner can give it (its footprint may still need more)
+// Device scratch of rb_price_noalloc, in which every buffer is rounded up to 256 bytes, at most 19 of them
+constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(64) << 20, NOALLOC_SLACK = 19 * 256;
+
+// pb: path blocks of 32 per tile (1, 2 or 4); 0 takes fused_pb_choice.  bytes: the footprint from which on
+// the request is cut into fewer items (its footprint may still be above it).  The same for every caller but a server
+// of a smaller budget: the items decide the order of the sums, and a request prices to the same bits everywhere
 int plan_fused_request(const Request& req, const Layout& lay, int mode, FusedHostReq& out,
-                       std::string& err, int pb = 0, size_t bytes = SIZE_MAX);
+                       std::string& err, int pb = 0, size_t bytes = NOALLOC_SCRATCH_BYTES - NOALLOC_SLACK);
 
 // Units, groups, payoff groups, options and P_j tables (Np entries per unit) of a request
 void fused_tables(const Request& req, const Layout& lay, int Np, int frag_stride, int pshift, FusedHostReq& out,

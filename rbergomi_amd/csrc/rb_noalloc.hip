@@ -29,10 +29,9 @@
 
 namespace {
 
-constexpr size_t NOALLOC_SCRATCH_BYTES = size_t(64) << 20;  // 64 MiB per device
 constexpr int NOALLOC_MAX_DEVICES = 64;
 
-static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[rb::NOALLOC_SCRATCH_BYTES];
 
 std::mutex g_noalloc_mu;  // serialises calls; guards g_scratch
 std::array<void*, NOALLOC_MAX_DEVICES> g_scratch{};
@@ -77,10 +76,9 @@ extern "C" int rb_price_noalloc(double xi, const double* H, const double* eta, c
     if (N > 1024) return fail(RB_ERR_LIMIT, "rb_price_noalloc covers N <= 1024 (the fused Toeplitz-GEMM kernel)");
     const Layout lay = make_layout(r);
     FusedHostReq fh;
-    // every carved buffer is rounded up to 256 bytes: at most 19 buffers
-    rc = plan_fused_request(r, lay, mode, fh, err, 0, NOALLOC_SCRATCH_BYTES - 19 * 256);
+    rc = plan_fused_request(r, lay, mode, fh, err);
     if (rc) return fail(rc, err);
-    const size_t need = FusedBatch::footprint({&fh}) + 19 * 256;
+    const size_t need = FusedBatch::footprint({&fh}) + NOALLOC_SLACK;
     if (need > NOALLOC_SCRATCH_BYTES)
         return fail(RB_ERR_LIMIT, "request needs about " + std::to_string(need >> 20) + " MiB of device scratch, above the " +
                                       std::to_string(NOALLOC_SCRATCH_BYTES >> 20) +

@@ -96,7 +96,7 @@ int request_of(const rb_request* q, int precision, int method, int comp, Request
     return validate(r, err);
 }
 
-// bytes: the device memory a job may take at most
+// bytes: the device memory there is for all jobs
 int plan_job(const rb_request* q, int precision, int method, int comp, size_t bytes, Job& j, std::string& err) {
     if (!q->price || !q->stat) {
         err = "null output arrays";
@@ -119,7 +119,8 @@ int plan_job(const rb_request* q, int precision, int method, int comp, size_t by
         j.long_path = true;
         return FftFused::plan(r, j.lay, j.footprint, err);
     }
-    rc = plan_fused_request(r, j.lay, fused_mode_of(precision), j.fh, err, 0, bytes);
+    rc = plan_fused_request(r, j.lay, fused_mode_of(precision), j.fh, err, 0,
+                            std::min(bytes, NOALLOC_SCRATCH_BYTES - NOALLOC_SLACK));
     if (rc) return rc;
     // alone it must fit one workgroup's LDS; batches are closed before a request that would push
     // their combined LDS over the limit

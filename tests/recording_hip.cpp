@@ -13,6 +13,7 @@
 #include <mutex>
 #include <string>
 
+#include "rb_fused.h"
 #include "rb_path64.h"
 
 namespace {
@@ -180,6 +181,8 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t ld
                   " nsplit " + std::to_string(a.nsplit) + " perp " + std::to_string(a.cache_perp) +
                   " mH0 " + std::to_string(int(1e6 * a.units[0].H + 0.5));
     }
+    if (name.find("k_fusedI") != std::string::npos)
+        record += " items " + std::to_string(static_cast<const rb::FusedBatchArgs*>(args[0])->total_items);
     // results to tell apart: price I + 1, standard error I + 1001, vol I + 2001
     if (name.find("k_reduce_iv") != std::string::npos)
         for (int k = 0; k < 3; ++k)

@@ -47,6 +47,10 @@ T, K = np.repeat(opts[0], 100), np.tile(opts[1], 5)
 H, eta, rho = np.linspace(0.05, 0.4, 10), np.full(10, 1.9), np.full(10, -0.7)
 # 5000 options: 20 MB of sums in 256 items, 80 MB in 1024, of 64 MiB
 rb.price_noalloc(0.04, H, eta, rho, T, K, 64, 1 << 18, [1])
+# the same items, so the same sums, in a call that allocates
+noalloc = [f["items"] for _, f in launches("k_fusedI")]
+rb.price_v2(0.04, H, eta, rho, T, K, 64, 1 << 18, [1], precision=rb.PREC_SPLIT_FP16)
+assert [f["items"] for _, f in launches("k_fusedI")] == noalloc == [256]
 # the same request in a server of 32 MiB
 s = Server(max_device_bytes=32 << 20)
 s.wait(s.submit(Request(0.04, H, eta, rho, T, K, 64, 1 << 18, [1])))

@@ -17,12 +17,12 @@
 //      rb_payoff64.hip in chunks of paths.
 //
 // What bounds it: vector issue (per thread of 16 steps and unit about 900 instructions of Gaussians, 1500 of
-// butterflies, 100 of each group: 0.55 ms of N = 4096's 0.76 below).  Sixteen points per thread keep
-// four waves per SIMD in registers (no spills to N = 2048, 19 beyond) and LDS (9 KB a wave); at N > 4096,
+// butterflies, 100 of each group; 61% of N = 4096's time below at the measured issue costs).  Sixteen points per thread keep
+// four waves per SIMD in registers (no spills to N = 2048, 17 to 4096, plain MC 25) and LDS (9 KB a wave); at N > 4096,
 // where one workgroup fills the LDS, two waves of thirty-two points each.  The form before it, one
 // pair per 256 threads with the payoffs of both paths priced between barriers by one thread per option
-// and the tables formed on the host, took, one maturity, N = 4096, M = 32768, 1.02 ms (now 0.76), N =
-// 2048, M = 65536 1.02 (0.53), plain MC 1.56 and 1.09 (0.82 and 0.57), N = 512, M = 200000 1.61 (0.39), and
+// and the tables formed on the host, took, one maturity, N = 4096, M = 32768, 1.02 ms (now 0.67), N =
+// 2048, M = 65536 1.02 (0.53), plain MC 1.56 and 1.09 (0.74 and 0.53), N = 512, M = 200000 1.61 (0.34), and
 // its tables 1.3 ms of each request at N = 4096.
 #include <hip/hip_runtime.h>
 

@@ -5,7 +5,7 @@
 // coefficients, the payoff groups (group, rho), the option list and the assignment of 32-row
 // output blocks to the four waves of a workgroup (balanced triangular work).
 // FusedBatch concatenates any number of such requests into one launch: one table of requests,
-// one list of work items (up to 1024 paths of one request each, at least 256 items per request
+// one list of work items (up to 1024 paths of one request each, about 1024 items per request
 // where its tiles allow, the last eighth of a very large request in items an eighth of the
 // size) ordered by decreasing cost and handed out through an atomic counter,
 // and one ordered reduction of every request's option sums.

@@ -102,9 +102,9 @@ struct DevArena {
 };
 
 // LDS of one fused launch over `reqs`: the largest W1 tile, cross-wave partials, per-path records
-// and option sums of its requests.  When the partials are what keeps the launch above half of a
-// CU's LDS (lds_cu / 2), their chunk of groups is cut so that two workgroups share the CU (the
-// same sums in the same order, so the same bits); *cap receives that chunk cap (0: none).  The
+// and option sums of its requests.  When the partials are what keeps the launch above a third
+// or half of a CU's LDS (lds_cu), their chunk of groups is cut so that three or two workgroups share the
+// CU (the same sums in the same order, so the same bits); *cap receives that chunk cap (0: none).  The
 // LDS fields of *a are set; returns the bytes one workgroup needs, the kernel's static request
 // record included.
 size_t fused_batch_lds(const std::vector<const FusedHostReq*>& reqs, size_t lds_cu, FusedBatchArgs* a, int* cap);
@@ -112,7 +112,9 @@ size_t fused_batch_lds(const std::vector<const FusedHostReq*>& reqs, size_t lds_
 // Whether the last request of `reqs` may join the launch of the others: the launch must fit one
 // workgroup's LDS (lds_block), and a launch that fits two workgroups per CU (half of lds_cu) is
 // not pushed above that, since its requests then run on half the waves.  (A request refused here
-// goes to another launch, which the server runs alongside on its own stream.)
+// goes to another launch, which the server runs alongside on its own stream.)  The step from three workgroups
+// to two is not guarded: refused like the other, it left the serving trace where it was (1.784 to 1.786 s a step,
+// 1.780 to 1.786 without; 48 requests 20.56 ms and 20.59).
 bool fused_batch_accepts(const std::vector<const FusedHostReq*>& reqs, size_t lds_block, size_t lds_cu);
 
 // Any number of requests priced by one launch of the fused kernel.

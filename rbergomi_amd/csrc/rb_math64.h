@@ -5,7 +5,7 @@
 // arguments need: no special cases that cannot occur, the scale factors of the model folded into
 // the tables, and 32- and 64-entry tables (in LDS) in place of longer polynomials.  The
 // polynomials are Chebyshev interpolants or Lawson-weighted least-squares fits made in 50 digits;
-// errors (checked on the host against long double, tests/test_math64_cpu.py) stay at one to two
+// errors (checked against long double on the host, tests/test_math64_cpu.py, and the device, tests/test_gpu_math64.py) stay at one to two
 // units in the last place.  Host and device compile the same code, except that the host uses the
 // library's square root and division where the device refines v_rsq_f64 and v_rcp_f64.
 #pragma once

@@ -393,7 +393,10 @@ int path64_fft_log2(int N) {
 // 1126, 1894, 1718 against 1304, 1565, 1596, 1879, 2000; plain MC, one unit at 224, 256, 384: 831, 731, 942
 // against 721, 768, 971.  Since Romano-Touzi's transforms form four quads of Gaussians together they take 48 r
 // less (r: padded over real length); whole calls at N = 224, 360: 619, 759 against 627, 836, three groups at 360 934
-// against 991, five at 380 1012 against 1067.  Beyond N = 384 products lose even where transforms fill their
+// against 991, five at 380 1012 against 1067.  The constants are Philox plans'; with the Gaussians read from memory (8e6
+// paths*steps, N from 104 to 384, one and three units, one to nine groups, both estimators) the choice is the faster kernel
+// in 94 of 104 plans and within 7% of it in the rest (one unit and group, N = 208, 224, 240, 336, 384: transforms 83,
+// 76, 74, 102, 93 us against 71, 74, 79, 95, 106).  Beyond N = 384 products lose even where transforms fill their
 // length least (N = 400, plain MC, five groups: 1548 against 1350).
 bool path64_uses_fft(int N, int units, int groups, bool mc) {
     if (N > PATH64_MFMA_MAX_N) return true;

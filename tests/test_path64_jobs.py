@@ -94,3 +94,17 @@ def test_units_of_one_workgroup_price_as_alone(N, M, method):
     for h in range(3):
         p, _, s = rb.price_v2(0.04, H3[h:h + 1], ETA3[h:h + 1], RHO3[h:h + 1], T, K, N, M, [3, N], **kw)
         assert np.array_equal(p, price[2 * h:2 * h + 2]) and np.array_equal(s, stat[2 * h:2 * h + 2])
+
+
+@pytest.mark.gpu
+def test_spectra_above_the_pinned_size_price_as_alone():
+    """Beyond N = 4096 the spectra are formed on the host: 40 of them are copied from pageable memory, one is not."""
+    import rbergomi_amd as rb
+    n, N, M = 40, 5000, 700
+    H, eta, rho = np.linspace(0.05, 0.44, n), np.full(n, 1.2), np.full(n, -0.6)
+    kw = dict(precision=rb.PREC_SPLIT_FP16)
+    print("pageable spectra", flush=True)
+    price, _, stat = rb.price_v2(0.04, H, eta, rho, [1.0], [1.0], N, M, [3], **kw)
+    for h in (0, 17, n - 1):
+        p, _, s = rb.price_v2(0.04, H[h:h + 1], eta[:1], rho[:1], [1.0], [1.0], N, M, [3], **kw)
+        assert p[0] == price[h] and s[0] == stat[h]

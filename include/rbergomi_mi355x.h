@@ -279,7 +279,9 @@ typedef struct rb_server_config {
     int precision;            /* RB_PREC_SPLIT_FP16, RB_PREC_SPLIT_BF16 or RB_PREC_FP32_GEMM */
     int max_inflight;         /* batches on the device at once (>= 1) */
     int max_batch_requests;   /* requests per batch (>= 1) */
-    long max_device_bytes;    /* admission budget for the batches in flight */
+    long max_device_bytes;    /* admission budget for the batches in flight.  Below 64 MiB, a request whose
+                               * partial sums it cannot hold is summed in fewer, larger work items (the same
+                               * prices to rounding, not to the bit) */
     double max_batch_path_steps;  /* work cap of one batch, sum of M*N (0: none); a request above
                                    * it runs as a batch of its own.  Short batches bound how long a
                                    * small request waits behind large ones. */
